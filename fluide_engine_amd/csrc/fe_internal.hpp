@@ -389,6 +389,19 @@ struct SolverScalars {
     int32_t confirm;   // a relative stop met on the recurrence awaits the recomputed residual
 };
 
+// One component's Jacobi solve of the viscosity step.
+constexpr int kDiffRing = 8;  // checks between snapshots of the state
+struct DiffState {
+    double tol;
+    double rr;               // ||b - A x||^2 at the last check
+    double ring[kDiffRing];  // and at the last checks, by check number
+    int32_t max_it;
+    int32_t it;              // sweeps of the solve
+    int32_t end;             // x_end is its result, once known
+    int32_t converged;
+    int32_t changed;         // the last checked state differs from the snapshot
+};
+
 // ---------------------------------------------------------------------------
 // Host-side scene.
 // ---------------------------------------------------------------------------
@@ -561,6 +574,10 @@ struct fe_scene {
     double* dx[2] = {nullptr, nullptr};
     uint16_t* dcode = nullptr;
     double* db = nullptr;
+    double* dsnap = nullptr;                 // an earlier iterate
+    double* dpart = nullptr;                 // residual partials, one per workgroup of a sweep
+    fe::DiffState* dstate = nullptr;         // per component
+    fe::DiffState* dstate_host = nullptr;    // pinned; allocated last
     uint8_t* dmark[3] = {nullptr, nullptr, nullptr};
     fe_solve_stats diff_stats[3] = {};
 

@@ -13,6 +13,8 @@
 //   * solver: the reference's CudaJacobiIterationSolver(1000, 5, 1e-14) (:10)
 //     semantics: sweep, and after sweep it (it > 0, it % interval == 0) stop
 //     when ||b - A x||_2 < tolerance.
+// The three components' solves are independent; they run side by side in the
+// same launches, each with its own stop (DiffState).
 // Everything is FP64 (x, b, the row arithmetic in the reference's operation
 // order with contraction off, the residual); the face velocities stay FP32
 // and are exact in FP64.  The 16-bit row code has the pressure
@@ -29,72 +31,104 @@ namespace fe {
 
 namespace {
 
-struct FaceDims {
-    int nx, ny, nz;
+// The three components' faces back to back: component c's start at off[c] in
+// every array, its workgroups are blk[c] .. blk[c + 1] (multiples of 8 each,
+// so the XCD remap holds within a component).
+struct DiffGrid {
+    int nx[3], ny[3];
+    int64_t nf[3], off[3];
+    int64_t blk[4];
 };
 
-__device__ inline void face_ijk(const FaceDims& d, int64_t f, int& i, int& j, int& k) {
-    split_index(f, d.nx, d.ny, i, j, k);
+constexpr int kDiffPer = 2;  // faces per thread of a sweep, kBlock apart
+constexpr int kDiffOpen = INT32_MAX;  // DiffState::end of a solve that goes on
+
+__device__ inline int diff_component(const DiffGrid& D, int64_t b) { return (b >= D.blk[1]) + (b >= D.blk[2]); }
+
+// The workgroup's component and its first face there.
+__device__ inline int64_t diff_first(const DiffGrid& D, int c) {
+    const int64_t lb = xcd_remap((int64_t)blockIdx.x - D.blk[c], D.blk[c + 1] - D.blk[c]);
+    return lb * (kBlock * kDiffPer);
 }
 
-// Markers and row codes of component C, and x0 = u.
-__global__ __launch_bounds__(kBlock) void k_diff_markers(Geom g, int C, FaceDims d, const double* __restrict__ sdf,
-                                                         const double* __restrict__ csdf, uint8_t* __restrict__ mark,
-                                                         int64_t padded) {
+// Face markers of the three components.
+__global__ __launch_bounds__(kBlock) void k_diff_markers(Geom g, DiffGrid D, const double* __restrict__ sdf,
+                                                         const double* __restrict__ csdf, uint8_t* __restrict__ m0,
+                                                         uint8_t* __restrict__ m1, uint8_t* __restrict__ m2) {
 #pragma clang fp contract(off)
-    const int64_t f = xcd_remap(blockIdx.x, padded) * kBlock + threadIdx.x;
-    const int64_t nf = (int64_t)d.nx * d.ny * d.nz;
-    if (f >= nf) return;
-    int idx[3];
-    face_ijk(d, f, idx[0], idx[1], idx[2]);
-    double p[3];
+    const int C = diff_component(D, blockIdx.x);
+    uint8_t* mark = C == 0 ? m0 : (C == 1 ? m1 : m2);
+    const int64_t f0 = diff_first(D, C) + threadIdx.x;
 #pragma unroll
-    for (int a = 0; a < 3; ++a) p[a] = g.cod[C][a] + g.hd[a] * (double)idx[a];  // GetX/Y/ZPos
-    uint8_t m = FE_AIR;
-    if (sample_sdf64(g, sdf, p) < 0)
-        m = FE_FLUID;
-    else if (csdf && sample_collider64(g, csdf, p) < 0)
-        m = FE_BOUNDRY;
-    mark[f] = m;
-}
-
-__global__ __launch_bounds__(kBlock) void k_diff_build(FaceDims d, const uint8_t* __restrict__ mark,
-                                                       const float* __restrict__ u, uint16_t* __restrict__ code,
-                                                       double* __restrict__ x0, double* __restrict__ b, double cx,
-                                                       double cy, double cz, int64_t padded) {
-#pragma clang fp contract(off)
-    const int64_t f = xcd_remap(blockIdx.x, padded) * kBlock + threadIdx.x;
-    const int64_t nf = (int64_t)d.nx * d.ny * d.nz;
-    if (f >= nf) return;
-    uint16_t cd = 0;
-    double bb = (double)u[f];
-    if (mark[f] == FE_FLUID) {
-        int i, j, k;
-        face_ijk(d, f, i, j, k);
-        const int64_t sy = d.nx, sz = (int64_t)d.nx * d.ny;
-        const bool in[6] = {i > 0, i + 1 < d.nx, j > 0, j + 1 < d.ny, k > 0, k + 1 < d.nz};
-        const int64_t nb[6] = {f - 1, f + 1, f - sy, f + sy, f - sz, f + sz};
-        cd = kFluidBit;
+    for (int t = 0; t < kDiffPer; ++t) {
+        const int64_t f = f0 + t * kBlock;
+        if (f >= D.nf[C]) return;
+        int idx[3];
+        split_index(f, D.nx[C], D.ny[C], idx[0], idx[1], idx[2]);
+        double p[3];
 #pragma unroll
-        for (int q = 0; q < 6; ++q) {
-            if (!in[q]) continue;
-            const uint8_t m = mark[nb[q]];
-            if (m == FE_AIR) continue;
-            cd = (uint16_t)(cd + (1u << (6 + 2 * (q >> 1))));
-            if (m == FE_FLUID) cd |= (uint16_t)(1u << q);
-        }
-        // BuildVectors' BOUNDRY terms in its order: i+1, i-1, j+1, j-1, k+1, k-1
-        const double c[3] = {cx, cy, cz};
-        const int order[6] = {1, 0, 3, 2, 5, 4};
-#pragma unroll
-        for (int t = 0; t < 6; ++t) {
-            const int q = order[t];
-            if (in[q] && mark[nb[q]] == FE_BOUNDRY) bb += c[q >> 1] * (double)u[nb[q]];
-        }
+        for (int a = 0; a < 3; ++a) p[a] = g.cod[C][a] + g.hd[a] * (double)idx[a];  // GetX/Y/ZPos
+        uint8_t m = FE_AIR;
+        if (sample_sdf64(g, sdf, p) < 0)
+            m = FE_FLUID;
+        else if (csdf && sample_collider64(g, csdf, p) < 0)
+            m = FE_BOUNDRY;
+        mark[f] = m;
     }
-    code[f] = cd;
-    x0[f] = (double)u[f];
-    b[f] = bb;
+}
+
+// Row codes, right-hand sides and x0 = u, into both iterates: an identity row
+// has the solution b = u, so no sweep needs to visit it.
+__global__ __launch_bounds__(kBlock) void k_diff_build(DiffGrid D, FaceSet uu, const uint8_t* __restrict__ m0,
+                                                       const uint8_t* __restrict__ m1, const uint8_t* __restrict__ m2,
+                                                       uint16_t* __restrict__ code, double* __restrict__ x0,
+                                                       double* __restrict__ x1, double* __restrict__ b, double cx,
+                                                       double cy, double cz, DiffState* __restrict__ st,
+                                                       DiffState init) {
+#pragma clang fp contract(off)
+    if (blockIdx.x == 0 && threadIdx.x < 3) st[threadIdx.x] = init;
+    const int C = diff_component(D, blockIdx.x);
+    const uint8_t* __restrict__ mark = C == 0 ? m0 : (C == 1 ? m1 : m2);
+    const float* __restrict__ u = uu.a[C];
+    const int64_t f0 = diff_first(D, C) + threadIdx.x;
+    const int nx = D.nx[C], ny = D.ny[C];
+    const int64_t sy = nx, sz = (int64_t)nx * ny, nf = D.nf[C];
+#pragma unroll
+    for (int e = 0; e < kDiffPer; ++e) {
+        const int64_t f = f0 + e * kBlock;
+        if (f >= nf) return;
+        uint16_t cd = 0;
+        double bb = (double)u[f];
+        const int64_t o = D.off[C] + f;
+        x0[o] = bb;
+        x1[o] = bb;
+        if (mark[f] == FE_FLUID) {
+            int i, j, k;
+            split_index(f, nx, ny, i, j, k);
+            const int nz = (int)(nf / sz);
+            const bool in[6] = {i > 0, i + 1 < nx, j > 0, j + 1 < ny, k > 0, k + 1 < nz};
+            const int64_t nb[6] = {f - 1, f + 1, f - sy, f + sy, f - sz, f + sz};
+            cd = kFluidBit;
+#pragma unroll
+            for (int q = 0; q < 6; ++q) {
+                if (!in[q]) continue;
+                const uint8_t m = mark[nb[q]];
+                if (m == FE_AIR) continue;
+                cd = (uint16_t)(cd + (1u << (6 + 2 * (q >> 1))));
+                if (m == FE_FLUID) cd |= (uint16_t)(1u << q);
+            }
+            // BuildVectors' BOUNDRY terms in its order: i+1, i-1, j+1, j-1, k+1, k-1
+            const double c[3] = {cx, cy, cz};
+            const int order[6] = {1, 0, 3, 2, 5, 4};
+#pragma unroll
+            for (int t = 0; t < 6; ++t) {
+                const int q = order[t];
+                if (in[q] && mark[nb[q]] == FE_BOUNDRY) bb += c[q >> 1] * (double)u[nb[q]];
+            }
+        }
+        code[o] = cd;
+        b[o] = bb;
+    }
 }
 
 // Centre 1 + c_a per non-AIR neighbour, summed in BuildMatrix's order (x, y, z).
@@ -111,184 +145,272 @@ __device__ inline double diff_center(uint16_t cd, const double (&c)[3]) {
 }
 
 // Sum of the off-diagonal terms A_ij x_j of a FLUID row in the reference
-// Jacobi order (i-1, i+1, j-1, j+1, k-1, k+1); uncoupled terms are zero.
-__device__ inline double diff_offdiag(uint16_t cd, int64_t f, int64_t sy, int64_t sz, const double (&c)[3],
-                                      const double* __restrict__ x) {
+// Jacobi order (i-1, i+1, j-1, j+1, k-1, k+1).  An uncoupled term adds 0,
+// which changes no sum that started at +0.
+__device__ inline double diff_offdiag(uint16_t cd, const double (&c)[3], const double (&nb)[6]) {
 #pragma clang fp contract(off)
-    const int64_t nb[6] = {f - 1, f + 1, f - sy, f + sy, f - sz, f + sz};
     double r = 0.0;
 #pragma unroll
-    for (int q = 0; q < 6; ++q)
-        if (cd & (1u << q)) r += (-c[q >> 1]) * x[nb[q]];
+    for (int q = 0; q < 6; ++q) r += (cd & (1u << q)) ? (-c[q >> 1]) * nb[q] : 0.0;
     return r;
 }
 
-__global__ __launch_bounds__(kBlock) void k_diff_jacobi(FaceDims d, const uint16_t* __restrict__ code,
-                                                        const double* __restrict__ b, const double* __restrict__ xo,
-                                                        double* __restrict__ xn, double cx, double cy, double cz,
-                                                        const SolverScalars* sc, int64_t padded) {
+// Jacobi sweep number `it` of the three components, x_{it+1} from x_it = xo
+// into xn.  CHECK: also the partials of ||b - A x_it||^2 (BLAS::Residual,
+// src/linear_system/blas.cpp:21-37; the off-diagonal sums are the sweep's),
+// and whether any value differs from the snapshot of an earlier state, which
+// `snap` 1 renews.  !WRITE: the partials only (a check after the last sweep).
+//
+// Bound by the latency of its loads (1.5 M faces at 96x80x64 in 7.4 us, of
+// which about 20 MB are read for the fluid rows, from cache): the row code
+// decides only whether a thread reads at all, and the six neighbours and b of
+// all its rows are then loaded together instead of one after another under the
+// code's bits.
+template <bool CHECK, bool WRITE>
+__global__ __launch_bounds__(kBlock) void k_diff_sweep(DiffGrid D, const uint16_t* __restrict__ code,
+                                                       const double* __restrict__ b, const double* __restrict__ xo,
+                                                       double* __restrict__ xn, double cx, double cy, double cz,
+                                                       int it, int snap, double* __restrict__ xs,
+                                                       DiffState* __restrict__ st, double* __restrict__ part) {
 #pragma clang fp contract(off)
-    if (sc->done) return;  // converged at an earlier check: x stays in the other buffer
-    const int64_t f = xcd_remap(blockIdx.x, padded) * kBlock + threadIdx.x;
-    const int64_t nf = (int64_t)d.nx * d.ny * d.nz;
-    if (f >= nf) return;
-    const uint16_t cd = code[f];
-    const double bb = b[f];
-    if (!(cd & kFluidBit)) {
-        xn[f] = bb;  // identity row: (b - 0) / 1
+    const int C = diff_component(D, blockIdx.x);
+    const int64_t f0 = diff_first(D, C) + threadIdx.x;
+    const int64_t nf = D.nf[C], sy = D.nx[C], sz = sy * D.ny[C], last = nf - 1;
+    code += D.off[C];
+    b += D.off[C];
+    xo += D.off[C];
+    xn += D.off[C];
+    xs += D.off[C];
+    uint16_t cd[kDiffPer];
+#pragma unroll
+    for (int t = 0; t < kDiffPer; ++t) {
+        const int64_t f = f0 + t * kBlock;
+        cd[t] = f < nf ? code[f] : (uint16_t)0;
+    }
+    if (it >= st[C].end) return;  // uniform: x_end stays in its buffer
+    const double c[3] = {cx, cy, cz};
+    double bb[kDiffPer], xc[kDiffPer], xp[kDiffPer], nb[kDiffPer][6];
+#pragma unroll
+    for (int t = 0; t < kDiffPer; ++t) {
+        if (!(cd[t] & kFluidBit)) continue;
+        const int64_t f = f0 + t * kBlock;
+        bb[t] = b[f];
+        nb[t][0] = xo[f > 0 ? f - 1 : 0];
+        nb[t][1] = xo[f < last ? f + 1 : last];
+        nb[t][2] = xo[f >= sy ? f - sy : 0];
+        nb[t][3] = xo[f + sy <= last ? f + sy : last];
+        nb[t][4] = xo[f >= sz ? f - sz : 0];
+        nb[t][5] = xo[f + sz <= last ? f + sz : last];
+        if (CHECK) xc[t] = xo[f];
+        if (CHECK && WRITE) xp[t] = xs[f];
+    }
+    double v[1] = {0.0};
+    int changed = 0;
+#pragma unroll
+    for (int t = 0; t < kDiffPer; ++t) {
+        if (!(cd[t] & kFluidBit)) continue;  // b - x is 0 on an identity row
+        const double off = diff_offdiag(cd[t], c, nb[t]);
+        const double center = diff_center(cd[t], c);
+        if (WRITE) xn[f0 + t * kBlock] = (bb[t] - off) / center;
+        if (CHECK) {
+            const double r = (bb[t] - center * xc[t]) - off;
+            v[0] += r * r;
+            if (WRITE) {
+                changed |= __double_as_longlong(xc[t]) != __double_as_longlong(xp[t]);
+                if (snap) xs[f0 + t * kBlock] = xc[t];
+            }
+        }
+    }
+    if (CHECK) {
+        if (WRITE) {
+            changed = __syncthreads_or(changed);
+            if (changed && threadIdx.x == 0) st[C].changed = 1;  // every writer writes the same
+        }
+        write_partials<1>(v, part);
+    }
+}
+
+// One workgroup per component: check number q (q >= 1, after sweep
+// j = q * interval, on the state x_{j+1}), from the partials that sweep j + 1
+// left.
+//
+// A state that equals the snapshot L <= kDiffRing checks before it, bit for
+// bit, starts the same L * interval sweeps again: all later states and checks
+// are ones already seen, none of which met the tolerance, so the solve's last
+// state is at most L * interval sweeps away and its last residual is known.
+// Rounding brings every solve there (the sweep is a contraction; cycles of 2
+// and 4 sweeps seen), and the reference's tolerance of 1e-14 on an absolute
+// norm is below what rounding leaves on all but tiny grids: at 96x80x64 the
+// states repeat from sweep 155 of the 1000.
+__global__ __launch_bounds__(kBlock) void k_diff_check(DiffGrid D, const double* __restrict__ part, int q,
+                                                       int interval, int compared, DiffState* __restrict__ st) {
+    const int C = blockIdx.x;
+    DiffState* S = st + C;
+    if (S->end != kDiffOpen) return;
+    double t[1];
+    sum_partials<1>(part + D.blk[C], (int)(D.blk[C + 1] - D.blk[C]), t);
+    if (threadIdx.x != 0) return;
+    const int k = q * interval + 1;  // the state checked
+    S->rr = t[0];
+    S->ring[q % kDiffRing] = t[0];
+    if (sqrt(t[0]) < S->tol) {
+        S->converged = 1;
+        S->it = k;
+        S->end = k;
         return;
     }
-    const double c[3] = {cx, cy, cz};
-    const double off = diff_offdiag(cd, f, d.nx, (int64_t)d.nx * d.ny, c, xo);
-    xn[f] = (bb - off) / diff_center(cd, c);
-}
-
-// Partials of ||b - A x||^2 (BLAS::Residual, src/linear_system/blas.cpp:21-37).
-__global__ __launch_bounds__(kBlock) void k_diff_residual(FaceDims d, const uint16_t* __restrict__ code,
-                                                          const double* __restrict__ b,
-                                                          const double* __restrict__ x, double cx, double cy,
-                                                          double cz, const SolverScalars* sc,
-                                                          double* __restrict__ part, int64_t chunk, int64_t padded) {
-#pragma clang fp contract(off)
-    const int64_t nf = (int64_t)d.nx * d.ny * d.nz;
-    const Span sp = block_span(nf, chunk, padded);
-    const double c[3] = {cx, cy, cz};
-    double v[1] = {0.0};
-    if (!sc->done) {
-        for (int64_t f = sp.c0 + threadIdx.x; f < sp.c1; f += kBlock) {
-            const uint16_t cd = code[f];
-            double r = b[f];
-            if (cd & kFluidBit)
-                r = (r - diff_center(cd, c) * x[f]) - diff_offdiag(cd, f, d.nx, (int64_t)d.nx * d.ny, c, x);
-            else
-                r = r - x[f];
-            v[0] += r * r;
-        }
+    if (compared && !S->changed) {
+        const int L = (q - 1) % kDiffRing + 1;  // checks since the snapshot
+        const int last = (S->max_it - 1) / interval;
+        S->rr = S->ring[(q - ((q - last) % L + L) % L) % kDiffRing];
+        S->end = k + (S->max_it - k) % (L * interval);
     }
-    write_partials<1>(v, part);
+    S->changed = 0;
 }
 
-// One block: the convergence check after sweep `it` (0-based).
-__global__ __launch_bounds__(kBlock) void k_diff_check(const double* __restrict__ part, int nparts, int it,
-                                                       SolverScalars* sc) {
-    if (sc->done) return;
-    double t[1];
-    sum_partials<1>(part, nparts, t);
-    if (threadIdx.x == 0) {
-        sc->rr = t[0];
-        if (sqrt(t[0]) < sc->tol) {
-            sc->done = 1;
-            sc->converged = 1;
-            sc->it = it + 1;
-        }
+__global__ __launch_bounds__(kBlock) void k_diff_store(DiffGrid D, const double* __restrict__ x0,
+                                                       const double* __restrict__ x1, int odd, FaceSet u) {
+    const int C = diff_component(D, blockIdx.x);
+    const double* __restrict__ x = ((odd >> C) & 1 ? x1 : x0) + D.off[C];
+    const int64_t f0 = diff_first(D, C) + threadIdx.x;
+#pragma unroll
+    for (int t = 0; t < kDiffPer; ++t) {
+        const int64_t f = f0 + t * kBlock;
+        if (f < D.nf[C]) u.a[C][f] = (float)x[f];  // output->x/y/z(i, j, k) = _system.x(i, j, k)
     }
 }
 
-__global__ __launch_bounds__(kBlock) void k_diff_store(const double* __restrict__ x, float* __restrict__ u,
-                                                       int64_t n) {
-    const int64_t f = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    if (f < n) u[f] = (float)x[f];  // output->x/y/z(i, j, k) = _system.x(i, j, k)
+DiffGrid diff_grid(const Geom& g) {
+    DiffGrid D{};
+    int64_t off = 0;
+    for (int c = 0; c < 3; ++c) {
+        D.nx[c] = face_dim(g, c, 0);
+        D.ny[c] = face_dim(g, c, 1);
+        D.nf[c] = face_count(g, c);
+        D.off[c] = off;
+        off += (D.nf[c] + 15) / 16 * 16;
+        D.blk[c + 1] = D.blk[c] + pad_blocks((D.nf[c] + kBlock * kDiffPer - 1) / (kBlock * kDiffPer));
+    }
+    return D;
 }
-
-FaceDims face_dims(const Geom& g, int c) { return {face_dim(g, c, 0), face_dim(g, c, 1), face_dim(g, c, 2)}; }
 
 }  // namespace
 
 hipError_t diffusion_alloc(fe_scene* s) {
-    if (s->dx[0]) return hipSuccess;
-    int64_t nf = 0;
-    for (int c = 0; c < 3; ++c) nf = std::max<int64_t>(nf, face_count(s->g, c));
+    if (s->dstate_host) return hipSuccess;
+    const DiffGrid D = diff_grid(s->g);
+    const int64_t n = D.off[2] + D.nf[2];
     hipError_t e;
     for (int b = 0; b < 2; ++b)
-        if ((e = hipMalloc((void**)&s->dx[b], sizeof(double) * nf)) != hipSuccess) return e;
-    if ((e = hipMalloc((void**)&s->dcode, sizeof(uint16_t) * nf)) != hipSuccess) return e;
-    if ((e = hipMalloc((void**)&s->db, sizeof(double) * nf)) != hipSuccess) return e;
+        if ((e = hipMalloc((void**)&s->dx[b], sizeof(double) * n)) != hipSuccess) return e;
+    if ((e = hipMalloc((void**)&s->dcode, sizeof(uint16_t) * n)) != hipSuccess) return e;
+    if ((e = hipMalloc((void**)&s->db, sizeof(double) * n)) != hipSuccess) return e;
+    if ((e = hipMalloc((void**)&s->dsnap, sizeof(double) * n)) != hipSuccess) return e;
+    if ((e = hipMalloc((void**)&s->dpart, sizeof(double) * D.blk[3])) != hipSuccess) return e;
+    if ((e = hipMalloc((void**)&s->dstate, sizeof(DiffState) * 3)) != hipSuccess) return e;
     for (int c = 0; c < 3; ++c)
         if ((e = hipMalloc((void**)&s->dmark[c], face_count(s->g, c))) != hipSuccess) return e;
-    return hipSuccess;
+    return hipHostMalloc((void**)&s->dstate_host, sizeof(DiffState) * 3, hipHostMallocDefault);
 }
 
 void diffusion_free(fe_scene* s) {
-    for (int b = 0; b < 2; ++b) {
-        if (s->dx[b]) (void)hipFree(s->dx[b]);
-        s->dx[b] = nullptr;
-    }
-    if (s->dcode) (void)hipFree(s->dcode);
-    s->dcode = nullptr;
-    if (s->db) (void)hipFree(s->db);
-    s->db = nullptr;
-    for (int c = 0; c < 3; ++c) {
-        if (s->dmark[c]) (void)hipFree(s->dmark[c]);
-        s->dmark[c] = nullptr;
-    }
+    auto release = [](auto*& p) {
+        if (p) (void)hipFree(p);
+        p = nullptr;
+    };
+    for (int b = 0; b < 2; ++b) release(s->dx[b]);
+    release(s->dcode);
+    release(s->db);
+    release(s->dsnap);
+    release(s->dpart);
+    release(s->dstate);
+    for (int c = 0; c < 3; ++c) release(s->dmark[c]);
+    if (s->dstate_host) (void)hipHostFree(s->dstate_host);
+    s->dstate_host = nullptr;
 }
 
 // ComputeDiffusion without its trailing ApplyBoundryCondition: the three
-// component solves in order x, y, z, each a Jacobi solve on the scene's stream
-// in batches of sweeps with one host read of the stopping flag per batch.
+// component solves (each reads and writes its own component only) as Jacobi
+// solves side by side on the scene's stream, in batches of sweeps with one
+// host read of the stopping flags per batch.  The check after sweep j is taken
+// from sweep j + 1, which reads the same rows: it leaves x_{j+1} in its input
+// buffer, so a stop found there loses nothing.
 hipError_t launch_diffusion(fe_scene* s, double dt, const fe_solver_desc* d) {
     const Geom& g = s->g;
     const double nu = s->desc.viscosity;
     const double c[3] = {(dt * nu) / (g.hd[0] * g.hd[0]), (dt * nu) / (g.hd[1] * g.hd[1]),
                          (dt * nu) / (g.hd[2] * g.hd[2])};
     hipError_t e;
-    if ((e = diffusion_alloc(s)) != hipSuccess) return e;
-    constexpr int kBatch = 50;  // sweeps between host reads of the stopping flag
-    for (int comp = 0; comp < 3; ++comp) {
-        const FaceDims fd = face_dims(g, comp);
-        const int64_t nf = face_count(g, comp);
-        const int64_t padded = pad_blocks((nf + kBlock - 1) / kBlock);
-        const SolverShape sh = solver_shape_n(nf);
-        if (sh.blocks > s->npartials) return hipErrorInvalidValue;  // partial sums must fit the scene's buffer
-        hipLaunchKernelGGL(k_diff_markers, dim3((unsigned)padded), dim3(kBlock), 0, s->stream, g, comp, fd,
-                           (const double*)s->sdf, (const double*)(s->has_collider ? s->csdf : nullptr),
-                           s->dmark[comp], padded);
-        hipLaunchKernelGGL(k_diff_build, dim3((unsigned)padded), dim3(kBlock), 0, s->stream, fd,
-                           (const uint8_t*)s->dmark[comp], (const float*)s->u[comp], s->dcode, s->dx[0], s->db, c[0],
-                           c[1], c[2], padded);
-        SolverScalars init{};
-        init.tol = d->tolerance;
-        init.max_it = d->max_iterations;
-        init.it = d->max_iterations;
-        if ((e = hipMemcpyAsync(s->sc, &init, sizeof(SolverScalars), hipMemcpyHostToDevice, s->stream)) != hipSuccess)
-            return e;
-        int it = 0;
-        bool done = false;
-        while (it < d->max_iterations && !done) {
-            const int end = std::min(d->max_iterations, it + kBatch);
-            for (; it < end; ++it) {
-                hipLaunchKernelGGL(k_diff_jacobi, dim3((unsigned)padded), dim3(kBlock), 0, s->stream, fd,
-                                   (const uint16_t*)s->dcode, (const double*)s->db, (const double*)s->dx[it & 1],
-                                   s->dx[(it + 1) & 1], c[0], c[1], c[2], (const SolverScalars*)s->sc, padded);
-                if (it != 0 && d->check_interval > 0 && it % d->check_interval == 0) {
-                    hipLaunchKernelGGL(k_diff_residual, dim3((unsigned)sh.blocks), dim3(kBlock), 0, s->stream, fd,
-                                       (const uint16_t*)s->dcode, (const double*)s->db,
-                                       (const double*)s->dx[(it + 1) & 1], c[0], c[1], c[2],
-                                       (const SolverScalars*)s->sc, s->partials, sh.chunk, sh.blocks);
-                    hipLaunchKernelGGL(k_diff_check, dim3(1), dim3(kBlock), 0, s->stream, (const double*)s->partials,
-                                       (int)sh.blocks, it, s->sc);
-                }
+    if ((e = diffusion_alloc(s)) != hipSuccess) {
+        diffusion_free(s);
+        return e;
+    }
+    const DiffGrid D = diff_grid(g);
+    const dim3 grid((unsigned)D.blk[3]), block(kBlock);
+    const FaceSet u{{s->u[0], s->u[1], s->u[2]}};
+    hipLaunchKernelGGL(k_diff_markers, grid, block, 0, s->stream, g, D, (const double*)s->sdf,
+                       (const double*)(s->has_collider ? s->csdf : nullptr), s->dmark[0], s->dmark[1], s->dmark[2]);
+    DiffState init{};
+    init.tol = d->tolerance;
+    init.max_it = d->max_iterations;
+    init.it = d->max_iterations;
+    init.end = kDiffOpen;
+    hipLaunchKernelGGL(k_diff_build, grid, block, 0, s->stream, D, u, (const uint8_t*)s->dmark[0],
+                       (const uint8_t*)s->dmark[1], (const uint8_t*)s->dmark[2], s->dcode, s->dx[0], s->dx[1], s->db,
+                       c[0], c[1], c[2], s->dstate, init);
+    constexpr int kBatch = 50;  // sweeps between host reads of the stopping flags
+    const int interval = d->check_interval;
+    auto checked = [&](int j) { return interval > 0 && j > 0 && j % interval == 0; };  // after sweep j
+    auto sweep = [&](auto kernel, int it, int snap) {
+        hipLaunchKernelGGL(kernel, grid, block, 0, s->stream, D, (const uint16_t*)s->dcode, (const double*)s->db,
+                           (const double*)s->dx[it & 1], s->dx[(it + 1) & 1], c[0], c[1], c[2], it, snap, s->dsnap,
+                           s->dstate, s->dpart);
+    };
+    auto check = [&](int q, int compared) {
+        hipLaunchKernelGGL(k_diff_check, dim3(3), block, 0, s->stream, D, (const double*)s->dpart, q, interval,
+                           compared, s->dstate);
+    };
+    for (int comp = 0; comp < 3; ++comp) s->dstate_host[comp] = init;
+    int it = 0;
+    bool done = false;
+    while (it < d->max_iterations && !done) {
+        const int end = std::min(d->max_iterations, it + kBatch);
+        for (; it < end; ++it) {
+            if (checked(it - 1)) {
+                const int q = (it - 1) / interval;
+                sweep(k_diff_sweep<true, true>, it, q % kDiffRing == 0);
+                check(q, q > kDiffRing);
+            } else {
+                sweep(k_diff_sweep<false, true>, it, 0);
             }
-            if ((e = hipGetLastError()) != hipSuccess) return e;
-            if ((e = hipMemcpyAsync(s->sc_host, s->sc, sizeof(SolverScalars), hipMemcpyDeviceToHost, s->stream)) !=
-                hipSuccess)
-                return e;
-            if ((e = hipStreamSynchronize(s->stream)) != hipSuccess) return e;
-            done = s->sc_host->done != 0;
         }
-        const int executed = done ? s->sc_host->it : d->max_iterations;
-        hipLaunchKernelGGL(k_diff_store, dim3((unsigned)((nf + kBlock - 1) / kBlock)), dim3(kBlock), 0, s->stream,
-                           (const double*)s->dx[executed & 1], s->u[comp], nf);
+        if (it == d->max_iterations && checked(it - 1)) {
+            sweep(k_diff_sweep<true, false>, it, 0);
+            check((it - 1) / interval, 0);
+        }
         if ((e = hipGetLastError()) != hipSuccess) return e;
+        if ((e = hipMemcpyAsync(s->dstate_host, s->dstate, sizeof(DiffState) * 3, hipMemcpyDeviceToHost,
+                                s->stream)) != hipSuccess)
+            return e;
+        if ((e = hipStreamSynchronize(s->stream)) != hipSuccess) return e;
+        done = true;
+        for (int comp = 0; comp < 3; ++comp) done = done && s->dstate_host[comp].end <= it;
+    }
+    int odd = 0;
+    for (int comp = 0; comp < 3; ++comp) {
+        const DiffState& h = s->dstate_host[comp];
+        odd |= (std::min(h.end, d->max_iterations) & 1) << comp;
         fe_solve_stats& st = s->diff_stats[comp];
         st = fe_solve_stats{};
-        st.iterations = executed;
-        st.converged = done ? 1 : 0;
-        st.abs_residual = d->check_interval > 0 && executed > d->check_interval ? std::sqrt(s->sc_host->rr) : -1.0;
+        st.iterations = h.it;
+        st.converged = h.converged;
+        st.abs_residual = interval > 0 && h.it > interval ? std::sqrt(h.rr) : -1.0;
         st.rel_residual = -1.0;
         st.ms = 0.0;
     }
-    return hipSuccess;
+    hipLaunchKernelGGL(k_diff_store, grid, block, 0, s->stream, D, (const double*)s->dx[0], (const double*)s->dx[1],
+                       odd, u);
+    return hipGetLastError();
 }
 
 }  // namespace fe

@@ -130,3 +130,29 @@ def test_substep_with_viscosity_parity(ctx):
     gst = g.last_diffusion_stats()
     assert all(s.iterations > 5 for s in gst)
     g.close()
+
+
+@pytest.mark.parametrize("n,nu,cap,interval", [((12, 10, 8), 0.3, 1000, 5), ((12, 10, 8), 0.3, 1001, 4),
+                                               ((33, 9, 17), 0.05, 997, 7), ((2, 2, 2), 0.1, 501, 1),
+                                               ((5, 31, 3), 0.2, 6, 5), ((16, 16, 33), 0.1, 300, 0)])
+def test_diffusion_repeated_states(ctx, n, nu, cap, interval):
+    """An unreachable tolerance: the sweeps end in repeated states long before
+    the cap, and the counts, the last residual and the values are those of
+    the whole number of sweeps (odd and even intervals and caps, none at all;
+    residuals of rounding size, so within a factor of 4 of the oracle's)."""
+    print(f"[gpu] diffusion repeated states n={n} cap={cap} interval={interval}", flush=True)
+    g, o = _pair(ctx, n, (1.0, 0.8, 1.1), nu, seed=sum(n))
+    g.set_diffusion_solver(capi.solver(capi.SOLVER_JACOBI, cap, interval, 1e-30))
+    o.set_diffusion_solver(orc.solver(orc.JACOBI, cap, interval if interval else cap + 1, 1e-30))
+    dt = 1.0 / 120
+    g.run_stage(capi.STAGE_DIFFUSION, dt)
+    ost = o.diffusion(dt)
+    gst = g.last_diffusion_stats()
+    assert all(s.iterations == cap and not s.converged for s in gst)
+    _compare(g, o, gst, ost)
+    for s in gst:
+        if interval and cap > interval:
+            assert 0.0 <= s.abs_residual < 1e-12 if cap > 100 else s.abs_residual > 1e-12
+        else:
+            assert s.abs_residual == -1.0
+    g.close()
