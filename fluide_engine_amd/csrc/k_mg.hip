@@ -95,7 +95,8 @@ __global__ __launch_bounds__(kBlock) void k_mg_coarsen(const uint8_t* __restrict
 // by k_mg_coarsen's rule -- AIR if a child is AIR, else FLUID if a child is
 // FLUID, else BOUNDRY, over the children that exist.  It also leaves the
 // fine-tile flags of the fused V-cycle's finest level (a block's level-0
-// region is two 16 x 16 x 8 tiles): whether the tile holds a FLUID cell.
+// region is two 16 x 16 x 8 tiles or eight 8 x 8 x 8 ones): whether the tile
+// holds a FLUID cell.
 constexpr int kPyr = 4;
 constexpr int kPyrThreads = 512;
 constexpr uint8_t kNoCell = 255;  // a cell beyond its level's dims
@@ -106,6 +107,7 @@ struct PyrArgs {
     uint8_t* flags[kPyr + 1];
     uint8_t* tfl;         // tile flags of level 0 (null: not wanted)
     int tiles[3];         // tile counts of level 0's fused tiles
+    int rx, ry, rz;       // and their level-1 cells per axis (8 or 4)
 };
 
 __global__ __launch_bounds__(kPyrThreads) void k_mg_pyramid(PyrArgs a) {
@@ -144,14 +146,17 @@ __global__ __launch_bounds__(kPyrThreads) void k_mg_pyramid(PyrArgs a) {
         L[0][t] = out;
     }
     if (a.tfl) {
-        // tiles of 8 x 8 x 4 level-1 cells: this block's lower and upper halves in z
-        const int lower = __syncthreads_or(t < 256 ? fluid0 : 0);
-        const int upper = __syncthreads_or(t >= 256 ? fluid0 : 0);
-        if (t < 2) {
-            const int tz = 2 * B[2] + t;
-            if (B[0] < a.tiles[0] && B[1] < a.tiles[1] && tz < a.tiles[2])
-                a.tfl[(int64_t)B[0] + (int64_t)a.tiles[0] * ((int64_t)B[1] + (int64_t)a.tiles[1] * tz)] =
-                    (uint8_t)(t == 0 ? lower : upper);
+        // the tiles of this block: 8 / rx by 8 / ry by 8 / rz
+        __shared__ int has[8];
+        if (t < 8) has[t] = 0;
+        __syncthreads();
+        const int mx = 8 / a.rx, my = 8 / a.ry, mz = 8 / a.rz;
+        if (fluid0) has[(t % 8) / a.rx + mx * ((t / 8) % 8 / a.ry + my * (t / 64 / a.rz))] = 1;
+        __syncthreads();
+        if (t < mx * my * mz) {
+            const int tx = mx * B[0] + t % mx, ty = my * B[1] + (t / mx) % my, tz = mz * B[2] + t / (mx * my);
+            if (tx < a.tiles[0] && ty < a.tiles[1] && tz < a.tiles[2])
+                a.tfl[(int64_t)tx + (int64_t)a.tiles[0] * ((int64_t)ty + (int64_t)a.tiles[1] * tz)] = (uint8_t)has[t];
         }
     } else {
         __syncthreads();
@@ -593,7 +598,8 @@ __global__ __launch_bounds__(kBlock) void k_mg_prolong(const float* __restrict__
 // level has 16 large tiles for 256 CUs, and each workgroup's chain of LDS
 // phases sets the kernel's time), so they take small tiles: 2.5x fewer cells
 // per thread in every phase for more halo work in all.  A cell's value does
-// not depend on the tile it is computed in.
+// not depend on the tile it is computed in.  A finest level of few tiles is
+// such a level too (small_finest).
 // ---------------------------------------------------------------------------
 template <int RX, int RY, int RZ>
 struct FusedTile {
@@ -1221,6 +1227,198 @@ __global__ __launch_bounds__(kTailThreads) void k_mg_tail(TailArgs a, const floa
 }
 
 // ---------------------------------------------------------------------------
+// The last two levels of the fused V-cycle in one workgroup: the descent into
+// the coarsest level, its Chebyshev iteration, and the ascent.  Bound by the
+// chain of phases between barriers (a level of 16^3 over one of 8^3: 16
+// barriers); it replaces three launches (4.7 + 4.2 + 5.1 us and the gaps
+// between them) with one.
+//
+// A thread keeps up to four fine cells (right-hand side, diagonal, weight and
+// place, in registers) and at most one coarse cell.  The iterates lie in LDS
+// with a border of zeros, so the FLUID-row forms need neither codes nor
+// clamps there: a cell's neighbours are at fixed offsets, and every cell that
+// is not FLUID holds 0, as does the border.  The terms and their order are the
+// tiles' and the tail's, so the values are too.
+// ---------------------------------------------------------------------------
+constexpr int kBotThreads = 1024;
+constexpr int kBotPer = 4;  // fine cells per thread: a coarsest level of 512 cells halves one of at most 4096
+constexpr int kBotLds = 20000;  // floats of LDS at most (80 KB)
+static_assert(kBotThreads * kBotPer >= 8 * kCoarseMax && kBotThreads >= kCoarseMax, "a place for every cell");
+
+struct BottomArgs {
+    int n[3], c[3];          // the fine and the coarsest level
+    float ih2[3], cih2[3];
+    int pf, pc;              // padded cells of each
+};
+
+// Offset of cell (i, j, k) in an array of dims n with a border of one.
+__device__ inline int bordered(int i, int j, int k, const int n[3]) {
+    return (i + 1) + (n[0] + 2) * ((j + 1) + (n[1] + 2) * (k + 1));
+}
+
+__device__ inline void bordered_neighbours(const float* x, int p, int sy, int sz, float (&nb)[6]) {
+    nb[0] = x[p - 1];
+    nb[1] = x[p + 1];
+    nb[2] = x[p - sy];
+    nb[3] = x[p + sy];
+    nb[4] = x[p - sz];
+    nb[5] = x[p + sz];
+}
+
+__global__ __launch_bounds__(kBotThreads) void k_mg_bottom(BottomArgs a, const float* __restrict__ b,
+                                                           const uint16_t* __restrict__ code,
+                                                           const uint16_t* __restrict__ ccode,
+                                                           float* __restrict__ out,
+                                                           const SolverScalars* __restrict__ st) {
+    extern __shared__ float lds[];
+    float* X = lds;           // fine iterates
+    float* Y = X + a.pf;
+    float* U = Y + a.pf;      // coarse iterates
+    float* V = U + a.pc;
+    const int done = st->done;  // read with the data, tested before the first write
+    const int nf = a.n[0] * a.n[1] * a.n[2], nc = a.c[0] * a.c[1] * a.c[2];
+    float bf[kBotPer];
+    uint32_t cd[kBotPer];
+#pragma unroll
+    for (int u = 0; u < kBotPer; ++u) {
+        const int f = threadIdx.x + u * kBotThreads;
+        bf[u] = f < nf ? b[f] : 0.0f;
+        cd[u] = f < nf ? (uint32_t)code[f] : 0u;
+    }
+    const bool con = (int)threadIdx.x < nc;
+    const uint32_t ccd = con ? (uint32_t)ccode[threadIdx.x] : 0u;
+    for (int e = threadIdx.x; e < 2 * (a.pf + a.pc); e += kBotThreads) lds[e] = 0.0f;
+    constexpr MgSmooth SM = kMgCoarse;
+    const CodeLanes fl = code_lanes(a.ih2, SM.omega), cl = code_lanes(a.cih2, 1.0f);
+    const float nih2[3] = {-a.ih2[0], -a.ih2[1], -a.ih2[2]}, cnih2[3] = {-a.cih2[0], -a.cih2[1], -a.cih2[2]};
+    const int sy = a.n[0] + 2, sz = sy * (a.n[1] + 2), csy = a.c[0] + 2, csz = csy * (a.c[1] + 2);
+    float cen[kBotPer], wgt[kBotPer];
+    int p[kBotPer];
+#pragma unroll
+    for (int u = 0; u < kBotPer; ++u) {
+        const int li = code_lane(cd[u]);
+        cen[u] = lane_read(fl.cen, li);
+        wgt[u] = lane_read(fl.wgt, li);
+        int i, j, k;
+        cell_ijk(threadIdx.x + u * kBotThreads, a.n[0], a.n[1], i, j, k);
+        p[u] = bordered(i, j, k, a.n);
+    }
+    const int cli = code_lane(ccd);
+    const float ccen = lane_read(cl.cen, cli), cw = lane_read(cl.wgt, cli);
+    int I, J, K;
+    cell_ijk(threadIdx.x, a.c[0], a.c[1], I, J, K);
+    const int cp = bordered(I, J, K, a.c);
+    const bool cfl = (ccd & kFluidBit) != 0;  // false where there is no cell
+    __syncthreads();
+    if (done) return;  // uniform: the solve has stopped
+    // x1, the first sweep from zero
+#pragma unroll
+    for (int u = 0; u < kBotPer; ++u)
+        if (cd[u] & kFluidBit) X[p[u]] = wgt[u] * bf[u];
+    __syncthreads();
+    // x2, kept for the ascent
+    float x2[kBotPer];
+#pragma unroll
+    for (int u = 0; u < kBotPer; ++u) {
+        x2[u] = 0.0f;
+        if (!(cd[u] & kFluidBit)) continue;
+        float nb[6];
+        bordered_neighbours(X, p[u], sy, sz, nb);
+        const float x1 = X[p[u]];
+        x2[u] = mg_cheb2(x1, 0.0f, SM.w21 * wgt[u], bf[u] - mg_apply_fluid_row(cen[u], x1, nb, nih2), SM.beta);
+        Y[p[u]] = x2[u];
+    }
+    __syncthreads();
+    // r = b - A x2 (over x1, which nothing reads any more)
+#pragma unroll
+    for (int u = 0; u < kBotPer; ++u) {
+        if (!(cd[u] & kFluidBit)) continue;
+        float nb[6];
+        bordered_neighbours(Y, p[u], sy, sz, nb);
+        X[p[u]] = bf[u] - mg_apply_fluid_row(cen[u], x2[u], nb, nih2);
+    }
+    __syncthreads();
+    // the coarsest level: b = R r and kCoarseSweeps steps of Chebyshev
+    // iteration from zero (the three-term recurrence of k_mg_tail)
+    const float theta = 0.5f * (kChebHi + kChebLo), delta = 0.5f * (kChebHi - kChebLo);
+    const float sigma = theta / delta;
+    float rho = 1.0f / sigma;
+    float bc = 0.0f, d = 0.0f, xc = 0.0f;
+    if (cfl) {
+        int ix[4], iy[4], iz[4];
+        float wx[4], wy[4], wz[4];
+        restrict_taps(I, a.n[0], a.c[0], ix, wx);
+        restrict_taps(J, a.n[1], a.c[1], iy, wy);
+        restrict_taps(K, a.n[2], a.c[2], iz, wz);
+        float acc = 0.0f;
+#pragma unroll
+        for (int tk = 0; tk < 4; ++tk) {
+#pragma unroll
+            for (int tj = 0; tj < 4; ++tj) {
+                const float wjk = wy[tj] * wz[tk];
+#pragma unroll
+                for (int ti = 0; ti < 4; ++ti) acc += (wx[ti] * wjk) * X[bordered(ix[ti], iy[tj], iz[tk], a.n)];
+            }
+        }
+        bc = acc * 0.125f;
+        d = (1.0f / theta) * (cw * bc);
+        xc = d;
+        U[cp] = xc;
+    }
+    __syncthreads();
+    static_assert(kCoarseSweeps % 2 == 0, "the last step writes V");
+    for (int q = 1; q < kCoarseSweeps; ++q) {
+        const float rn = 1.0f / (2.0f * sigma - rho);
+        const float c1 = rn * rho, c2 = 2.0f * rn / delta;
+        const float* in = q & 1 ? U : V;
+        float* to = q & 1 ? V : U;
+        if (cfl) {
+            float nb[6];
+            bordered_neighbours(in, cp, csy, csz, nb);
+            d = c1 * d + c2 * (cw * (bc - mg_apply_fluid_row(ccen, xc, nb, cnih2)));
+            xc = xc + d;
+            to[cp] = xc;
+        }
+        rho = rn;
+        __syncthreads();
+    }
+    // the ascent: y = x2 + P xc, two steps
+#pragma unroll
+    for (int u = 0; u < kBotPer; ++u) {
+        if (!(cd[u] & kFluidBit)) continue;
+        int i, j, k;
+        cell_ijk(threadIdx.x + u * kBotThreads, a.n[0], a.n[1], i, j, k);
+        x2[u] = x2[u] + prolong_at3(i, j, k, a.c[0], a.c[1], a.c[2],
+                                    [&](int A, int B, int C) { return V[bordered(A, B, C, a.c)]; });
+        Y[p[u]] = x2[u];
+    }
+    __syncthreads();
+    float xp[kBotPer];
+#pragma unroll
+    for (int u = 0; u < kBotPer; ++u) {
+        xp[u] = 0.0f;
+        if (!(cd[u] & kFluidBit)) continue;
+        float nb[6];
+        bordered_neighbours(Y, p[u], sy, sz, nb);
+        xp[u] = mg_sweep_fluid_row(cen[u], wgt[u], x2[u], bf[u], nb, nih2);
+        X[p[u]] = xp[u];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kBotPer; ++u) {
+        const int f = threadIdx.x + u * kBotThreads;
+        if (f >= nf) break;
+        float o = 0.0f;
+        if (cd[u] & kFluidBit) {
+            float nb[6];
+            bordered_neighbours(X, p[u], sy, sz, nb);
+            o = mg_cheb2(xp[u], x2[u], SM.w21 * wgt[u], bf[u] - mg_apply_fluid_row(cen[u], xp[u], nb, nih2), SM.beta);
+        }
+        out[f] = o;
+    }
+}
+
+// ---------------------------------------------------------------------------
 // Host side
 // ---------------------------------------------------------------------------
 static inline dim3 grid1(int64_t n) { return dim3((unsigned)((n + kBlock - 1) / kBlock)); }
@@ -1249,6 +1447,22 @@ static FusedArgs fused_args(const MGLevel& l, const MGLevel& c) {
     a.tiles[2] = (c.n[2] + T::rz - 1) / T::rz;
     a.padded = pad_blocks((int64_t)a.tiles[0] * a.tiles[1] * a.tiles[2]);
     return a;
+}
+
+// Whether the finest level takes the small tiles: up to two of them per CU.
+// There the level's kernels are bound by the latency of a workgroup's chain of
+// phases, and a small tile has 2.5x fewer cells per thread in each; above, by
+// throughput, and the small tiles' halos cost more than they save.  Measured
+// on whole solves to 1e-10 (large tiles / small): 32^3 0.61 / 0.52 ms, 48^3
+// 0.74 / 0.65, 64^3 (512 tiles) 0.875 / 0.838, 80x64x72 (720) 1.01 / 1.05,
+// 96^3 1.24 / 1.39, 128^3 1.74 / 2.11.
+static bool small_finest(const MGLevel& l) {
+    constexpr int64_t kCus = 256;
+    return l.cells <= 2 * kCus * TileCoarse::coarse * 8;
+}
+
+static FusedArgs finest_args(const MGLevel& l, const MGLevel& c) {
+    return small_finest(l) ? fused_args<TileCoarse>(l, c) : fused_args<TileFinest>(l, c);
 }
 
 void mg_free(fe_scene* s);
@@ -1303,7 +1517,7 @@ static hipError_t mg_alloc(fe_scene* s) {
         if ((e = hipMalloc((void**)&l.r, n * sizeof(float))) != hipSuccess) break;
     }
     // the fused V-cycle's level-0 tile flags and r.z partials
-    const FusedArgs fa = fused_args<TileFinest>(lv[0], lv[1]);
+    const FusedArgs fa = finest_args(lv[0], lv[1]);
     s->mg_npz = fa.padded;
     if (e == hipSuccess) e = hipMalloc((void**)&s->mg_tfl, (size_t)fa.padded);
     if (e == hipSuccess) e = hipMalloc((void**)&s->mg_pz, sizeof(double) * (size_t)fa.padded);
@@ -1351,9 +1565,13 @@ hipError_t mg_setup(fe_scene* s) {
         pa.flags[q] = lv[q].flags;
     }
     if (s->tune.mg == FE_MG_FUSED) {
-        const FusedArgs fa = fused_args<TileFinest>(lv[0], lv[1]);
+        const FusedArgs fa = finest_args(lv[0], lv[1]);
         pa.tfl = s->mg_tfl;
         for (int a = 0; a < 3; ++a) pa.tiles[a] = fa.tiles[a];
+        const bool small = small_finest(lv[0]);
+        pa.rx = small ? TileCoarse::rx : TileFinest::rx;
+        pa.ry = small ? TileCoarse::ry : TileFinest::ry;
+        pa.rz = small ? TileCoarse::rz : TileFinest::rz;
     }
     const unsigned nb = (unsigned)(((lv[1].n[0] + 7) / 8) * ((lv[1].n[1] + 7) / 8) * ((lv[1].n[2] + 7) / 8));
     hipLaunchKernelGGL(k_mg_pyramid, dim3(nb), dim3(kPyrThreads), 0, s->stream, pa);
@@ -1411,6 +1629,21 @@ static void launch_tail(fe_scene* s, SolverScalars* st) {
     hipLaunchKernelGGL(k_mg_tail, dim3(1), dim3(kTailThreads), 0, s->stream, ta, (const float*)lv[T].b, lv[T].x2, st);
 }
 
+// Level q and the coarsest one below it, for k_mg_bottom.
+static BottomArgs bottom_args(const MGLevel& l, const MGLevel& c) {
+    BottomArgs a;
+    a.pf = a.pc = 1;
+    for (int q = 0; q < 3; ++q) {
+        a.n[q] = l.n[q];
+        a.c[q] = c.n[q];
+        a.ih2[q] = l.ih2[q];
+        a.cih2[q] = c.ih2[q];
+        a.pf *= l.n[q] + 2;
+        a.pc *= c.n[q] + 2;
+    }
+    return a;
+}
+
 // The fused V-cycle: level q's descent writes its pre-smoothed x2 and level
 // q+1's right-hand side; the tail leaves level T's result in lv[T].x2; level
 // q's ascent reads x2 and the coarse result and writes its own result to x
@@ -1421,36 +1654,57 @@ static hipError_t mg_apply_fused(fe_scene* s, const float* r, float* z, SolverSc
     std::vector<MGLevel>& lv = s->mg;
     const int T = s->mg_tail;
     lv[0].b = const_cast<float*>(r);
-    for (int q = 0; q < T; ++q) {
+    const bool small = small_finest(lv[0]);
+    auto down = [&](auto kernel, int q, const FusedArgs& a) {
         const MGLevel& l = lv[q];
         const MGLevel& c = lv[q + 1];
-        const FusedArgs a = q == 0 ? fused_args<TileFinest>(l, c) : fused_args<TileCoarse>(l, c);
         const dim3 grid((unsigned)a.padded);
         if (q == 0)
-            launch_timed(s, FE_KERNEL_MG_DOWN, tag, k_mg_down<true, TileFinest>, grid, dim3(kFusedThreads), a,
-                         (const float*)l.b, (const uint16_t*)l.code, l.x2, (const uint16_t*)c.code, c.b,
-                         (const SolverScalars*)st, pconf, nparts, (const uint8_t*)s->mg_tfl);
+            launch_timed(s, FE_KERNEL_MG_DOWN, tag, kernel, grid, dim3(kFusedThreads), a, (const float*)l.b,
+                         (const uint16_t*)l.code, l.x2, (const uint16_t*)c.code, c.b, (const SolverScalars*)st, pconf,
+                         nparts, (const uint8_t*)s->mg_tfl);
         else
-            hipLaunchKernelGGL((k_mg_down<false, TileCoarse>), grid, dim3(kFusedThreads), 0, s->stream, a, (const float*)l.b,
+            hipLaunchKernelGGL(kernel, grid, dim3(kFusedThreads), 0, s->stream, a, (const float*)l.b,
                                (const uint16_t*)l.code, l.x2, (const uint16_t*)c.code, c.b, (const SolverScalars*)st,
                                (const double*)nullptr, 0, (const uint8_t*)nullptr);
-    }
-    launch_tail(s, st);
-    for (int q = T - 1; q >= 0; --q) {
+    };
+    auto up = [&](auto kernel, int q, const FusedArgs& a) {
         const MGLevel& l = lv[q];
         const MGLevel& c = lv[q + 1];
-        const FusedArgs a = q == 0 ? fused_args<TileFinest>(l, c) : fused_args<TileCoarse>(l, c);
         const dim3 grid((unsigned)a.padded);
         const float* xc = q + 1 == T ? c.x2 : c.x;
         if (q == 0)
-            launch_timed(s, FE_KERNEL_MG_UP, tag, k_mg_up<true, TileFinest>, grid, dim3(kFusedThreads), a,
-                         (const float*)l.x2, xc, (const float*)l.b, (const uint16_t*)l.code, z, prz,
-                         (const SolverScalars*)st, (const uint8_t*)s->mg_tfl);
+            launch_timed(s, FE_KERNEL_MG_UP, tag, kernel, grid, dim3(kFusedThreads), a, (const float*)l.x2, xc,
+                         (const float*)l.b, (const uint16_t*)l.code, z, prz, (const SolverScalars*)st,
+                         (const uint8_t*)s->mg_tfl);
         else
-            hipLaunchKernelGGL((k_mg_up<false, TileCoarse>), grid, dim3(kFusedThreads), 0, s->stream, a, (const float*)l.x2, xc,
+            hipLaunchKernelGGL(kernel, grid, dim3(kFusedThreads), 0, s->stream, a, (const float*)l.x2, xc,
                                (const float*)l.b, (const uint16_t*)l.code, l.x, (double*)nullptr,
                                (const SolverScalars*)st, (const uint8_t*)nullptr);
-    }
+    };
+    const FusedArgs a0 = finest_args(lv[0], lv[1]);
+    if (small)
+        down(k_mg_down<true, TileCoarse>, 0, a0);
+    else
+        down(k_mg_down<true, TileFinest>, 0, a0);
+    // the last level above the coarsest goes with it into one workgroup, where
+    // their iterates fit its LDS (all but very long grids)
+    BottomArgs ba{};
+    const bool bottom = T >= 2 && T + 1 == (int)lv.size() &&
+                        2 * ((ba = bottom_args(lv[T - 1], lv[T])).pf + ba.pc) <= kBotLds;
+    const int B = bottom ? T - 1 : T;
+    for (int q = 1; q < B; ++q) down(k_mg_down<false, TileCoarse>, q, fused_args<TileCoarse>(lv[q], lv[q + 1]));
+    if (bottom)
+        hipLaunchKernelGGL(k_mg_bottom, dim3(1), dim3(kBotThreads), sizeof(float) * 2 * (ba.pf + ba.pc), s->stream, ba,
+                           (const float*)lv[B].b, (const uint16_t*)lv[B].code, (const uint16_t*)lv[T].code, lv[B].x,
+                           (const SolverScalars*)st);
+    else
+        launch_tail(s, st);
+    for (int q = B - 1; q > 0; --q) up(k_mg_up<false, TileCoarse>, q, fused_args<TileCoarse>(lv[q], lv[q + 1]));
+    if (small)
+        up(k_mg_up<true, TileCoarse>, 0, a0);
+    else
+        up(k_mg_up<true, TileFinest>, 0, a0);
     return hipGetLastError();
 }
 
