@@ -1251,6 +1251,16 @@ struct BottomArgs {
     int pf, pc;              // padded cells of each
 };
 
+// cell_ijk of a cell below 4096 without integer divisions: (c + 1/2) / n lies
+// at least 1 / (2 n) from an integer, and its rounding error is below
+// 4096 * 2^-22 / n.
+__device__ inline void small_cell_ijk(int c, int nx, int ny, float rx, float ry, int& i, int& j, int& k) {
+    const int q = (int)(((float)c + 0.5f) * rx);
+    i = c - q * nx;
+    k = (int)(((float)q + 0.5f) * ry);
+    j = q - k * ny;
+}
+
 // Offset of cell (i, j, k) in an array of dims n with a border of one.
 __device__ inline int bordered(int i, int j, int k, const int n[3]) {
     return (i + 1) + (n[0] + 2) * ((j + 1) + (n[1] + 2) * (k + 1));
@@ -1287,26 +1297,28 @@ __global__ __launch_bounds__(kBotThreads) void k_mg_bottom(BottomArgs a, const f
     }
     const bool con = (int)threadIdx.x < nc;
     const uint32_t ccd = con ? (uint32_t)ccode[threadIdx.x] : 0u;
-    for (int e = threadIdx.x; e < 2 * (a.pf + a.pc); e += kBotThreads) lds[e] = 0.0f;
+    for (int e = threadIdx.x; e < (2 * (a.pf + a.pc) + 3) / 4; e += kBotThreads)
+        reinterpret_cast<float4*>(lds)[e] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     constexpr MgSmooth SM = kMgCoarse;
     const CodeLanes fl = code_lanes(a.ih2, SM.omega), cl = code_lanes(a.cih2, 1.0f);
     const float nih2[3] = {-a.ih2[0], -a.ih2[1], -a.ih2[2]}, cnih2[3] = {-a.cih2[0], -a.cih2[1], -a.cih2[2]};
     const int sy = a.n[0] + 2, sz = sy * (a.n[1] + 2), csy = a.c[0] + 2, csz = csy * (a.c[1] + 2);
     float cen[kBotPer], wgt[kBotPer];
     int p[kBotPer];
+    const float rx = 1.0f / (float)a.n[0], ry = 1.0f / (float)a.n[1];
 #pragma unroll
     for (int u = 0; u < kBotPer; ++u) {
         const int li = code_lane(cd[u]);
         cen[u] = lane_read(fl.cen, li);
         wgt[u] = lane_read(fl.wgt, li);
         int i, j, k;
-        cell_ijk(threadIdx.x + u * kBotThreads, a.n[0], a.n[1], i, j, k);
+        small_cell_ijk(threadIdx.x + u * kBotThreads, a.n[0], a.n[1], rx, ry, i, j, k);
         p[u] = bordered(i, j, k, a.n);
     }
     const int cli = code_lane(ccd);
     const float ccen = lane_read(cl.cen, cli), cw = lane_read(cl.wgt, cli);
     int I, J, K;
-    cell_ijk(threadIdx.x, a.c[0], a.c[1], I, J, K);
+    small_cell_ijk(threadIdx.x, a.c[0], a.c[1], 1.0f / (float)a.c[0], 1.0f / (float)a.c[1], I, J, K);
     const int cp = bordered(I, J, K, a.c);
     const bool cfl = (ccd & kFluidBit) != 0;  // false where there is no cell
     __syncthreads();
@@ -1387,7 +1399,7 @@ __global__ __launch_bounds__(kBotThreads) void k_mg_bottom(BottomArgs a, const f
     for (int u = 0; u < kBotPer; ++u) {
         if (!(cd[u] & kFluidBit)) continue;
         int i, j, k;
-        cell_ijk(threadIdx.x + u * kBotThreads, a.n[0], a.n[1], i, j, k);
+        small_cell_ijk(threadIdx.x + u * kBotThreads, a.n[0], a.n[1], rx, ry, i, j, k);
         x2[u] = x2[u] + prolong_at3(i, j, k, a.c[0], a.c[1], a.c[2],
                                     [&](int A, int B, int C) { return V[bordered(A, B, C, a.c)]; });
         Y[p[u]] = x2[u];
@@ -1695,7 +1707,7 @@ static hipError_t mg_apply_fused(fe_scene* s, const float* r, float* z, SolverSc
     const int B = bottom ? T - 1 : T;
     for (int q = 1; q < B; ++q) down(k_mg_down<false, TileCoarse>, q, fused_args<TileCoarse>(lv[q], lv[q + 1]));
     if (bottom)
-        hipLaunchKernelGGL(k_mg_bottom, dim3(1), dim3(kBotThreads), sizeof(float) * 2 * (ba.pf + ba.pc), s->stream, ba,
+        hipLaunchKernelGGL(k_mg_bottom, dim3(1), dim3(kBotThreads), sizeof(float) * (2 * (ba.pf + ba.pc) + 3), s->stream, ba,
                            (const float*)lv[B].b, (const uint16_t*)lv[B].code, (const uint16_t*)lv[T].code, lv[B].x,
                            (const SolverScalars*)st);
     else
