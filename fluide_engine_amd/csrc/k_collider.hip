@@ -217,16 +217,25 @@ __global__ __launch_bounds__(kBlock) void k_sdf_extrapolate(Geom g, double* __re
 // ---------------------------------------------------------------------------
 // Mesh colliders: Mesh2SDF::Build (src/3d/mesh_2_sdf.cpp:14-95) of a
 // TriangleMeshCollider (src/3d/triangle_mesh_collider.cpp:5-9) on the
-// collider's own node grid, one thread per node looping over all triangles
-// (the loop index is uniform, so each triangle's vertices and index box are
-// scalar loads shared by the wave):
+// collider's own node grid:
 //   * distance: the minimum of DistanceToTriangle over the triangles whose
 //     index box holds the node, starting from max(h) * (nx + ny + nz);
 //   * sign: negated where TriangleMesh::IsInside (src/3d/triangle_mesh.cpp:120-163)
 //     holds, i.e. the summed half solid angles reach 2 pi - 0.001 in magnitude.
 // FP64 in the reference's operation order with contraction off, so the
-// distances are the reference's bit for bit; the angle sum goes through the
-// device atan2, which only feeds the threshold.
+// distances are the reference's bit for bit; the angle sum only feeds the
+// threshold.
+//
+// Bound by the FP64 operations of the angles, one term for each node and
+// triangle.  A term atan2(om, k) is the argument of k + i om, so the terms are
+// multiplied as complex numbers (4 operations instead of an atan2 each), with
+// the whole turns counted where a product passes the negative real axis, and
+// one atan2 at the end.  The three lengths in k come from the hardware's
+// reciprocal square root and one Newton step (relative error below 1e-14).
+// The waves of a workgroup take the same 64 nodes and a slice of the
+// triangles each; the loop index is uniform in a wave, so vertices and index
+// boxes are scalar loads, and a box that no node of the wave is in costs no
+// vector instruction.
 // ---------------------------------------------------------------------------
 struct D3 {
     double x, y, z;
@@ -312,10 +321,42 @@ __device__ inline double triangle_distance(const D3& x, const D3& p0, const D3& 
     return dlen(dsub(c, x));
 }
 
+// |a| from the square s of a length: 0 gives 1e-150, not 0 (the caller sees a
+// vanishing product).
+__device__ inline double quick_length(double s) {
+    s = fmax(s, 1e-300);
+    const double y = __builtin_amdgcn_rsq(s);
+    const double n = s * y;
+    return fma(0.5 * y, fma(-n, n, s), n);
+}
+
+// A sum of angles as a complex number of that argument (scaled at will) and
+// whole turns.  The sign bit of `im` tells the halves apart, so that +0 and -0
+// on the negative axis stand for +pi and -pi, as in atan2.
+struct AngleSum {
+    double re = 1.0, im = 0.0;
+    int turns = 0;
+};
+
+// Adds atan2(om, k).  Two angles of one half add up to one of the other only
+// by passing the negative axis; both products in `im` then have one sign, so
+// rounding cannot hide it.
+__device__ inline void add_angle(AngleSum& z, double k, double om) {
+    const double re = fma(z.re, k, -(z.im * om)), im = fma(z.re, om, z.im * k);
+    const int a = __double2hiint(z.im), b = __double2hiint(om), c = __double2hiint(im);
+    const int passed = (~(a ^ b) & (a ^ c)) >> 31;  // -1 or 0
+    z.turns += passed & ((a >> 31) | 1);
+    // keep the larger part in [0.5, 1)
+    const int e = -__builtin_amdgcn_frexp_exp(fmax(fabs(re), fabs(im)));
+    z.re = __builtin_amdgcn_ldexp(re, e);
+    z.im = __builtin_amdgcn_ldexp(im, e);
+}
+
 // One triangle's term of TriangleMesh::IsInside: atan2(det[A B C],
 // |A||B||C| + |C| A.B + |A| B.C + |B| C.A), A, B, C = vertices - x, the
-// determinant in ADet's term order (:154-163).
-__device__ inline double half_solid_angle(const D3& x, const D3& p0, const D3& p1, const D3& p2) {
+// determinant in ADet's term order (:154-163), whose sign decides between +pi
+// and -pi for a node in the triangle's plane.
+__device__ inline void add_half_solid_angle(AngleSum& z, const D3& x, const D3& p0, const D3& p1, const D3& p2) {
 #pragma clang fp contract(off)
     const D3 A = dsub(p0, x), B = dsub(p1, x), C = dsub(p2, x);
     double omega = A.x * B.y * C.z;
@@ -324,38 +365,69 @@ __device__ inline double half_solid_angle(const D3& x, const D3& p0, const D3& p
     omega -= C.x * B.y * A.z;
     omega -= B.x * A.y * C.z;
     omega -= A.x * C.y * B.z;
-    const double nA = dlen(A), nB = dlen(B), nC = dlen(C);
-    double k = nA * nB * nC;
-    k += nC * ddot(A, B);
-    k += nA * ddot(B, C);
-    k += nB * ddot(C, A);
-    return atan2(omega, k);
+    auto dot = [](const D3& a, const D3& b) { return fma(a.z, b.z, fma(a.y, b.y, a.x * b.x)); };
+    const double nA = quick_length(dot(A, A)), nB = quick_length(dot(B, B)), nC = quick_length(dot(C, C));
+    const double n3 = nA * nB * nC;
+    double k = fma(nB, dot(C, A), fma(nA, dot(B, C), fma(nC, dot(A, B), n3)));
+    if (fabs(omega) + fabs(k) <= 1e-9 * n3) {
+        // a node on an edge or a vertex, where k is rounding: the reference's own
+        const double lA = dlen(A), lB = dlen(B), lC = dlen(C);
+        k = lA * lB * lC;
+        k += lC * ddot(A, B);
+        k += lA * ddot(B, C);
+        k += lB * ddot(C, A);
+        if (k == 0.0 && omega == 0.0) k = 1.0;  // atan2(0, 0) is 0
+    }
+    add_angle(z, k, omega);
 }
 
 constexpr double kPi = 3.14159265358979323846;  // src/common/math_utils.hpp:11
 
 // tv: 9 doubles per triangle (its three vertices); tb: 6 ints per triangle,
 // the index box i0, j0, k0, i1, j1, k1 (inclusive).
-__global__ __launch_bounds__(kBlock) void k_mesh_sdf(NodeGrid3 G, const double* __restrict__ tv,
-                                                     const int32_t* __restrict__ tb, int64_t nt, double fill,
-                                                     double* __restrict__ out) {
+template <int SLICES>
+__global__ __launch_bounds__(64 * SLICES) void k_mesh_sdf(NodeGrid3 G, const double* __restrict__ tv,
+                                                          const int32_t* __restrict__ tb, int64_t nt, double fill,
+                                                          double* __restrict__ out) {
 #pragma clang fp contract(off)
-    const int64_t c = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    __shared__ double sd[SLICES][64], sa[SLICES][64];
+    const int lane = threadIdx.x & 63, slice = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int64_t nn = (int64_t)G.n[0] * G.n[1] * G.n[2];
-    if (c >= nn) return;
+    const int64_t c0 = (int64_t)blockIdx.x * 64, c = c0 + lane, c1 = min(c0 + 63, nn - 1);
     int i, j, k;
-    split_index(c, G.n[0], G.n[1], i, j, k);
+    split_index(min(c, nn - 1), G.n[0], G.n[1], i, j, k);
+    // bounds of the wave's nodes
+    int j0, k0, j1, k1, t0, t1;
+    split_index(c0, G.n[0], G.n[1], t0, j0, k0);
+    split_index(c1, G.n[0], G.n[1], t1, j1, k1);
+    const bool row = j0 == j1 && k0 == k1, plane = k0 == k1;
+    const int wi0 = row ? t0 : 0, wi1 = row ? t1 : G.n[0] - 1;
+    const int wj0 = plane ? j0 : 0, wj1 = plane ? j1 : G.n[1] - 1;
     const D3 x{G.o[0] + (double)i * G.h[0], G.o[1] + (double)j * G.h[1], G.o[2] + (double)k * G.h[2]};
-    double d = fill, ret = 0;
-    for (int64_t t = 0; t < nt; ++t) {
+    double d = fill;
+    AngleSum z;
+    const int64_t per = (nt + SLICES - 1) / SLICES, end = min(per * (slice + 1), nt);
+    for (int64_t t = per * slice; t < end; ++t) {
         const double* P = tv + 9 * t;
         const int32_t* B = tb + 6 * t;
         const D3 p0{P[0], P[1], P[2]}, p1{P[3], P[4], P[5]}, p2{P[6], P[7], P[8]};
-        if (i >= B[0] && j >= B[1] && k >= B[2] && i <= B[3] && j <= B[4] && k <= B[5]) {
-            const double dist = triangle_distance(x, p0, p1, p2);
-            if (dist < d) d = dist;
+        if (B[0] <= wi1 && B[3] >= wi0 && B[1] <= wj1 && B[4] >= wj0 && B[2] <= k1 && B[5] >= k0) {
+            if (i >= B[0] && j >= B[1] && k >= B[2] && i <= B[3] && j <= B[4] && k <= B[5]) {
+                const double dist = triangle_distance(x, p0, p1, p2);
+                if (dist < d) d = dist;
+            }
         }
-        ret += half_solid_angle(x, p0, p1, p2);
+        add_half_solid_angle(z, x, p0, p1, p2);
+    }
+    sd[slice][lane] = d;
+    sa[slice][lane] = fma(2.0 * kPi, (double)z.turns, atan2(z.im, z.re));
+    __syncthreads();
+    if (slice != 0 || c >= nn) return;
+    double ret = 0.0;
+#pragma unroll
+    for (int q = 0; q < SLICES; ++q) {
+        if (sd[q][lane] < d) d = sd[q][lane];
+        ret += sa[q][lane];
     }
     if (fabs(ret) >= 2.0 * kPi - 0.001) d = d * -1.0;
     out[c] = d;
@@ -420,10 +492,15 @@ bool mesh_prepare(const NodeGrid3& G, const double* verts, int64_t nv, const int
     return true;
 }
 
+constexpr int64_t kManySlices = 1 << 17;
 hipError_t launch_mesh_sdf(hipStream_t st, const NodeGrid3& G, const double* tv_dev, const int32_t* tb_dev,
                            int64_t nt, double fill, double* out) {
     const int64_t nn = (int64_t)G.n[0] * G.n[1] * G.n[2];
-    hipLaunchKernelGGL(k_mesh_sdf, grid_n(nn), dim3(kBlock), 0, st, G, tv_dev, tb_dev, nt, fill, out);
+    const dim3 grid((unsigned)((nn + 63) / 64));
+    if (nn <= kManySlices)
+        hipLaunchKernelGGL(k_mesh_sdf<16>, grid, dim3(64 * 16), 0, st, G, tv_dev, tb_dev, nt, fill, out);
+    else
+        hipLaunchKernelGGL(k_mesh_sdf<4>, grid, dim3(64 * 4), 0, st, G, tv_dev, tb_dev, nt, fill, out);
     return hipGetLastError();
 }
 

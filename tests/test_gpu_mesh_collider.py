@@ -54,6 +54,22 @@ def test_mesh_sdf_bit_exact(ctx, name, grid):
     assert (got < 0).sum() > 0
 
 
+@pytest.mark.parametrize("size,levels", [((3, 3, 3), 0), ((5, 13, 1), 1), ((64, 2, 33), 2), ((51, 53, 49), 0)])
+def test_mesh_sdf_nodes_on_the_mesh(ctx, size, levels):
+    """Fewer nodes than a wavefront, ragged rows, fewer triangles than slices
+    and both slice counts; a box whose faces, edges and corners hold nodes
+    (spacing and corners exact in binary), beside an icosphere and a single
+    open triangle."""
+    print(f"[gpu] mesh sdf nodes on the mesh size={size}", flush=True)
+    h = (1 / 16,) * 3
+    v1, t1 = box((1 / 16, 1 / 16, 0.0), (2 / 16, 3 / 16, 2 / 16))
+    for v, t in ((v1, t1), (v1[:3], np.array([[0, 1, 2]], np.int32)),
+                 icosphere((1.3, 1.4, 1.1), 0.8, levels=levels)):
+        got = capi.mesh_sdf(ctx, size, (0.0, 0.0, 0.0), h, v, t)
+        want = orc.mesh_to_sdf(size, (0.0, 0.0, 0.0), h, v, t)
+        assert np.array_equal(got, want), (int((got != want).sum()), float(np.abs(got - want).max()))
+
+
 def test_mesh_sdf_errors(ctx):
     print("[gpu] mesh sdf errors", flush=True)
     v, t = box((0.2, 0.2, 0.2), (0.5, 0.5, 0.5))
