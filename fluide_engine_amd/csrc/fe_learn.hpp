@@ -23,6 +23,7 @@ constexpr int kNetLayers = 7;  // enc0..enc3, dec2, dec1, dec0
 constexpr int kNetIn = 16;     // input channels (3 used)
 constexpr int kNetLayerIn[kNetLayers] = {16, 16, 32, 48, 112, 80, 48};
 constexpr int kNetLayerOut[kNetLayers] = {16, 32, 48, 64, 48, 32, 16};
+constexpr int kNetLayerLevel[kNetLayers] = {0, 1, 2, 3, 2, 1, 0};
 
 struct NetLayer {
     int cin = 0, cout = 0;
@@ -82,8 +83,9 @@ struct fe_net {
     float *gD0 = nullptr, *gC0 = nullptr, *gE0 = nullptr, *gD1 = nullptr, *gC1 = nullptr, *gE1 = nullptr,
           *gP1 = nullptr, *gD2 = nullptr, *gC2 = nullptr, *gE2 = nullptr, *gP2 = nullptr, *gE3 = nullptr,
           *gP3 = nullptr;
-    float* wpart = nullptr;  // weight-gradient partials
-    int64_t wpart_cap = 0;
+    float *wpart = nullptr, *bpart = nullptr;  // weight- and bias-gradient partials
+    uint16_t* Xt[4] = {nullptr, nullptr, nullptr, nullptr};  // per level: a layer's input as zero-bordered planes
+    uint16_t* Gt[4] = {nullptr, nullptr, nullptr, nullptr};  // and its dpre as planes
     double* red = nullptr;   // reduction partials (FP64)
     int64_t red_cap = 0;
     float* losses = nullptr; // per training step

@@ -11,8 +11,8 @@
 // + j], B[4 (l / 16) + j][l % 16] and returns C[4 (l / 16) + i][l % 16].
 // The backward data pass is the same kernel on the flipped, transposed weights;
 // the weight gradient is a GEMM over voxels (M = input channel, N = output
-// channel, K = voxel), one partial per wavefront summed in a fixed order, so
-// every gradient is reproducible run to run.
+// channel, K = voxel) on channel planes, one partial per workgroup summed in a
+// fixed order, so every gradient is reproducible run to run.
 #include <algorithm>
 #include <cmath>
 #include <vector>
@@ -139,84 +139,238 @@ __global__ __launch_bounds__(256) void k_pack(int cin, int cout, const float* __
 }
 
 // ---------------------------------------------------------------------------
-// Weight gradient: dW[t][ci][co] = sum_v X[v + off(t)][ci] * G[v][co]
+// Weight gradient: dW[t][ci][co] = sum_v X[v + off(t)][ci] * G[v][co], and the
+// bias gradient db[co] = sum_v G[v][co].
+//
+// The contraction runs over voxels, so both operands are taken from channel
+// planes, where a lane's 8 voxels are one 16-byte load.  Rows are filled up to
+// segments of 8 voxels: G as [co][segment], zero in the fill, X as
+// [ci][nz + 2][ny + 2][row] with a border of zeros (8 wide in x, which keeps
+// rows aligned), so no tap tests bounds.  A wavefront holds the 9 taps of one z offset
+// for 16 input channels and all output channels: per y offset one 16-byte and
+// two 4-byte loads give all three x offsets by shifting, so 9 NT matrix
+// instructions (v_mfma_f32_16x16x32_bf16) take 3 + NT wide loads.  Bound by
+// the first-level cache's loads.  The bias is one more product, with ones.
+// At 64x96x80, the layers of the finest level (48 -> 16 and 16 -> 16
+// channels): 450 and 417 us with one tap per wavefront and 2-byte loads.
 // ---------------------------------------------------------------------------
-template <int KC, int NT>
-__global__ __launch_bounds__(256) void k_wgrad(Lv d, const uint16_t* __restrict__ X, const uint16_t* __restrict__ G,
-                                               float* __restrict__ part, int64_t vpw) {
-    const int wave = threadIdx.x >> 6, l = threadIdx.x & 63;
-    const int t = blockIdx.y;
-    const int64_t pw = (int64_t)blockIdx.x * 4 + wave;
-    const int64_t v0 = pw * vpw, v1 = min(v0 + vpw, d.V);
-    const int row = l & 15, kq = l >> 4;
-    constexpr int cin = KC * 16, cout = NT * 16;
-    const int dx = t % 3 - 1, dy = (t / 3) % 3 - 1, dz = t / 9 - 1;
-    const int64_t off = dx + (int64_t)dy * d.nx + (int64_t)dz * d.nx * d.ny;
-    f4 acc[KC][NT];
+typedef __bf16 b8 __attribute__((ext_vector_type(8)));
+typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+
+constexpr int kEdge = 8;  // the zero border of X's rows
+
+struct Planes {
+    int nx8;         // segments of a row
+    int px, py;      // X: row length and rows of a z slice
+    int64_t xn, gn;  // elements of a channel's plane of X and G
+    int64_t steps;   // 4 segments each, the last one's rest zero in G
+};
+__host__ __device__ inline Planes planes_of(const Lv& d) {
+    Planes P;
+    P.nx8 = (d.nx + 7) / 8;
+    P.px = 8 * P.nx8 + 2 * kEdge;
+    P.py = d.ny + 2;
+    P.xn = (int64_t)P.px * P.py * (d.nz + 2);
+    P.steps = ((int64_t)P.nx8 * d.ny * d.nz + 3) / 4;
+    P.gn = 32 * P.steps;
+    return P;
+}
+
+constexpr int kMaxCh = 112;
+
+// A workgroup's 8 segments of a channel-last array, as pairs of channels:
+// f(voxel, channel pair) gives a pair's bits; they go to channel planes (X's
+// or G's place for each segment) by way of LDS (rows of C + 2: the transposed
+// reads spread over the banks).  The fill of a segment is zero.
+template <bool IS_X, typename F>
+__device__ inline void segments_to_planes(const Lv& d, int C, uint16_t* __restrict__ out, F f) {
+    __shared__ uint16_t lds[64 * (kMaxCh + 2)];
+    __shared__ int64_t voxel[8], place[8];
+    __shared__ int count[8];
+    const Planes P = planes_of(d);
+    if (threadIdx.x < 8) {
+        const int64_t seg = (int64_t)blockIdx.x * 8 + threadIdx.x, r = seg / P.nx8;
+        const int x = 8 * (int)(seg - r * P.nx8);
+        const int64_t z = r / d.ny;
+        const int y = (int)(r - z * d.ny);
+        voxel[threadIdx.x] = r * d.nx + x;
+        place[threadIdx.x] = IS_X ? ((z + 1) * P.py + (y + 1)) * P.px + kEdge + x : 8 * seg;
+        count[threadIdx.x] = z < d.nz ? min(8, d.nx - x) : 0;
+    }
+    __syncthreads();
+    const int half = C / 2;
+    for (int e = threadIdx.x; e < 64 * half; e += 256) {
+        const int slot = e / half, pair = e - slot * half;
+        uint32_t w = 0;
+        if ((slot & 7) < count[slot >> 3]) w = f(voxel[slot >> 3] + (slot & 7), pair);
+        *reinterpret_cast<uint32_t*>(lds + slot * (C + 2) + 2 * pair) = w;
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < C * 8; e += 256) {
+        const int c = e >> 3, q = e & 7;
+        if (count[q] == 0) continue;
+        u4 w;
 #pragma unroll
-    for (int kc = 0; kc < KC; ++kc)
+        for (int h = 0; h < 4; ++h)
+            w[h] = (uint32_t)lds[(8 * q + 2 * h) * (C + 2) + c] |
+                   ((uint32_t)lds[(8 * q + 2 * h + 1) * (C + 2) + c] << 16);
+        *reinterpret_cast<u4*>(out + c * (IS_X ? P.xn : P.gn) + place[q]) = w;
+    }
+}
+
+// Channel-last X to planes (their border is zero from the allocation on).
+__global__ __launch_bounds__(256) void k_planes(Lv d, int C, const uint16_t* __restrict__ X,
+                                                uint16_t* __restrict__ Xt) {
+    const uint32_t* in = reinterpret_cast<const uint32_t*>(X);
+    segments_to_planes<true>(d, C, Xt, [&](int64_t v, int pair) { return in[v * (C / 2) + pair]; });
+}
+
+// dpre = bf16(y > 0 ? g : 0), channel-last and as planes
+__global__ __launch_bounds__(256) void k_mask(Lv d, int C, const float* __restrict__ g,
+                                              const uint16_t* __restrict__ y, uint16_t* __restrict__ dpre,
+                                              uint16_t* __restrict__ Gt) {
+    const float2* gi = reinterpret_cast<const float2*>(g);
+    const uint32_t* yi = reinterpret_cast<const uint32_t*>(y);
+    uint32_t* o = reinterpret_cast<uint32_t*>(dpre);
+    auto mask = [](uint32_t h, float v) { return h != 0 && !(h & 0x8000u) ? (uint32_t)to_bf16(v) : 0u; };
+    segments_to_planes<false>(d, C, Gt, [&](int64_t v, int pair) {
+        const int64_t e = v * (C / 2) + pair;
+        const float2 a = gi[e];
+        const uint32_t h = yi[e];
+        const uint32_t w = mask(h & 0xFFFFu, a.x) | (mask(h >> 16, a.y) << 16);
+        o[e] = w;
+        return w;
+    });
+}
+
+__device__ inline b8 as_b8(const u4& w) { return __builtin_bit_cast(b8, w); }
+
+// blockIdx.y = 3 kc + dz (16 input channels, z offset dz - 1).  Wave w of block
+// b takes the 32-voxel steps [ (4 b + w) spw, ... + spw ).
+template <int NT>
+__global__ __launch_bounds__(256) void k_wgrad(Lv d, int cin, const uint16_t* __restrict__ Xt,
+                                               const uint16_t* __restrict__ Gt, float* __restrict__ part,
+                                               float* __restrict__ bpart, int64_t spw) {
+    __shared__ float sm[4][NT * 256];
+    const int wave = threadIdx.x >> 6, l = threadIdx.x & 63, row = l & 15, kq = l >> 4;
+    const int kc = blockIdx.y / 3, dz = blockIdx.y % 3;
+    constexpr int cout = NT * 16;
+    const Planes P = planes_of(d);
+    const int64_t s0 = min((4 * (int64_t)blockIdx.x + wave) * spw, P.steps), s1 = min(s0 + spw, P.steps);
+    // this lane's 8 voxels: segment 4 s + kq (past the last one G is zero, and
+    // X is read at the last z)
+    const int nx8 = P.nx8;
+    int x8 = 0, y = 0, z = 0;
+    {
+        const int64_t seg = 4 * s0 + kq, r = seg / nx8;
+        x8 = (int)(seg - r * nx8);
+        z = (int)(r / d.ny);
+        y = (int)(r - (int64_t)z * d.ny);
+    }
+    const uint16_t* xp = Xt + (int64_t)(kc * 16 + row) * P.xn + kEdge;
+    const uint16_t* gp = Gt + (int64_t)row * P.gn + 8 * kq;
+    const bool bias = kc == 0 && dz == 1;  // uniform
+    f4 acc[9][NT], accb[NT];
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) acc[kc][nt] = f4{0.f, 0.f, 0.f, 0.f};
-    for (int64_t vs = v0; vs < v1; vs += 16) {
-        s4 a[KC], b[NT];
+    for (int nt = 0; nt < NT; ++nt) {
+        accb[nt] = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int64_t v = vs + 4 * kq + j;
-            const bool vin = v < v1;
-            int x = 0, y = 0, z = 0;
-            if (vin) decode(d, v, x, y, z);
-            const bool ok = vin && (unsigned)(x + dx) < (unsigned)d.nx && (unsigned)(y + dy) < (unsigned)d.ny &&
-                            (unsigned)(z + dz) < (unsigned)d.nz;
-            const int64_t u = ok ? v + off : 0;
+        for (int t = 0; t < 9; ++t) acc[t][nt] = f4{0.f, 0.f, 0.f, 0.f};
+    }
+    const b8 ones = as_b8(u4{0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u});
+    for (int64_t s = s0; s < s1; ++s) {
+        b8 b[NT];
 #pragma unroll
-            for (int kc = 0; kc < KC; ++kc) a[kc][j] = ok ? (short)X[u * cin + kc * 16 + row] : (short)0;
+        for (int nt = 0; nt < NT; ++nt)
+            b[nt] = as_b8(*reinterpret_cast<const u4*>(gp + (int64_t)nt * 16 * P.gn + 32 * s));
+        u4 m[3];
+        uint32_t lo[3], hi[3];
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt) b[nt][j] = vin ? (short)G[v * cout + nt * 16 + row] : (short)0;
+        for (int dy = 0; dy < 3; ++dy) {
+            const uint16_t* p = xp + ((int64_t)(min(z, d.nz - 1) + dz) * P.py + (y + dy)) * P.px + 8 * x8;
+            m[dy] = *reinterpret_cast<const u4*>(p);
+            lo[dy] = *reinterpret_cast<const uint32_t*>(p - 2);
+            hi[dy] = *reinterpret_cast<const uint32_t*>(p + 8);
         }
 #pragma unroll
-        for (int kc = 0; kc < KC; ++kc)
+        for (int dy = 0; dy < 3; ++dy) {
+            const uint32_t a01 = __builtin_amdgcn_alignbit(m[dy][1], m[dy][0], 16),
+                           a12 = __builtin_amdgcn_alignbit(m[dy][2], m[dy][1], 16),
+                           a23 = __builtin_amdgcn_alignbit(m[dy][3], m[dy][2], 16);
+            const b8 left = as_b8(u4{__builtin_amdgcn_alignbit(m[dy][0], lo[dy], 16), a01, a12, a23}),
+                     mid = as_b8(m[dy]),
+                     right = as_b8(u4{a01, a12, a23, __builtin_amdgcn_alignbit(hi[dy], m[dy][3], 16)});
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) {
+                acc[3 * dy][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(left, b[nt], acc[3 * dy][nt], 0, 0, 0);
+                acc[3 * dy + 1][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(mid, b[nt], acc[3 * dy + 1][nt], 0, 0, 0);
+                acc[3 * dy + 2][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(right, b[nt], acc[3 * dy + 2][nt], 0, 0, 0);
+            }
+        }
+        if (bias) {
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt)
-                acc[kc][nt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[kc], b[nt], acc[kc][nt], 0, 0, 0);
+                accb[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, b[nt], accb[nt], 0, 0, 0);
+        }
+        x8 += 4;
+        while (x8 >= nx8) {
+            x8 -= nx8;
+            if (++y == d.ny) {
+                y = 0;
+                ++z;
+            }
+        }
     }
-    float* P = part + (pw * 27 + t) * (int64_t)cin * cout;
+    // the block's sum, waves in order, tap by tap
 #pragma unroll
-    for (int kc = 0; kc < KC; ++kc)
+    for (int t = 0; t < 9; ++t) {
+        __syncthreads();
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) P[(kc * 16 + 4 * kq + i) * cout + nt * 16 + row] = acc[kc][nt][i];
-}
-
-// out[i] = sum_p part[p * size + i], p ascending
-__global__ __launch_bounds__(256) void k_reduce_parts(int64_t nparts, int64_t size, const float* __restrict__ part,
-                                                      float* __restrict__ out) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= size) return;
-    float s = 0.0f;
-    for (int64_t p = 0; p < nparts; ++p) s += part[p * size + i];
-    out[i] = s;
-}
-
-// per-block column sums of a BF16 [V][C] array (bias gradients)
-__global__ __launch_bounds__(256) void k_colsum(int64_t V, int C, const uint16_t* __restrict__ G,
-                                                float* __restrict__ part, int64_t chunk) {
-    __shared__ float sm[256];
-    const int R = 256 / C;
-    const int tid = threadIdx.x;
-    const int64_t b0 = (int64_t)blockIdx.x * chunk, b1 = min(b0 + chunk, V);
-    float s = 0.0f;
-    if (tid < R * C) {
-        const int c = tid % C, r = tid / C;
-        for (int64_t v = b0 + r; v < b1; v += R) s += from_bf16(G[v * C + c]);
+            for (int i = 0; i < 4; ++i) sm[wave][(4 * kq + i) * cout + nt * 16 + row] = acc[t][nt][i];
+        __syncthreads();
+        float* o = part + (((int64_t)blockIdx.x * 27 + 9 * dz + t) * cin + kc * 16) * cout;
+#pragma unroll
+        for (int e = 0; e < NT; ++e) {
+            const int i = threadIdx.x + 256 * e;
+            o[i] = ((sm[0][i] + sm[1][i]) + sm[2][i]) + sm[3][i];
+        }
     }
-    sm[tid] = s;
+    if (bias) {  // every row of ones . G is the column sum
+        __syncthreads();
+        if (kq == 0) {
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) sm[wave][nt * 16 + row] = accb[nt][0];
+        }
+        __syncthreads();
+        if (threadIdx.x < cout) {
+            const int i = threadIdx.x;
+            bpart[(int64_t)blockIdx.x * cout + i] = ((sm[0][i] + sm[1][i]) + sm[2][i]) + sm[3][i];
+        }
+    }
+}
+
+// out[i] = sum_p part[p * size + i] for the weights and, behind them, the
+// biases: 16 outputs per block, the partials dealt to 16 threads each and
+// their sums added in order.
+__global__ __launch_bounds__(256) void k_reduce_parts(int nparts, int64_t wsize, const float* __restrict__ wpart,
+                                                      float* __restrict__ w, int bsize,
+                                                      const float* __restrict__ bpart, float* __restrict__ b) {
+    __shared__ float sm[16][17];
+    const int col = threadIdx.x & 15, sl = threadIdx.x >> 4;
+    int64_t i = (int64_t)blockIdx.x * 16 + col;  // both sizes are multiples of 16
+    const bool isw = i < wsize;
+    if (!isw) i -= wsize;
+    const float* part = isw ? wpart : bpart;
+    const int64_t size = isw ? wsize : bsize;
+    float s = 0.0f;
+    for (int p = sl; p < nparts; p += 16) s += part[p * size + i];
+    sm[sl][col] = s;
     __syncthreads();
-    if (tid < C) {
-        float t = 0.0f;
-        for (int r = 0; r < R; ++r) t += sm[r * C + tid];
-        part[(int64_t)blockIdx.x * C + tid] = t;
-    }
+    if (sl != 0) return;
+    for (int q = 1; q < 16; ++q) s += sm[q][col];
+    (isw ? w : b)[i] = s;
 }
 
 // ---------------------------------------------------------------------------
@@ -385,15 +539,6 @@ __global__ __launch_bounds__(256) void k_codes(Lv d, const uint8_t* __restrict__
                        (uint32_t)d.nz);
 }
 
-// dpre = bf16(y > 0 ? g : 0)
-__global__ __launch_bounds__(256) void k_mask(int64_t n, const float* __restrict__ g, const uint16_t* __restrict__ y,
-                                              uint16_t* __restrict__ dpre) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    const uint16_t h = y[i];
-    dpre[i] = (h != 0 && !(h & 0x8000)) ? to_bf16(g[i]) : (uint16_t)0;
-}
-
 // gCoarse[p][c] = sum over the 8 children of gC[child][c], c < Cc
 __global__ __launch_bounds__(256) void k_up_bwd(Lv f, Lv c, int Cc, int Ct, const float* __restrict__ gC,
                                                 float* __restrict__ gCoarse) {
@@ -534,29 +679,30 @@ hipError_t launch_conv(hipStream_t st, const Lv& d, const uint16_t* X, int cin, 
     return hipGetLastError();
 }
 
-int64_t wgrad_vpw(int64_t V) {
-    int64_t vpw = (V + 255) / 256;
-    vpw = std::max<int64_t>(16, (vpw + 15) / 16 * 16);
-    return vpw;
-}
-int64_t wgrad_parts(int64_t V) {
-    const int64_t waves = (V + wgrad_vpw(V) - 1) / wgrad_vpw(V);
-    return (waves + 3) / 4 * 4;
+// Workgroups along the voxels: about 16 waves per CU in all, and a few steps
+// (32 voxels each) per wave at least.
+struct WgradShape {
+    int64_t spw;  // steps per wave
+    int blocks;   // partials
+};
+WgradShape wgrad_shape(const Lv& d, int cin) {
+    const int64_t steps = planes_of(d).steps;
+    const int64_t want = 4096 / (4 * 3 * (cin / 16)), most = std::max<int64_t>(1, steps / 16);
+    const int64_t blocks = std::max<int64_t>(1, std::min(want, most));
+    WgradShape w;
+    w.spw = (steps + 4 * blocks - 1) / (4 * blocks);
+    w.blocks = (int)((steps + 4 * w.spw - 1) / (4 * w.spw));
+    return w;
 }
 
-hipError_t launch_wgrad(hipStream_t st, const Lv& d, const uint16_t* X, int cin, const uint16_t* G, int cout,
-                        float* part) {
-    const int64_t vpw = wgrad_vpw(d.V);
-    const dim3 grid((unsigned)(wgrad_parts(d.V) / 4), 27);
-    const int key = (cin / 16) * 10 + cout / 16;
-    switch (key) {
-        case 11: hipLaunchKernelGGL((k_wgrad<1, 1>), grid, dim3(256), 0, st, d, X, G, part, vpw); break;
-        case 12: hipLaunchKernelGGL((k_wgrad<1, 2>), grid, dim3(256), 0, st, d, X, G, part, vpw); break;
-        case 23: hipLaunchKernelGGL((k_wgrad<2, 3>), grid, dim3(256), 0, st, d, X, G, part, vpw); break;
-        case 34: hipLaunchKernelGGL((k_wgrad<3, 4>), grid, dim3(256), 0, st, d, X, G, part, vpw); break;
-        case 73: hipLaunchKernelGGL((k_wgrad<7, 3>), grid, dim3(256), 0, st, d, X, G, part, vpw); break;
-        case 52: hipLaunchKernelGGL((k_wgrad<5, 2>), grid, dim3(256), 0, st, d, X, G, part, vpw); break;
-        case 31: hipLaunchKernelGGL((k_wgrad<3, 1>), grid, dim3(256), 0, st, d, X, G, part, vpw); break;
+hipError_t launch_wgrad(hipStream_t st, const Lv& d, const uint16_t* Xt, int cin, const uint16_t* Gt, int cout,
+                        float* part, float* bpart, const WgradShape& w) {
+    const dim3 grid((unsigned)w.blocks, (unsigned)(3 * (cin / 16)));
+    switch (cout / 16) {
+        case 1: hipLaunchKernelGGL(k_wgrad<1>, grid, dim3(256), 0, st, d, cin, Xt, Gt, part, bpart, w.spw); break;
+        case 2: hipLaunchKernelGGL(k_wgrad<2>, grid, dim3(256), 0, st, d, cin, Xt, Gt, part, bpart, w.spw); break;
+        case 3: hipLaunchKernelGGL(k_wgrad<3>, grid, dim3(256), 0, st, d, cin, Xt, Gt, part, bpart, w.spw); break;
+        case 4: hipLaunchKernelGGL(k_wgrad<4>, grid, dim3(256), 0, st, d, cin, Xt, Gt, part, bpart, w.spw); break;
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
@@ -583,8 +729,12 @@ void free_buffers(fe_net* n) {
     release(n->D0f);
     release(n->gD0); release(n->gC0); release(n->gE0); release(n->gD1); release(n->gC1); release(n->gE1);
     release(n->gP1); release(n->gD2); release(n->gC2); release(n->gE2); release(n->gP2); release(n->gE3);
-    release(n->gP3); release(n->wpart); release(n->red);
-    n->wpart_cap = n->red_cap = 0;
+    release(n->gP3); release(n->wpart); release(n->bpart); release(n->red);
+    for (int l = 0; l < 4; ++l) {
+        release(n->Xt[l]);
+        release(n->Gt[l]);
+    }
+    n->red_cap = 0;
     for (auto& l : n->lv) l = NetLevel{};
 }
 
@@ -594,16 +744,15 @@ hipError_t layer_back(fe_net* n, int li, const Lv& d, const uint16_t* X, const u
     NetLayer& L = n->L[li];
     hipStream_t st = n->stream;
     hipError_t e;
-    const int64_t ny = d.V * L.cout;
-    hipLaunchKernelGGL(k_mask, g1(ny), dim3(256), 0, st, ny, gY, Y, n->dpre);
-    if ((e = launch_wgrad(st, d, X, L.cin, n->dpre, L.cout, n->wpart)) != hipSuccess) return e;
+    const dim3 segments((unsigned)((planes_of(d).steps + 1) / 2));  // 8 per workgroup
+    uint16_t *Xt = n->Xt[kNetLayerLevel[li]], *Gt = n->Gt[kNetLayerLevel[li]];
+    hipLaunchKernelGGL(k_mask, segments, dim3(256), 0, st, d, L.cout, gY, Y, n->dpre, Gt);
+    hipLaunchKernelGGL(k_planes, segments, dim3(256), 0, st, d, L.cin, X, Xt);
+    const WgradShape w = wgrad_shape(d, L.cin);
+    if ((e = launch_wgrad(st, d, Xt, L.cin, Gt, L.cout, n->wpart, n->bpart, w)) != hipSuccess) return e;
     const int64_t wsz = 27LL * L.cin * L.cout;
-    hipLaunchKernelGGL(k_reduce_parts, g1(wsz), dim3(256), 0, st, wgrad_parts(d.V), wsz, (const float*)n->wpart, L.gw);
-    const int nb = (int)std::min<int64_t>(256, (d.V + 255) / 256);
-    const int64_t chunk = (d.V + nb - 1) / nb;
-    hipLaunchKernelGGL(k_colsum, dim3(nb), dim3(256), 0, st, d.V, L.cout, (const uint16_t*)n->dpre, n->wpart, chunk);
-    hipLaunchKernelGGL(k_reduce_parts, g1(L.cout), dim3(256), 0, st, (int64_t)nb, (int64_t)L.cout,
-                       (const float*)n->wpart, L.gb);
+    hipLaunchKernelGGL(k_reduce_parts, dim3((unsigned)((wsz + L.cout) / 16)), dim3(256), 0, st, w.blocks, wsz,
+                       (const float*)n->wpart, L.gw, L.cout, (const float*)n->bpart, L.gb);
     if (gX) return launch_conv(st, d, n->dpre, L.cout, L.cin, L.wpt, nullptr, 0, nullptr, gX);
     return hipGetLastError();
 }
@@ -723,8 +872,11 @@ hipError_t net_ensure(fe_net* n, const int nn[3]) {
     }
     const int64_t V0 = n->lv[0].V, V1 = n->lv[1].V, V2 = n->lv[2].V, V3 = n->lv[3].V;
     hipError_t e;
-#define NA(p, cnt) \
-    if ((e = alloc(&n->p, (cnt))) != hipSuccess) return e
+#define NA(p, cnt)                                     \
+    if ((e = alloc(&n->p, (cnt))) != hipSuccess) {     \
+        free_buffers(n); /* the next call starts over */ \
+        return e;                                      \
+    }
     NA(X0, V0 * 16); NA(E0, V0 * 16); NA(P1, V1 * 16); NA(E1, V1 * 32); NA(P2, V2 * 32); NA(E2, V2 * 48);
     NA(P3, V3 * 48); NA(E3, V3 * 64); NA(C2, V2 * 112); NA(D2, V2 * 48); NA(C1, V1 * 80); NA(D1, V1 * 32);
     NA(C0, V0 * 48); NA(D0, V0 * 16);
@@ -733,12 +885,29 @@ hipError_t net_ensure(fe_net* n, const int nn[3]) {
     NA(gD0, V0 * 16); NA(gC0, V0 * 48); NA(gE0, V0 * 16); NA(gD1, V1 * 32); NA(gC1, V1 * 80); NA(gE1, V1 * 32);
     NA(gP1, V1 * 16); NA(gD2, V2 * 48); NA(gC2, V2 * 112); NA(gE2, V2 * 48); NA(gP2, V2 * 32); NA(gE3, V3 * 64);
     NA(gP3, V3 * 48);
-    const int level_of[kNetLayers] = {0, 1, 2, 3, 2, 1, 0};
-    int64_t wp = 256LL * 64;  // column-sum partials
-    for (int i = 0; i < kNetLayers; ++i)
-        wp = std::max<int64_t>(wp, wgrad_parts(n->lv[level_of[i]].V) * 27LL * kNetLayerIn[i] * kNetLayerOut[i]);
+    int64_t wp = 0, bp = 0;
+    for (int i = 0; i < kNetLayers; ++i) {
+        const int64_t blocks = wgrad_shape(lv_of(n->lv[kNetLayerLevel[i]]), kNetLayerIn[i]).blocks;
+        wp = std::max<int64_t>(wp, blocks * 27LL * kNetLayerIn[i] * kNetLayerOut[i]);
+        bp = std::max<int64_t>(bp, blocks * kNetLayerOut[i]);
+    }
     NA(wpart, wp);
-    n->wpart_cap = wp;
+    NA(bpart, bp);
+    // the layers of a level share its planes, whose fill and border stay zero
+    for (int l = 0; l < 4; ++l) {
+        int ci = 0, co = 0;
+        for (int i = 0; i < kNetLayers; ++i)
+            if (kNetLayerLevel[i] == l) {
+                ci = std::max(ci, kNetLayerIn[i]);
+                co = std::max(co, kNetLayerOut[i]);
+            }
+        const Planes P = planes_of(lv_of(n->lv[l]));
+        const int64_t xw = ci * P.xn / 2, gw = co * P.gn / 2;  // in 32-bit words
+        NA(Xt[l], 2 * xw);
+        NA(Gt[l], 2 * gw);
+        hipLaunchKernelGGL(k_zero_f, g1(xw), dim3(256), 0, n->stream, xw, reinterpret_cast<float*>(n->Xt[l]));
+        hipLaunchKernelGGL(k_zero_f, g1(gw), dim3(256), 0, n->stream, gw, reinterpret_cast<float*>(n->Gt[l]));
+    }
     NA(red, (int64_t)red_blocks(V0) * 17);  // at most 17 sums per block
     n->red_cap = (int64_t)red_blocks(V0) * 17;
 #undef NA

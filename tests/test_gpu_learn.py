@@ -69,6 +69,14 @@ def test_forward_backward_matches_restatement(ctx, shape, loss_kind):
     net.close()
 
 
+@pytest.mark.parametrize("shape", [(8, 8, 8), (8, 40, 24), (16, 24, 104)])
+def test_gradients_on_ragged_levels(ctx, shape):
+    """Coarse levels whose rows are no multiple of the weight gradient's 8-voxel
+    segments (12, 6, 3 and 52, 26, 13 voxels), down to a level of one voxel;
+    bounds as above."""
+    test_forward_backward_matches_restatement(ctx, shape, "mse")
+
+
 def _dam_scene(ctx, n, box_hi, seed=0):
     desc = capi.scene_desc((n, n, n), method=capi.FLIP, blend=0.03, max_particles=8 * n ** 3)
     x = capi.seed_particles(desc, [capi.box((-1, -1, -1), box_hi)], seed=seed)
