@@ -1,14 +1,11 @@
 // k_learn.hip -- the pressure warm-start network on the device: forward,
-// backward and Adam, BF16 operands on MFMA (v_mfma_f32_16x16x16_bf16) with
+// backward and Adam, BF16 operands on MFMA with
 // FP32 accumulation.  No counterpart in the reference.
 //
-// Convolutions are implicit GEMMs over channel-last BF16 activations.  One
-// wavefront computes 16 consecutive voxels x all output channels: for each of
-// the 27 taps and each 16-channel chunk of the input it loads its A fragment
-// (4 BF16 of one voxel, 8 bytes per lane) and issues one MFMA per 16 output
-// channels against the packed weights (8 bytes per lane, contiguous).  The
-// MFMA's lane layout (checked on the device): lane l holds A[l % 16][4 (l / 16)
-// + j], B[4 (l / 16) + j][l % 16] and returns C[4 (l / 16) + i][l % 16].
+// Convolutions are implicit GEMMs over channel-last BF16 activations, K = 27
+// taps x input channels, 32 at a time (v_mfma_f32_16x16x32_bf16; a lane holds
+// A[l % 16][8 (l / 16) + j], B[8 (l / 16) + j][l % 16] and returns
+// C[4 (l / 16) + i][l % 16], checked on the device).
 // The backward data pass is the same kernel on the flipped, transposed weights;
 // the weight gradient is a GEMM over voxels (M = input channel, N = output
 // channel, K = voxel) on channel planes, one partial per workgroup summed in a
@@ -24,7 +21,6 @@ namespace fe {
 
 namespace {
 
-typedef short s4 __attribute__((ext_vector_type(4)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 
 struct Lv {
@@ -54,87 +50,135 @@ inline dim3 g1(int64_t n) { return dim3((unsigned)((n + 255) / 256)); }
 // ---------------------------------------------------------------------------
 // Convolution (forward, and backward data on the flipped weights)
 // ---------------------------------------------------------------------------
-template <int NT>
-__global__ __launch_bounds__(256) void k_conv(Lv d, const uint16_t* __restrict__ X, int cin,
-                                              const s4* __restrict__ Wp, const float* __restrict__ bias, int relu,
+// A wavefront computes 16 MT consecutive voxels x 16 NT output channels.  K
+// runs over (tap, channel) pairs 32 at a time; the 8 channels of a lane belong
+// to one tap, whose offset comes from a table in LDS.  A voxel outside the grid
+// reads at an offset past the buffer's end, which the load gives as zeros.
+// Bound by the first-level cache: per 32 of K it reads MT KB of activations
+// and NT KB of packed weights for MT NT matrix instructions, so a large level
+// takes MT = 4.  At 64x96x80 (us per launch, with one 16-voxel tile and 16 of
+// K per step before): 16 and 48 -> 16 channels on the finest level 100 (mean),
+// 16 -> 48 there and 32, 112 -> 48 below 73 (mean), 48 -> 112 on the third 80.
+typedef __bf16 b8 __attribute__((ext_vector_type(8)));
+typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+__device__ inline b8 as_b8(const u4& w) { return __builtin_bit_cast(b8, w); }
+
+__host__ __device__ inline int conv_chunks(int cin) { return (27 * cin + 31) / 32; }
+constexpr int kMaxCh = 112;
+constexpr int kMaxChunks = (27 * kMaxCh + 31) / 32;
+constexpr uint32_t kConvReach = 0x7FFFFFFFu;  // bytes a load may reach from its wave's base
+
+template <int MT, int NT>
+__global__ __launch_bounds__(256) void k_conv(Lv d, const uint16_t* __restrict__ X, int cin, int cout,
+                                              const u4* __restrict__ Wp, const float* __restrict__ bias, int relu,
                                               uint16_t* __restrict__ Ybf, float* __restrict__ Yf) {
-    const int wave = threadIdx.x >> 6, l = threadIdx.x & 63;
-    const int64_t tile = (int64_t)blockIdx.x * 4 + wave;
-    if (tile * 16 >= d.V) return;  // uniform per wavefront
-    const int row = l & 15, kq = l >> 4;
-    const int64_t va = tile * 16 + row;
-    const bool rowok = va < d.V;
-    int x = 0, y = 0, z = 0;
-    if (rowok) decode(d, va, x, y, z);
-    const int KC = cin >> 4;
-    f4 acc[NT];
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) acc[nt] = f4{0.f, 0.f, 0.f, 0.f};
-    for (int t = 0; t < 27; ++t) {
+    __shared__ int2 table[4 * kMaxChunks];  // per chunk and lane group: byte offset, tap (27: none)
+    const int chunks = conv_chunks(cin);
+    for (int e = threadIdx.x; e < 4 * chunks; e += 256) {
+        const int t = 8 * e / cin, ch = 8 * e - t * cin;
         const int dx = t % 3 - 1, dy = (t / 3) % 3 - 1, dz = t / 9 - 1;
-        const bool ok = rowok && (unsigned)(x + dx) < (unsigned)d.nx && (unsigned)(y + dy) < (unsigned)d.ny &&
-                        (unsigned)(z + dz) < (unsigned)d.nz;
-        const int64_t u = ok ? va + dx + (int64_t)dy * d.nx + (int64_t)dz * d.nx * d.ny : 0;
-        const s4* xa = reinterpret_cast<const s4*>(X + u * cin) + kq;
-        const s4* wb = Wp + (int64_t)t * KC * NT * 64 + l;
-        for (int kc = 0; kc < KC; ++kc) {
-            s4 a = s4{0, 0, 0, 0};
-            if (ok) a = xa[kc * 4];
+        table[e] = t < 27 ? make_int2(2 * ((dx + d.nx * (dy + d.ny * dz)) * cin + ch), t) : make_int2(0, 27);
+    }
+    __syncthreads();
+    const int wave = threadIdx.x >> 6, l = threadIdx.x & 63, row = l & 15, kq = l >> 4;
+    const int64_t v0 = ((int64_t)blockIdx.x * 4 + wave) * (16 * MT);
+    if (v0 >= d.V) return;  // uniform per wavefront
+    const int nt0 = blockIdx.y * NT, nts = cout / 16;
+    // the buffer starts a z slice and a row before the wave's first voxel
+    const int64_t reach = (int64_t)d.nx * d.ny + d.nx + 1;
+    const int64_t vb = v0 > reach ? v0 - reach : 0;
+    const int64_t bytes = (d.V - vb) * cin * 2;
+    const __amdgpu_buffer_rsrc_t buf = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint16_t*>(X + vb * cin), 0, (int)(bytes < (int64_t)kConvReach ? bytes : (int64_t)kConvReach), 0x00020000);
+    // per tile: which of the 27 taps lie inside the grid, and the voxel's offset
+    uint32_t mask[MT], at[MT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+        const int64_t v = v0 + 16 * m + row;
+        mask[m] = 0;
+        at[m] = (uint32_t)((v - vb) * cin * 2);
+        if (v < d.V) {
+            int x, y, z;
+            decode(d, v, x, y, z);
+            const uint32_t xm = (x > 0) | 2 | ((x + 1 < d.nx) << 2);
+            const bool ym[3] = {y > 0, true, y + 1 < d.ny}, zm[3] = {z > 0, true, z + 1 < d.nz};
+#pragma unroll
+            for (int q = 0; q < 9; ++q) mask[m] |= ym[q % 3] && zm[q / 3] ? xm << (3 * q) : 0u;
+        }
+    }
+    f4 acc[MT][NT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) acc[m][nt] = f4{0.f, 0.f, 0.f, 0.f};
+    const u4* wb = Wp + (int64_t)nt0 * 64 + l;
+    auto load = [&](int c, b8 (&a)[MT], b8 (&b)[NT]) {
+        const int2 e = table[4 * c + kq];
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) b[nt] = as_b8(wb[((int64_t)c * nts + nt) * 64]);
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            const uint32_t o = (mask[m] >> e.y) & 1u ? at[m] + (uint32_t)e.x : 0xFFFFFFF0u;
+            a[m] = as_b8(__builtin_bit_cast(u4, __builtin_amdgcn_raw_buffer_load_b128(buf, (int)o, 0, 0)));
+        }
+    };
+    b8 a[MT], b[NT], an[MT], bn[NT];
+    load(0, a, b);
+    for (int c = 0; c < chunks; ++c) {
+        load(min(c + 1, chunks - 1), an, bn);  // the next step's, before this one's products
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt)
-                acc[nt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, wb[(kc * NT + nt) * 64], acc[nt], 0, 0, 0);
-        }
-    }
-    const int cout = NT * 16;
+                acc[m][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[m], b[nt], acc[m][nt], 0, 0, 0);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int64_t v = tile * 16 + 4 * kq + i;
-        if (v >= d.V) continue;
+        for (int m = 0; m < MT; ++m) a[m] = an[m];
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
-            const int co = nt * 16 + row;
-            float val = acc[nt][i] + (bias ? bias[co] : 0.0f);
-            if (relu) val = fmaxf(val, 0.0f);
-            if (Ybf) Ybf[v * cout + co] = to_bf16(val);
-            if (Yf) Yf[v * cout + co] = val;
-        }
+        for (int nt = 0; nt < NT; ++nt) b[nt] = bn[nt];
     }
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int64_t v = v0 + 16 * m + 4 * kq + i;
+            if (v >= d.V) continue;
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) {
+                const int co = (nt0 + nt) * 16 + row;
+                float val = acc[m][nt][i] + (bias ? bias[co] : 0.0f);
+                if (relu) val = fmaxf(val, 0.0f);
+                if (Ybf) Ybf[v * cout + co] = to_bf16(val);
+                if (Yf) Yf[v * cout + co] = val;
+            }
+        }
 }
 
-// Packed BF16 weights: forward [t][kc][nt][lane][j] = W[t][16 kc + 4 (lane / 16) + j][16 nt + lane % 16];
+// Packed BF16 weights: forward [chunk][nt][lane][j] = W[t][ci][16 nt + lane % 16],
+// (t, ci) = pair 32 chunk + 8 (lane / 16) + j of the 27 cin, zero past the end;
 // backward data (cin' = cout, cout' = cin): W'[t][a][b] = W[26 - t][b][a], packed the same way.
+__device__ inline void packed_place(int64_t i, int cin, int cout, int& t, int& ci, int& co) {
+    const int j = (int)(i & 7), l = (int)(i >> 3) & 63, NT = cout / 16;
+    const int64_t r = i >> 9;
+    const int c = (int)(r / NT), nt = (int)(r - (int64_t)c * NT);
+    const int k = 32 * c + 8 * (l >> 4) + j;
+    t = k / cin;
+    ci = k - t * cin;
+    co = 16 * nt + (l & 15);
+}
+
+__host__ __device__ inline int64_t packed_size(int cin, int cout) { return 32LL * conv_chunks(cin) * cout; }
+
 __global__ __launch_bounds__(256) void k_pack(int cin, int cout, const float* __restrict__ w,
                                               uint16_t* __restrict__ wp, uint16_t* __restrict__ wpt) {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= 27LL * cin * cout) return;
-    {
-        const int KC = cin / 16, NT = cout / 16;
-        int64_t r = i;
-        const int j = (int)(r % 4);
-        r /= 4;
-        const int l = (int)(r % 64);
-        r /= 64;
-        const int nt = (int)(r % NT);
-        r /= NT;
-        const int kc = (int)(r % KC);
-        const int t = (int)(r / KC);
-        const int ci = kc * 16 + 4 * (l / 16) + j, co = nt * 16 + (l % 16);
-        wp[i] = to_bf16(w[((int64_t)t * cin + ci) * cout + co]);
+    int t, a, b;
+    if (i < packed_size(cin, cout)) {
+        packed_place(i, cin, cout, t, a, b);
+        wp[i] = t < 27 ? to_bf16(w[((int64_t)t * cin + a) * cout + b]) : (uint16_t)0;
     }
-    {
-        const int KC = cout / 16, NT = cin / 16;
-        int64_t r = i;
-        const int j = (int)(r % 4);
-        r /= 4;
-        const int l = (int)(r % 64);
-        r /= 64;
-        const int nt = (int)(r % NT);
-        r /= NT;
-        const int kc = (int)(r % KC);
-        const int t = (int)(r / KC);
-        const int a = kc * 16 + 4 * (l / 16) + j;  // an output channel of W
-        const int b = nt * 16 + (l % 16);          // an input channel of W
-        wpt[i] = to_bf16(w[((int64_t)(26 - t) * cin + b) * cout + a]);
+    if (i < packed_size(cout, cin)) {
+        packed_place(i, cout, cin, t, a, b);  // a: an output channel of W, b: an input channel
+        wpt[i] = t < 27 ? to_bf16(w[((int64_t)(26 - t) * cin + b) * cout + a]) : (uint16_t)0;
     }
 }
 
@@ -154,9 +198,6 @@ __global__ __launch_bounds__(256) void k_pack(int cin, int cout, const float* __
 // At 64x96x80, the layers of the finest level (48 -> 16 and 16 -> 16
 // channels): 450 and 417 us with one tap per wavefront and 2-byte loads.
 // ---------------------------------------------------------------------------
-typedef __bf16 b8 __attribute__((ext_vector_type(8)));
-typedef uint32_t u4 __attribute__((ext_vector_type(4)));
-
 constexpr int kEdge = 8;  // the zero border of X's rows
 
 struct Planes {
@@ -175,8 +216,6 @@ __host__ __device__ inline Planes planes_of(const Lv& d) {
     P.gn = 32 * P.steps;
     return P;
 }
-
-constexpr int kMaxCh = 112;
 
 // A workgroup's 8 segments of a channel-last array, as pairs of channels:
 // f(voxel, channel pair) gives a pair's bits; they go to channel planes (X's
@@ -242,8 +281,6 @@ __global__ __launch_bounds__(256) void k_mask(Lv d, int C, const float* __restri
         return w;
     });
 }
-
-__device__ inline b8 as_b8(const u4& w) { return __builtin_bit_cast(b8, w); }
 
 // blockIdx.y = 3 kc + dz (16 input channels, z offset dz - 1).  Wave w of block
 // b takes the 32-voxel steps [ (4 b + w) spw, ... + spw ).
@@ -662,21 +699,36 @@ __global__ __launch_bounds__(256) void k_zero_f(int64_t n, float* __restrict__ a
 // ---------------------------------------------------------------------------
 // Host drivers
 // ---------------------------------------------------------------------------
+template <int MT, int NT>
+hipError_t launch_conv_tile(hipStream_t st, const Lv& d, const uint16_t* X, int cin, int cout, const uint16_t* wp,
+                            const float* bias, int relu, uint16_t* ybf, float* yf) {
+    const dim3 grid((unsigned)((d.V + 64 * MT - 1) / (64 * MT)), (unsigned)(cout / 16 / NT));
+    hipLaunchKernelGGL((k_conv<MT, NT>), grid, dim3(256), 0, st, d, X, cin, cout, reinterpret_cast<const u4*>(wp),
+                       bias, relu, ybf, yf);
+    return hipGetLastError();
+}
+
+// Large tiles as long as they leave every SIMD a wave or two (1024 SIMDs); a
+// small level's launch is one wave's chain of loads, so it takes the most
+// waves: single tiles, an output group each.
 hipError_t launch_conv(hipStream_t st, const Lv& d, const uint16_t* X, int cin, int cout, const uint16_t* wp,
                        const float* bias, int relu, uint16_t* ybf, float* yf) {
-    const int64_t tiles = (d.V + 15) / 16;
-    const dim3 grid((unsigned)((tiles + 3) / 4));
-    const s4* W = reinterpret_cast<const s4*>(wp);
+    const int mt = d.V >= 64 * 2048 ? 4 : (d.V >= 32 * 1024 ? 2 : 1);
+    if (mt == 1) return launch_conv_tile<1, 1>(st, d, X, cin, cout, wp, bias, relu, ybf, yf);
+#define FE_CONV(NT)                                                                                        \
+    case NT:                                                                                               \
+        return mt == 4 ? launch_conv_tile<4, NT>(st, d, X, cin, cout, wp, bias, relu, ybf, yf)             \
+                       : launch_conv_tile<2, NT>(st, d, X, cin, cout, wp, bias, relu, ybf, yf)
     switch (cout / 16) {
-        case 1: hipLaunchKernelGGL(k_conv<1>, grid, dim3(256), 0, st, d, X, cin, W, bias, relu, ybf, yf); break;
-        case 2: hipLaunchKernelGGL(k_conv<2>, grid, dim3(256), 0, st, d, X, cin, W, bias, relu, ybf, yf); break;
-        case 3: hipLaunchKernelGGL(k_conv<3>, grid, dim3(256), 0, st, d, X, cin, W, bias, relu, ybf, yf); break;
-        case 4: hipLaunchKernelGGL(k_conv<4>, grid, dim3(256), 0, st, d, X, cin, W, bias, relu, ybf, yf); break;
-        case 5: hipLaunchKernelGGL(k_conv<5>, grid, dim3(256), 0, st, d, X, cin, W, bias, relu, ybf, yf); break;
-        case 7: hipLaunchKernelGGL(k_conv<7>, grid, dim3(256), 0, st, d, X, cin, W, bias, relu, ybf, yf); break;
+        FE_CONV(1);
+        FE_CONV(2);
+        FE_CONV(3);
+        FE_CONV(4);
+        FE_CONV(5);
+        FE_CONV(7);
         default: return hipErrorInvalidValue;
     }
-    return hipGetLastError();
+#undef FE_CONV
 }
 
 // Workgroups along the voxels: about 16 waves per CU in all, and a few steps
@@ -759,7 +811,7 @@ hipError_t layer_back(fe_net* n, int li, const Lv& d, const uint16_t* X, const u
 
 hipError_t pack_all(fe_net* n) {
     for (auto& L : n->L) {
-        const int64_t sz = 27LL * L.cin * L.cout;
+        const int64_t sz = std::max(packed_size(L.cin, L.cout), packed_size(L.cout, L.cin));
         hipLaunchKernelGGL(k_pack, g1(sz), dim3(256), 0, n->stream, L.cin, L.cout, (const float*)L.w, L.wp, L.wpt);
     }
     return hipGetLastError();
@@ -797,7 +849,9 @@ hipError_t net_alloc(fe_net* n, uint64_t seed) {
             if ((e = alloc(p, wsz)) != hipSuccess) return e;
         for (float** p : {&L.b, &L.gb, &L.mb, &L.vb})
             if ((e = alloc(p, L.cout)) != hipSuccess) return e;
-        if ((e = alloc(&L.wp, wsz)) != hipSuccess || (e = alloc(&L.wpt, wsz)) != hipSuccess) return e;
+        if ((e = alloc(&L.wp, packed_size(L.cin, L.cout))) != hipSuccess ||
+            (e = alloc(&L.wpt, packed_size(L.cout, L.cin))) != hipSuccess)
+            return e;
         std::vector<float> w((size_t)wsz), z((size_t)wsz, 0.0f), zb((size_t)L.cout, 0.0f);
         const double sd = std::sqrt(2.0 / (27.0 * L.cin));  // He initialisation
         for (auto& x : w) x = (float)(normal() * sd);
