@@ -387,6 +387,9 @@ struct SolverScalars {
     int32_t replace;   // the next (or last) update recomputes r = b - A x
     int32_t converged; // the stopping rule (not the iteration cap) ended the solve
     int32_t confirm;   // a relative stop met on the recurrence awaits the recomputed residual
+    int32_t phase;     // CG without multigrid: what the last launch left (CGPhase)
+    int32_t launches;  // and the launches up to the stop
+    int32_t xbuf;      // and the solution buffer it stopped on
 };
 
 // One component's Jacobi solve of the viscosity step.
@@ -408,7 +411,7 @@ struct DiffState {
 // The state of a conjugate-gradient solve between its launches (the
 // iterations' buffers rotate with the iteration count).
 struct CGRun {
-    int k = 0;        // spmv / update pairs launched
+    int k = 0;        // spmv / update pairs launched (without multigrid: steps launched)
     int dcur = 0;     // d[dcur] holds the current search direction
     double* xa = nullptr;  // current solution
     double* xb = nullptr;  // its ping-pong partner
@@ -530,6 +533,7 @@ struct fe_scene {
     float* z = nullptr;           // preconditioned residual
     float* d[2] = {nullptr, nullptr};
     float* q = nullptr;
+    float* q2 = nullptr;          // q's ping-pong partner (CG without multigrid)
     double* partials = nullptr;   // per-block FP64 partial sums (2 per block)
     uint8_t* chunk_fluid = nullptr;  // per solver block: its cells include a FLUID cell (from BuildSystem)
     int64_t npartials = 0;
@@ -558,6 +562,7 @@ struct fe_scene {
     hipEvent_t ev[fe::kMaxStages + 1] = {};
     double stage_ms[fe::kMaxStages] = {};
     fe_solve_stats last_stats{};
+    int last_cg_launches[2] = {0, 0};  // launches of the last CG solve without and with the diagonal preconditioner
     int last_cg_iters[3] = {0, 0, 0};  // iterations of the last CG solve per preconditioner (none, diagonal, multigrid)
     std::vector<fe::MGLevel> mg;  // multigrid hierarchy, built on first use
     int mg_tail = 0;              // first level handled by the one-workgroup tail kernel

@@ -218,16 +218,16 @@ __device__ inline Stencil64In stencil64_in(int64_t c, const uint16_t* __restrict
 }
 
 // ---------------------------------------------------------------------------
-// Conjugate gradient (ConjugateGradientSolver::Solve, src/linear_system/conjugate_gradient_solver.cpp:14-55),
-// two kernels per iteration:
+// Conjugate gradient (ConjugateGradientSolver::Solve, src/linear_system/conjugate_gradient_solver.cpp:14-55).
+// With the multigrid preconditioner, two kernels and a V-cycle per iteration:
 //   spmv:   [prologue: sigma' = r.z, r.r of the last update -> beta, trigger,
 //           stopping rule, next replacement flag]  d = z + beta*d_old (also at
 //           the 6 neighbours, on the fly), q = A d, partials of d.q
 //   update: [prologue: alpha = sigma / d.q]  x' = alpha*d + x (FP64);
 //           r = -alpha*q + r, or r = b - A x' in FP64 on residual replacement
 //           (every 50 iterations or after sigma grew, :32-49; x' at the
-//           neighbours is formed on the fly from x and d); z = M^-1 r;
-//           partials of r.z and r.r
+//           neighbours is formed on the fly from x and d); partials of r.r
+// Without it one kernel per iteration, k_cg_step below.
 // With the relative rule a stop is only accepted on a freshly replaced
 // residual, so the decision is taken on b - A x, not on the recurrence (with
 // the multigrid preconditioner the next V-cycle's first kernel tests the
@@ -241,11 +241,10 @@ __device__ inline Stencil64In stencil64_in(int64_t c, const uint16_t* __restrict
 constexpr double kReliableDrop2 = 1e-4;  // (100x in ||r||)^2
 __global__ __launch_bounds__(kBlock) void k_cg_init(Geom g, const uint16_t* __restrict__ code,
                                                     const float* __restrict__ b, double* __restrict__ x,
-                                                    float* __restrict__ r, float* __restrict__ z,
-                                                    float* __restrict__ d0, float* __restrict__ mgx, SolverScalars* sc,
+                                                    float* __restrict__ r, float* __restrict__ d0, float* __restrict__ mgx, SolverScalars* sc,
                                                     const double* __restrict__ pbb, double* __restrict__ pout,
-                                                    int nparts, float ihx2, float ihy2, float ihz2, int64_t chunk,
-                                                    int64_t padded) {
+                                                    int stride, int nparts, float ihx2, float ihy2, float ihz2,
+                                                    int64_t chunk, int64_t padded) {
     const int64_t nc = cell_count(g);
     const Span sp = block_span(nc, chunk, padded);
     const Stride st = stride_of(g.n[0], g.n[1], g.n[2]);
@@ -274,11 +273,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_init(Geom g, const uint16_t* __re
         if (!fl && t.xc != 0.0) x[c] = 0.0;  // written only where it is not 0 already
         const float rc = fl ? (float)((double)t.bc - code_apply64_nb(t.cd, ih2d, t.xc, t.nb)) : 0.0f;
         r[c] = rc;
-        float zc = rc;
-        if (pre == 1) {
-            zc = rc / code_center(t.cd, ih2);
-            z[c] = zc;
-        }
+        const float zc = pre == 1 ? rc / code_center(t.cd, ih2) : rc;
         if (mgx) mgx[c] = mg_weight(t.cd, ih2) * rc;  // the V-cycle's first sweep from zero
         d0[c] = 0.0f;
         if (pre != 2) v[0] += (double)rc * (double)zc;
@@ -291,7 +286,9 @@ __global__ __launch_bounds__(kBlock) void k_cg_init(Geom g, const uint16_t* __re
     span_groups_from<G, Stencil64In>(
         early ? g0 + (int64_t)G * kBlock : g0, sp.c1, [&](int64_t c) { return stencil64_in(c, code, x, b, st); },
         use);
-    write_partials<2>(v, pout);
+    __shared__ double sm[2][kBlock / 64];
+    block_reduce<2>(v, sm);
+    if (threadIdx.x < stride) pout[(int64_t)blockIdx.x * stride + threadIdx.x] = threadIdx.x < 2 ? v[threadIdx.x] : 0.0;
 }
 
 // State slots alternate with the iteration (spmv k reads slot k&1 and writes
@@ -330,17 +327,10 @@ __global__ __launch_bounds__(kBlock) void k_cg_spmv(Geom g, const uint16_t* __re
             code_neighbours(c, st, [&](int64_t n) { return dold[n]; }, raw[u].dn);
         }
     }
-    // ---- state update from the last update's r.z and r.r (every block alike);
-    // with the multigrid preconditioner r.z comes from the V-cycle's last sweep
+    // ---- state update (every block alike) from r.z of the V-cycle's last sweep
+    // and r.r of the last update
     double t[2];
-    if (pz) {  // r.z from the V-cycle's last sweep, r.r from the update: one pass
-        double u[2];
-        sum_partials_two(pz, 1, 0, nz, pin, 2, 1, nparts, u);
-        t[0] = u[0];
-        t[1] = u[1];
-    } else {
-        sum_partials<2>(pin, nparts, t);
-    }
+    sum_partials_two(pz, 1, 0, nz, pin, 2, 1, nparts, t);
     if (in->done) {  // uniform: an earlier spmv stopped the solve
         if (blockIdx.x == 0 && threadIdx.x == 0) *out = *in;
         return;
@@ -434,7 +424,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_update(Geom g, const uint16_t* __
                                                       const float* __restrict__ b, const double* __restrict__ xo,
                                                       double* __restrict__ xn, const float* __restrict__ d,
                                                       const float* __restrict__ q, float* __restrict__ r,
-                                                      float* __restrict__ z, float* __restrict__ mgx, SolverScalars* sc,
+                                                      float* __restrict__ mgx, SolverScalars* sc,
                                                       const double* __restrict__ pin, double* __restrict__ pout,
                                                       int nparts, float ihx2, float ihy2, float ihz2,
                                                       const uint8_t* __restrict__ cfl, int64_t chunk, int64_t padded) {
@@ -476,27 +466,20 @@ __global__ __launch_bounds__(kBlock) void k_cg_update(Geom g, const uint16_t* __
         sc->dq = t[0];
         sc->alpha = alpha;
     }
-    if (!body) {  // no FLUID cell: x, r, z and the first sweep stay 0
+    if (!body) {  // no FLUID cell: x, r and the first sweep stay 0
         if (threadIdx.x == 0) pout[2 * blockIdx.x] = pout[2 * blockIdx.x + 1] = 0.0;
         return;
     }
     const bool replace = sc->replace != 0;
-    const int pre_kind = sc->precond;
     const float ih2[3] = {ihx2, ihy2, ihz2};
     const double ih2d[3] = {ihx2, ihy2, ihz2};
     const Stride st = stride_of(g.n[0], g.n[1], g.n[2]);
     const float fa = (float)alpha;
     auto X = [&](int64_t n) { return alpha * (double)d[n] + xo[n]; };
-    double v[2] = {0.0, 0.0};
+    double v[2] = {0.0, 0.0};  // r.z comes from the V-cycle
     auto finish = [&](int64_t c, uint16_t cd, float rc) {
         r[c] = rc;
-        float zc = rc;
-        if (pre_kind == 1) {
-            zc = rc / code_center(cd, ih2);
-            z[c] = zc;
-        }
         if (mgx) mgx[c] = mg_weight(cd, ih2) * rc;  // the V-cycle's first sweep from zero
-        if (pre_kind != 2) v[0] += (double)rc * (double)zc;
         v[1] += (double)rc * (double)rc;
     };
     if (replace) {  // r = b - A x recomputed in FP64
@@ -523,12 +506,203 @@ __global__ __launch_bounds__(kBlock) void k_cg_update(Geom g, const uint16_t* __
                 t.d = d[c];
                 t.q = q[c];
                 t.r = r[c];
-                t.cd = (pre_kind == 1 || mgx) ? code[c] : (uint16_t)0;  // for z or the first sweep
+                t.cd = mgx ? code[c] : (uint16_t)0;  // for the first sweep
                 return t;
             },
             use);
     }
     write_partials<2>(v, pout);
+}
+
+// ---------------------------------------------------------------------------
+// One CG iteration without multigrid in one launch: (r, d, q = A d, x) of the
+// read buffers to those of the written ones,
+//   alpha = sigma / d.q,  r' = r - alpha q,  x' = x + alpha d (FP64),
+//   d' = z' + beta d,  q' = A d',
+// with r', z' and d' formed at the six neighbours too.  beta = sigma' / sigma
+// would need r'.z' before d' exists; by conjugacy (q.z = q.d) it is
+// alpha^2 q.M^-1 q - sigma, which the launch before has summed.  Only beta
+// takes that value: alpha and every test use the r.z and r.r summed from r
+// itself.  Where it is not positive (all rounding), and where the residual is
+// recomputed, the iteration takes two launches: r' = b - A x' with x', then
+// d' and q' with the sums of that r'.
+//
+// Bound by latency on all but large grids: the launch, the partial sums, the
+// state, one round of loads (issued before any of these is waited for), the
+// block's sums.  An iteration of 190 k cells in two launches took 12.7 us.
+// After a stop at x of buffer xbuf every launch returns.
+// ---------------------------------------------------------------------------
+enum CGPhase { kHaveR = 0, kHaveAll = 1, kHaveAllSummed = 2 };  // r; r, d, q; the same with sigma and r.r in the state
+
+struct CGBuffers {
+    const float *r, *d, *q;
+    const double* x;
+    float *ro, *dn, *qo;
+    double* xo;
+};
+
+// G: cells per thread of a group, kBlock apart.
+template <int G, bool DIAG>
+__global__ __launch_bounds__(kBlock) void k_cg_step(Geom g, const uint16_t* __restrict__ code,
+                                                    const float* __restrict__ b, CGBuffers B, int parity,
+                                                    const SolverScalars* __restrict__ in,
+                                                    SolverScalars* __restrict__ out, const double* __restrict__ pin,
+                                                    double* __restrict__ pout, int nparts, float ihx2, float ihy2,
+                                                    float ihz2, const uint8_t* __restrict__ cfl, int64_t chunk,
+                                                    int64_t padded) {
+    const int64_t nc = cell_count(g);
+    const Span sp = block_span(nc, chunk, padded);
+    const Stride st = stride_of(g.n[0], g.n[1], g.n[2]);
+    const bool body = sp.c0 < sp.c1 && cfl[sp.lb] != 0;
+    struct Raw {
+        uint16_t cd, cn[DIAG ? 6 : 1];
+        float r, d, q, rn[6], dn[6], qn[6];
+        double x;
+    };
+    auto fetch = [&](int64_t c) {
+        Raw w;
+        w.cd = code[c];
+        w.r = B.r[c];
+        w.d = B.d[c];
+        w.q = B.q[c];
+        w.x = B.x[c];
+        code_neighbours(c, st, [&](int64_t n) { return B.r[n]; }, w.rn);
+        code_neighbours(c, st, [&](int64_t n) { return B.d[n]; }, w.dn);
+        code_neighbours(c, st, [&](int64_t n) { return B.q[n]; }, w.qn);
+        if constexpr (DIAG) code_neighbours(c, st, [&](int64_t n) { return code[n]; }, w.cn);
+        return w;
+    };
+    // the thread's first group, at its last cell where it has fewer
+    Raw raw[G];
+    const int64_t g0 = sp.c0 + threadIdx.x;
+    if (body) {
+#pragma unroll
+        for (int u = 0; u < G; ++u) raw[u] = fetch(min(g0 + (int64_t)u * kBlock, sp.c1 - 1));
+    }
+    if (in->done) {  // uniform
+        if (blockIdx.x == 0 && threadIdx.x == 0) *out = *in;
+        return;
+    }
+    double t[4];  // r.z, r.r, d.q, q.M^-1 q of the read buffers
+    sum_partials<4>(pin, nparts, t);
+    const int phase = in->phase;
+    double sigma, rr, rr_ref;
+    int it, trig, repl, confirm, conv = 0, done = 0;
+    if (phase == kHaveAllSummed) {
+        sigma = in->sigma;
+        rr = in->rr;
+        rr_ref = in->rr_ref;
+        it = in->it;
+        trig = in->trigger;
+        repl = in->replace;
+        confirm = in->confirm;
+    } else {
+        sigma = t[0];
+        rr = t[1];
+        confirm = 0;
+        if (in->it < 0) {  // the sums are k_cg_init's
+            it = 0;
+            trig = 0;
+            rr_ref = rr;
+            conv = stop_rule(in, in->bnorm2, sigma, rr) ? 1 : 0;
+            done = (conv || in->max_it <= 0) ? 1 : 0;
+        } else {
+            const bool replaced = phase == kHaveR;
+            rr_ref = replaced ? rr : in->rr_ref;
+            it = in->it + 1;
+            trig = sigma > in->sigma ? 1 : 0;
+            bool stop = stop_rule(in, in->bnorm2, sigma, rr);
+            if (stop && in->relative && !replaced) {  // confirm on the true residual
+                stop = false;
+                trig = 1;
+                confirm = 1;
+            }
+            conv = stop ? 1 : 0;
+            done = (stop || it >= in->max_it) ? 1 : 0;
+        }
+        repl = (trig || (it % 50 == 0 && it > 0) || rr < kReliableDrop2 * rr_ref) ? 1 : 0;
+    }
+    double alpha = 0.0, beta = 0.0;
+    if (phase == kHaveR) {
+        beta = in->it < 0 ? 0.0 : sigma / in->sigma;
+    } else {
+        alpha = sigma / t[2];
+        beta = (alpha * alpha * t[3] - sigma) / sigma;
+        if (!(beta > 0.0)) repl = 1;
+    }
+    const bool only_d = phase == kHaveR, only_r = !only_d && repl;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        SolverScalars o = *in;
+        o.sigma_old = in->sigma;
+        o.sigma = sigma;
+        o.rr = rr;
+        o.dq = t[2];
+        o.alpha = alpha;
+        o.beta = beta;
+        o.it = it;
+        o.trigger = trig;
+        o.converged = conv;
+        o.done = done;
+        o.replace = repl;
+        o.rr_ref = rr_ref;
+        o.confirm = confirm;
+        o.phase = only_d ? kHaveAllSummed : (only_r ? kHaveR : kHaveAll);
+        o.launches = in->launches + 1;
+        o.xbuf = parity;
+        *out = o;
+    }
+    if (done) return;
+    if (!body) {  // no FLUID cell: every vector stays 0
+        if (threadIdx.x < 4) pout[4 * (int64_t)blockIdx.x + threadIdx.x] = 0.0;
+        return;
+    }
+    const float ih2[3] = {ihx2, ihy2, ihz2};
+    const double ih2d[3] = {ihx2, ihy2, ihz2};
+    const float fa = (float)alpha, fb = (float)beta;
+    double v[4] = {0.0, 0.0, 0.0, 0.0};
+    auto precond = [&](float r, uint16_t cd) { return DIAG ? r / code_center(cd, ih2) : r; };
+    auto direction = [&](int64_t c, uint16_t cd, float dc, const float (&nb)[6]) {
+        const float center = code_center(cd, ih2);
+        const float qc = code_apply_nb(cd, center, ih2, dc, nb);
+        B.dn[c] = dc;
+        B.qo[c] = qc;
+        v[2] += (double)dc * (double)qc;
+        v[3] += (double)qc * (double)(DIAG ? qc / center : qc);
+    };
+    auto residual = [&](int64_t c, uint16_t cd, float rc) {
+        B.ro[c] = rc;
+        v[0] += (double)rc * (double)precond(rc, cd);
+        v[1] += (double)rc * (double)rc;
+    };
+    auto use = [&](int64_t c, const Raw& w) {
+        float nb[6];
+        if (only_r) {
+            auto X = [&](int64_t n) { return alpha * (double)B.d[n] + B.x[n]; };
+            const double xc = alpha * (double)w.d + w.x;
+            B.xo[c] = xc;
+            B.dn[c] = w.d;
+            residual(c, w.cd, (float)((double)b[c] - code_apply64(w.cd, c, st, ih2d, xc, X)));
+        } else if (only_d) {
+            B.xo[c] = w.x;
+            B.ro[c] = w.r;
+#pragma unroll
+            for (int k = 0; k < 6; ++k) nb[k] = fmaf(fb, w.dn[k], precond(w.rn[k], w.cn[DIAG ? k : 0]));
+            direction(c, w.cd, fmaf(fb, w.d, precond(w.r, w.cd)), nb);
+        } else {
+            B.xo[c] = alpha * (double)w.d + w.x;
+            const float rc = fmaf(-fa, w.q, w.r);
+            residual(c, w.cd, rc);
+#pragma unroll
+            for (int k = 0; k < 6; ++k)
+                nb[k] = fmaf(fb, w.dn[k], precond(fmaf(-fa, w.qn[k], w.rn[k]), w.cn[DIAG ? k : 0]));
+            direction(c, w.cd, fmaf(fb, w.d, precond(rc, w.cd)), nb);
+        }
+    };
+#pragma unroll
+    for (int u = 0; u < G; ++u)
+        if (g0 + (int64_t)u * kBlock < sp.c1) use(g0 + (int64_t)u * kBlock, raw[u]);
+    for (int64_t c = g0 + (int64_t)G * kBlock; c < sp.c1; c += kBlock) use(c, fetch(c));
+    write_partials<4>(v, pout);
 }
 
 // Final ||b - A p||^2 and ||b||^2 in FP64 on the FP64 solution, with FP64
@@ -717,8 +891,6 @@ struct CGSetup {
     int precond = 0;
     bool mg = false, fused = false;
     float* mgx = nullptr;
-    const float* zr = nullptr;
-    const double* pz = nullptr;
     int nz = 0;
 };
 
@@ -730,7 +902,7 @@ static CGSetup cg_setup(fe_scene* s, int precond) {
     c.sh = solver_shape(s->g);
     c.nparts = (int)c.sh.blocks;
     c.PA = s->partials;                  // 2 per block
-    c.PB = s->partials + 2 * c.sh.blocks;  // 2 per block
+    c.PB = s->partials + (precond == 2 ? 2 : 4) * c.sh.blocks;  // 2 per block (without multigrid 4)
     c.PZ = s->partials + 4 * c.sh.blocks;  // r.z of the V-cycle, 1 per block
     // BuildSystem's invH * invH (single_phase_pressure_solver.cpp:102-103); exact
     // in FP32 for power-of-two spacings
@@ -740,8 +912,6 @@ static CGSetup cg_setup(fe_scene* s, int precond) {
     c.fused = c.mg && s->tune.mg == FE_MG_FUSED;
     if (c.fused) c.PZ = s->mg_pz;  // one r.z partial per workgroup of the level-0 ascent
     c.mgx = c.mg && !c.fused ? mg_first_sweep_target(s) : nullptr;  // the fused descent sweeps from b itself
-    c.zr = precond ? s->z : s->r;
-    c.pz = c.mg ? c.PZ : nullptr;
     c.nz = c.fused ? (int)s->mg_npz : c.nparts;
     return c;
 }
@@ -750,10 +920,10 @@ static void cg_update(fe_scene* s, const CGSetup& c, CGRun& R, int kk) {
     R.dcur = 1 - R.dcur;
     launch_timed(s, FE_KERNEL_CG_UPDATE, kk, k_cg_update, dim3((unsigned)c.sh.blocks), dim3(kBlock), c.g,
                  (const uint16_t*)s->code, (const float*)s->b, (const double*)R.xa, R.xb, (const float*)s->d[R.dcur],
-                 (const float*)s->q, s->r, s->z, c.mgx, s->sc + ((kk + 1) & 1), (const double*)c.PA, c.PB, c.nparts,
+                 (const float*)s->q, s->r, c.mgx, s->sc + ((kk + 1) & 1), (const double*)c.PA, c.PB, c.nparts,
                  c.ih2[0], c.ih2[1], c.ih2[2], (const uint8_t*)s->chunk_fluid, c.sh.chunk, c.sh.blocks);
     std::swap(R.xa, R.xb);
-    if (c.mg) (void)mg_apply(s, s->r, s->z, s->sc + ((kk + 1) & 1), c.PZ, kk, c.PB, c.nparts);
+    (void)mg_apply(s, s->r, s->z, s->sc + ((kk + 1) & 1), c.PZ, kk, c.PB, c.nparts);
 }
 
 // nb spmv launches with an update (and V-cycle) between each two; R.k is the
@@ -761,13 +931,37 @@ static void cg_update(fe_scene* s, const CGSetup& c, CGRun& R, int kk) {
 static void cg_batch(fe_scene* s, const CGSetup& c, CGRun& R, int nb) {
     for (int t = 0; t < nb; ++t) {
         launch_timed(s, FE_KERNEL_CG_SPMV, R.k, k_cg_spmv, dim3((unsigned)c.sh.blocks), dim3(kBlock), c.g,
-                     (const uint16_t*)s->code, c.zr, (const float*)s->d[R.dcur], s->d[1 - R.dcur], s->q,
-                     (const SolverScalars*)(s->sc + (R.k & 1)), s->sc + ((R.k + 1) & 1), (const double*)c.PB, c.pz,
-                     c.nz, c.PA, c.nparts, c.ih2[0], c.ih2[1], c.ih2[2], (const uint8_t*)s->chunk_fluid, c.sh.chunk,
+                     (const uint16_t*)s->code, (const float*)s->z, (const float*)s->d[R.dcur], s->d[1 - R.dcur], s->q,
+                     (const SolverScalars*)(s->sc + (R.k & 1)), s->sc + ((R.k + 1) & 1), (const double*)c.PB,
+                     (const double*)c.PZ, c.nz, c.PA, c.nparts, c.ih2[0], c.ih2[1], c.ih2[2], (const uint8_t*)s->chunk_fluid, c.sh.chunk,
                      c.sh.blocks);
         if (t == nb - 1) break;
         cg_update(s, c, R, R.k);
         ++R.k;
+    }
+}
+
+// n launches of k_cg_step.
+static void cg_steps(fe_scene* s, const CGSetup& c, CGRun& R, int n) {
+    double* const X[2] = {s->p, s->p2};
+    float* const r[2] = {s->r, s->z};
+    float* const q[2] = {s->q, s->q2};
+    double* const part[2] = {c.PB, c.PA};
+    auto step = [&](auto kernel) {
+        const int i = R.k & 1, o = 1 - i;
+        const CGBuffers B{r[i], s->d[i], q[i], X[i], r[o], s->d[o], q[o], X[o]};
+        launch_timed(s, FE_KERNEL_CG_SPMV, R.k, kernel, dim3((unsigned)c.sh.blocks), dim3(kBlock), c.g,
+                     (const uint16_t*)s->code, (const float*)s->b, B, i, (const SolverScalars*)(s->sc + i), s->sc + o,
+                     (const double*)part[i], part[o], c.nparts, c.ih2[0], c.ih2[1], c.ih2[2],
+                     (const uint8_t*)s->chunk_fluid, c.sh.chunk, c.sh.blocks);
+    };
+    // one cell per thread up to 2^18 cells, chunks of several above
+    const bool one = c.sh.chunk <= kBlock;
+    for (; n > 0; --n, ++R.k) {
+        if (c.precond)
+            one ? step(k_cg_step<1, true>) : step(k_cg_step<2, true>);
+        else
+            one ? step(k_cg_step<1, false>) : step(k_cg_step<2, false>);
     }
 }
 
@@ -783,6 +977,7 @@ static hipError_t cg_start(fe_scene* s, const CGSetup& c, CGRun& R) {
     ZeroList L;
     zero_add(L, s->z, 4 * nc);
     zero_add(L, s->q, 4 * nc);
+    if (!c.mg) zero_add(L, s->q2, 4 * nc);
     zero_add(L, s->d[1], 4 * nc);
     if (c.mg) zero_add(L, s->mg[0].x2, 4 * nc);
     // the fused V-cycle skips level-0 tiles without FLUID cells: the coarse
@@ -792,7 +987,7 @@ static hipError_t cg_start(fe_scene* s, const CGSetup& c, CGRun& R) {
     zero_add(L, s->p2, 8 * nc);
     hipLaunchKernelGGL(k_zero_many, dim3((unsigned)L.first[L.n]), dim3(kBlock), 0, s->stream, L);
     hipLaunchKernelGGL(k_cg_init, dim3((unsigned)c.sh.blocks), dim3(kBlock), 0, s->stream, c.g, s->code, s->b, s->p,
-                       s->r, s->z, s->d[0], c.mgx, s->sc, c.PA, c.PB, c.nparts, c.ih2[0], c.ih2[1], c.ih2[2],
+                       s->r, s->d[0], c.mgx, s->sc, c.PA, c.PB, c.mg ? 2 : 4, c.nparts, c.ih2[0], c.ih2[1], c.ih2[2],
                        c.sh.chunk, c.sh.blocks);
     if (c.mg && (e = mg_apply(s, s->r, s->z, s->sc, c.PZ, -1, nullptr, 0)) != hipSuccess) return e;
     R = CGRun{};
@@ -801,21 +996,33 @@ static hipError_t cg_start(fe_scene* s, const CGSetup& c, CGRun& R) {
     return hipGetLastError();
 }
 
-// Host-driven iterations: batches of spmv launches, the host reading the last
-// one's state slot.  resume: the state slot read last said "not done" after a
-// batch launched elsewhere (a captured substep), so the next update comes
-// first.  first: spmv launches in the first batch.
+// Host-driven iterations without multigrid: batches of steps, the host reading
+// the last one's state slot.  first: steps in the first batch.
+static hipError_t cg_step_loop(fe_scene* s, const CGSetup& c, CGRun& R, int first) {
+    hipError_t e;
+    for (int n = first;; n = std::min(std::max(R.k / 8, 8), 64)) {
+        cg_steps(s, c, R, n);
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+        if ((e = read_scalars(s, R.k & 1)) != hipSuccess) return e;
+        kt_flush(s, s->sc_host->done ? s->sc_host->launches - 1 : (1 << 30));
+        if (s->sc_host->done) return hipSuccess;  // the iteration cap ends every solve
+    }
+}
+
+// Host-driven iterations with multigrid: batches of spmv launches, the host
+// reading the last one's state slot.  resume: the state slot read last said
+// "not done" after a batch launched elsewhere (a captured substep), so the
+// next update comes first.  first: spmv launches in the first batch.
 static hipError_t cg_host_loop(fe_scene* s, const fe_solver_desc* d, const CGSetup& c, CGRun& R, int first,
                                bool resume) {
     hipError_t e;
-    const int batch = c.mg ? 4 : 16;
     if (resume) {
         cg_update(s, c, R, R.k);
         ++R.k;
     }
     for (;;) {
         const int nb = std::min(first, d->max_iterations + 1 - R.k);
-        first = c.mg ? 2 : batch;
+        first = 2;
         cg_batch(s, c, R, nb);
         if ((e = hipGetLastError()) != hipSuccess) return e;
         if ((e = read_scalars(s, (R.k + 1) & 1)) != hipSuccess) return e;
@@ -836,13 +1043,19 @@ hipError_t launch_pressure_solve(fe_scene* s, const fe_solver_desc* d) {
     const CGSetup c = cg_setup(s, init.precond);
     CGRun R;
     if ((e = cg_start(s, c, R)) != hipSuccess) return e;
-    // iterations per host check: fewer when each carries a V-cycle; the first
-    // check comes where the previous solve of this kind stopped (warm-started
-    // solves of consecutive substeps take similar counts), so a typical solve
-    // waits for the device once
-    const int prev = s->last_cg_iters[init.precond];
-    const int first = prev > 0 ? std::min(prev + 1, 64) : (c.mg ? 4 : 16);
-    if ((e = cg_host_loop(s, d, c, R, first, false)) != hipSuccess) return e;
+    // the first host check comes where the previous solve of this kind stopped
+    // (warm-started solves of consecutive substeps take similar counts), so a
+    // typical solve waits for the device once; a launch after the stop costs
+    // about 2 us
+    if (c.mg) {
+        const int prev = s->last_cg_iters[2];
+        if ((e = cg_host_loop(s, d, c, R, prev > 0 ? std::min(prev + 1, 64) : 4, false)) != hipSuccess) return e;
+    } else {
+        int& prev = s->last_cg_launches[init.precond];
+        if ((e = cg_step_loop(s, c, R, prev > 0 ? std::min(prev + 1, 1024) : 16)) != hipSuccess) return e;
+        prev = s->sc_host->launches;
+        if (s->sc_host->xbuf) R.xa = s->p2;
+    }
     if (R.xa != s->p) {
         s->p2 = s->p;
         s->p = R.xa;
@@ -862,9 +1075,17 @@ hipError_t capture_pressure_head(fe_scene* s, const fe_solver_desc* d, int iters
     const CGSetup c = cg_setup(s, init.precond);
     CGRun R;
     if ((e = cg_start(s, c, R)) != hipSuccess) return e;
-    cg_batch(s, c, R, std::max(1, std::min(iters, d->max_iterations + 1)));
-    if ((e = hipMemcpyAsync(s->sc_host, s->sc + ((R.k + 1) & 1), sizeof(SolverScalars), hipMemcpyDeviceToHost,
-                            s->stream)) != hipSuccess)
+    int slot;
+    if (c.mg) {
+        cg_batch(s, c, R, std::max(1, std::min(iters, d->max_iterations + 1)));
+        slot = (R.k + 1) & 1;
+    } else {  // recomputed residuals take a second launch
+        const int prev = s->last_cg_launches[c.precond];
+        cg_steps(s, c, R, std::max(2, prev > 0 ? std::min(prev + 2, 1024) : iters));
+        slot = R.k & 1;
+    }
+    if ((e = hipMemcpyAsync(s->sc_host, s->sc + slot, sizeof(SolverScalars), hipMemcpyDeviceToHost, s->stream)) !=
+        hipSuccess)
         return e;
     *out = R;
     return hipGetLastError();
@@ -880,9 +1101,16 @@ hipError_t finish_pressure_after_head(fe_scene* s, const fe_solver_desc* d, cons
     CGRun R = head;
     hipError_t e;
     *resumed = false;
-    if (!s->sc_host->done && R.k + 1 <= d->max_iterations) {
+    if (!c.mg) {
+        if (!s->sc_host->done) {
+            *resumed = true;
+            if ((e = cg_step_loop(s, c, R, 16)) != hipSuccess) return e;
+        }
+        s->last_cg_launches[c.precond] = s->sc_host->launches;
+        if (s->sc_host->xbuf) R.xa = s->p2;
+    } else if (!s->sc_host->done && R.k + 1 <= d->max_iterations) {
         *resumed = true;
-        if ((e = cg_host_loop(s, d, c, R, c.mg ? 2 : 16, true)) != hipSuccess) return e;
+        if ((e = cg_host_loop(s, d, c, R, 2, true)) != hipSuccess) return e;
     }
     if (R.xa != s->p &&
         (e = hipMemcpyAsync(s->p, R.xa, sizeof(double) * cell_count(s->g), hipMemcpyDeviceToDevice, s->stream)) !=
