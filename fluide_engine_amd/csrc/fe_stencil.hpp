@@ -236,36 +236,65 @@ __device__ inline Span block_span(int64_t nc, int64_t chunk, int64_t padded) {
     return s;
 }
 
+// A value of another lane by data-parallel primitive: 0 in the rows that ROWS
+// leaves out and where the source lies outside the row.
+template <int CTRL, int ROWS>
+__device__ inline double dpp_value(double x) {
+    return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(x), CTRL, ROWS, 0xf, true),
+                            __builtin_amdgcn_update_dpp(0, __double2loint(x), CTRL, ROWS, 0xf, true));
+}
+
+// The wavefront's sum, in lane 63: rows of 16 by shifts of 1, 2, 4, 8, then row
+// ends into the next rows.  Every step is a register move; the same sums by
+// cross-lane permutes take an LDS round trip (about 50 ns) each, which shows
+// in kernels of 5 us.
+__device__ inline double wave_sum(double x) {
+    x += dpp_value<0x111, 0xf>(x);
+    x += dpp_value<0x112, 0xf>(x);
+    x += dpp_value<0x114, 0xf>(x);
+    x += dpp_value<0x118, 0xf>(x);
+    x += dpp_value<0x142, 0xa>(x);
+    x += dpp_value<0x143, 0xc>(x);
+    return x;
+}
+
+// Every wavefront's sums to sm; the caller synchronises before reading them.
+template <int NV, int W>
+__device__ inline void wave_sums(const double (&v)[NV], double (*sm)[W]) {
+#pragma unroll
+    for (int q = 0; q < NV; ++q) {
+        const double x = wave_sum(v[q]);
+        if ((threadIdx.x & 63) == 63) sm[q][threadIdx.x >> 6] = x;
+    }
+}
+
+// Their total, waves in order.
+template <int W>
+__device__ inline double waves_total(const double (&row)[W]) {
+    double t = 0.0;
+#pragma unroll
+    for (int w = 0; w < W; ++w) t += row[w];
+    return t;
+}
+
 template <int NV>
 __device__ inline void block_reduce(double (&v)[NV], double (*sm)[kBlock / 64]) {
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-#pragma unroll
-    for (int q = 0; q < NV; ++q) {
-        double x = v[q];
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) x += __shfl_down(x, o, 64);
-        if (lane == 0) sm[q][wid] = x;
-    }
+    wave_sums(v, sm);
     __syncthreads();
 #pragma unroll
-    for (int q = 0; q < NV; ++q) {
-        double t = 0.0;
-#pragma unroll
-        for (int w = 0; w < kBlock / 64; ++w) t += sm[q][w];
-        v[q] = t;  // every thread holds the block total
-    }
+    for (int q = 0; q < NV; ++q) v[q] = waves_total(sm[q]);  // every thread holds the block total
     __syncthreads();
 }
 
-// One FP64 partial per block and value.
-template <int NV>
-__device__ inline void write_partials(double (&v)[NV], double* __restrict__ part) {
+// One FP64 partial per block and value, STRIDE places per block (those past NV
+// zero).  A kernel's last use of LDS: nothing waits for the sums to be read.
+template <int NV, int STRIDE = NV>
+__device__ inline void write_partials(const double (&v)[NV], double* __restrict__ part) {
     __shared__ double sm[NV][kBlock / 64];
-    block_reduce<NV>(v, sm);
-    if (threadIdx.x == 0) {
-#pragma unroll
-        for (int q = 0; q < NV; ++q) part[(int64_t)blockIdx.x * NV + q] = v[q];
-    }
+    wave_sums(v, sm);
+    __syncthreads();
+    if (threadIdx.x < STRIDE)
+        part[(int64_t)blockIdx.x * STRIDE + threadIdx.x] = threadIdx.x < NV ? waves_total(sm[threadIdx.x]) : 0.0;
 }
 
 // A thread's share of a partials array: entries b = first, first + step, ...
@@ -303,19 +332,6 @@ __device__ inline void sum_partials(const double* __restrict__ part, int nparts,
     for (int q = 0; q < NV; ++q) tot[q] = 0.0;
     add_partials<NV>(part, NV, 0, (int)threadIdx.x, kBlock, nparts, tot);
     block_reduce<NV>(tot, sm);
-}
-
-// Two sums in one pass: tot[0] over a[sa * b + oa] (b < na), tot[1] over
-// c[sc * b + oc] (b < nc), each in sum_partials' order, so the values are the same.
-__device__ inline void sum_partials_two(const double* __restrict__ a, int sa, int oa, int na,
-                                        const double* __restrict__ c, int sc, int oc, int nc, double (&tot)[2]) {
-    __shared__ double sm[2][kBlock / 64];
-    double ta[1] = {0.0}, tc[1] = {0.0};
-    add_partials<1>(a, sa, oa, (int)threadIdx.x, kBlock, na, ta);
-    add_partials<1>(c, sc, oc, (int)threadIdx.x, kBlock, nc, tc);
-    tot[0] = ta[0];
-    tot[1] = tc[0];
-    block_reduce<2>(tot, sm);
 }
 
 // Row code of cell (i,j,k) from the markers with BuildSystem's rules

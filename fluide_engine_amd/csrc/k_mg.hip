@@ -648,27 +648,17 @@ constexpr int kFusedThreads = 1024;  // 16 waves per tile
 
 // sum_partials for a kFusedThreads workgroup: every workgroup adds the NV-wide
 // partials in the same fixed order (threads strided over the partials, lanes
-// by the shuffle tree, waves in order), so all derive identical totals.
+// by wave_sum, waves in order), so all derive identical totals.
 template <int NV>
 __device__ inline void sum_partials_fused(const double* __restrict__ part, int nparts, double (&tot)[NV]) {
     __shared__ double sm[NV][kFusedThreads / 64];
 #pragma unroll
     for (int q = 0; q < NV; ++q) tot[q] = 0.0;
     add_partials<NV, 1>(part, NV, 0, (int)threadIdx.x, kFusedThreads, nparts, tot);
-#pragma unroll
-    for (int q = 0; q < NV; ++q) {
-        double x = tot[q];
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) x += __shfl_down(x, o, 64);
-        if ((threadIdx.x & 63) == 0) sm[q][threadIdx.x >> 6] = x;
-    }
+    wave_sums(tot, sm);
     __syncthreads();
 #pragma unroll
-    for (int q = 0; q < NV; ++q) {
-        double t = 0.0;
-        for (int w = 0; w < kFusedThreads / 64; ++w) t += sm[q][w];
-        tot[q] = t;
-    }
+    for (int q = 0; q < NV; ++q) tot[q] = waves_total(sm[q]);
     __syncthreads();
 }
 
@@ -976,18 +966,11 @@ __global__ __launch_bounds__(kFusedThreads) void k_mg_up(FusedArgs a, const floa
             out[fused_index(i, j, k, a.n)] = o;
         }
     }
-    if (L0 && prz) {  // one partial per workgroup: waves in order, lanes by the shuffle tree
-        __shared__ double sm[kFusedThreads / 64];
-        double x = v[0];
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) x += __shfl_down(x, o, 64);
-        if ((threadIdx.x & 63) == 0) sm[threadIdx.x >> 6] = x;
+    if (L0 && prz) {  // one partial per workgroup
+        __shared__ double sm[1][kFusedThreads / 64];
+        wave_sums(v, sm);
         __syncthreads();
-        if (threadIdx.x == 0) {
-            double t = 0.0;
-            for (int w = 0; w < kFusedThreads / 64; ++w) t += sm[w];
-            prz[blockIdx.x] = t;
-        }
+        if (threadIdx.x == 0) prz[blockIdx.x] = waves_total(sm[0]);
     }
 }
 

@@ -17,6 +17,7 @@
 // bit-identical scalars with no atomics and no inter-block fences (the kernel
 // boundary orders the writes); block 0 records the solver state.
 #include <algorithm>
+#include <type_traits>
 #include <utility>
 
 #include "fe_stencil.hpp"
@@ -286,13 +287,33 @@ __global__ __launch_bounds__(kBlock) void k_cg_init(Geom g, const uint16_t* __re
     span_groups_from<G, Stencil64In>(
         early ? g0 + (int64_t)G * kBlock : g0, sp.c1, [&](int64_t c) { return stencil64_in(c, code, x, b, st); },
         use);
-    __shared__ double sm[2][kBlock / 64];
-    block_reduce<2>(v, sm);
-    if (threadIdx.x < stride) pout[(int64_t)blockIdx.x * stride + threadIdx.x] = threadIdx.x < 2 ? v[threadIdx.x] : 0.0;
+    if (stride == 2)
+        write_partials<2>(v, pout);
+    else
+        write_partials<2, 4>(v, pout);
+}
+
+// The CG kernels' prologue: every block derives the iteration's scalars from the
+// last kernels' partials, alike.  The loads of the partials, of the state and
+// of the thread's first group of cells go out together; the first wavefront
+// alone adds up and decides (some hundred FP64 instructions with the quotients
+// and roots, which all waves of a SIMD would otherwise issue in turn), and
+// hands the plan to the others through LDS.
+//
+// G: cells per thread of a group, kBlock apart.  A chunk of 256 cells (grids up
+// to 2^18) is one group of 1, larger chunks take groups of 4; a thread with
+// fewer cells reads its chunk's last one again.
+template <typename F>
+inline void with_group(const SolverShape& sh, F f) {
+    if (sh.chunk <= kBlock)
+        f(std::integral_constant<int, 1>{});
+    else
+        f(std::integral_constant<int, 4>{});
 }
 
 // State slots alternate with the iteration (spmv k reads slot k&1 and writes
 // slot (k+1)&1), so no block can see a half-updated state.
+template <int G>
 __global__ __launch_bounds__(kBlock) void k_cg_spmv(Geom g, const uint16_t* __restrict__ code,
                                                     const float* __restrict__ z, const float* __restrict__ dold,
                                                     float* __restrict__ dnew, float* __restrict__ q,
@@ -301,125 +322,106 @@ __global__ __launch_bounds__(kBlock) void k_cg_spmv(Geom g, const uint16_t* __re
                                                     const double* __restrict__ pz, int nz, double* __restrict__ pout,
                                                     int nparts, float ihx2, float ihy2, float ihz2,
                                                     const uint8_t* __restrict__ cfl, int64_t chunk, int64_t padded) {
-    // The chunk's FLUID flag, then the loads of the thread's first group of
-    // cells, issued before the partial sums and the stop flag are waited for
-    // (they depend on neither; after a stop they go unused).
     const int64_t nc = cell_count(g);
     const Span sp = block_span(nc, chunk, padded);
     const Stride st = stride_of(g.n[0], g.n[1], g.n[2]);
-    const bool body = !cfl || cfl[sp.lb] != 0;
-    constexpr int G = 4;
+    const bool body = sp.c0 < sp.c1 && cfl[sp.lb] != 0;
     struct Raw {
         uint16_t cd;
         float zc, dc, zn[6], dn[6];
     };
+    auto fetch = [&](int64_t c) {
+        Raw w;
+        w.cd = code[c];
+        w.zc = z[c];
+        w.dc = dold[c];
+        code_neighbours(c, st, [&](int64_t n) { return z[n]; }, w.zn);
+        code_neighbours(c, st, [&](int64_t n) { return dold[n]; }, w.dn);
+        return w;
+    };
     const int64_t g0 = sp.c0 + threadIdx.x;
-    const bool pre = body && g0 + (int64_t)(G - 1) * kBlock < sp.c1;
     Raw raw[G];
-    if (pre) {
+    if (body) {
 #pragma unroll
-        for (int u = 0; u < G; ++u) {
-            const int64_t c = g0 + (int64_t)u * kBlock;
-            raw[u].cd = code[c];
-            raw[u].zc = z[c];
-            raw[u].dc = dold[c];
-            code_neighbours(c, st, [&](int64_t n) { return z[n]; }, raw[u].zn);
-            code_neighbours(c, st, [&](int64_t n) { return dold[n]; }, raw[u].dn);
-        }
+        for (int u = 0; u < G; ++u) raw[u] = fetch(min(g0 + (int64_t)u * kBlock, sp.c1 - 1));
     }
-    // ---- state update (every block alike) from r.z of the V-cycle's last sweep
-    // and r.r of the last update
-    double t[2];
-    sum_partials_two(pz, 1, 0, nz, pin, 2, 1, nparts, t);
-    if (in->done) {  // uniform: an earlier spmv stopped the solve
-        if (blockIdx.x == 0 && threadIdx.x == 0) *out = *in;
-        return;
+    // r.z of the V-cycle's last sweep and r.r of the last update
+    __shared__ double sm[2][kBlock / 64];
+    __shared__ double plan_beta;
+    __shared__ int plan_done;
+    {
+        double tz[1] = {0.0}, tr[1] = {0.0};
+        add_partials<1>(pz, 1, 0, (int)threadIdx.x, kBlock, nz, tz);
+        add_partials<1>(pin, 2, 1, (int)threadIdx.x, kBlock, nparts, tr);
+        const double t[2] = {tz[0], tr[0]};
+        wave_sums(t, sm);
     }
-    const int it_prev = in->it;
-    double beta, rr_ref;
-    int it, trig, done, conv, repl, confirm = 0;
-    if (it_prev < 0) {  // first iteration: partials come from k_cg_init
-        it = 0;
-        beta = 0.0;
-        trig = 0;
-        rr_ref = t[1];
-        conv = stop_rule(in, in->bnorm2, t[0], t[1]) ? 1 : 0;
-        done = (conv || in->max_it <= 0) ? 1 : 0;
-    } else {
-        rr_ref = in->replace ? t[1] : in->rr_ref;
-        const double sold = in->sigma;
-        it = it_prev + 1;
-        trig = t[0] > sold ? 1 : 0;
-        beta = t[0] / sold;
-        bool stop = stop_rule(in, in->bnorm2, t[0], t[1]);
-        if (stop && in->relative && !in->replace) {  // confirm on the true residual
-            stop = false;
-            trig = 1;
-            confirm = 1;
-        }
-        conv = stop ? 1 : 0;
-        done = (stop || it >= in->max_it) ? 1 : 0;
-    }
-    repl = (trig || (it % 50 == 0 && it > 0) || t[1] < kReliableDrop2 * rr_ref) ? 1 : 0;
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
+    __syncthreads();
+    if (threadIdx.x < 64) {
         SolverScalars o = *in;
-        o.sigma_old = in->sigma;
-        o.sigma = t[0];
-        o.rr = t[1];
-        o.beta = beta;
-        o.it = it;
-        o.trigger = trig;
-        o.converged = conv;
-        o.done = done;
-        o.replace = repl;
-        o.rr_ref = rr_ref;
-        o.confirm = confirm;
-        *out = o;
+        if (!o.done) {  // else: an earlier spmv stopped the solve
+            const double sigma = waves_total(sm[0]), rr = waves_total(sm[1]), sold = o.sigma;
+            const bool replaced = o.replace != 0;
+            o.sigma_old = sold;
+            o.sigma = sigma;
+            o.rr = rr;
+            o.confirm = 0;
+            if (o.it < 0) {  // first iteration: partials come from k_cg_init
+                o.it = 0;
+                o.beta = 0.0;
+                o.trigger = 0;
+                o.rr_ref = rr;
+                o.converged = stop_rule(in, o.bnorm2, sigma, rr) ? 1 : 0;
+                o.done = (o.converged || o.max_it <= 0) ? 1 : 0;
+            } else {
+                if (replaced) o.rr_ref = rr;
+                ++o.it;
+                o.trigger = sigma > sold ? 1 : 0;
+                o.beta = sigma / sold;
+                bool stop = stop_rule(in, o.bnorm2, sigma, rr);
+                if (stop && o.relative && !replaced) {  // confirm on the true residual
+                    stop = false;
+                    o.trigger = 1;
+                    o.confirm = 1;
+                }
+                o.converged = stop ? 1 : 0;
+                o.done = (stop || o.it >= o.max_it) ? 1 : 0;
+            }
+            o.replace = (o.trigger || (o.it % 50 == 0 && o.it > 0) || rr < kReliableDrop2 * o.rr_ref) ? 1 : 0;
+        }
+        if (threadIdx.x == 0) {
+            plan_beta = o.beta;
+            plan_done = o.done;
+            if (blockIdx.x == 0) *out = o;
+        }
     }
-    if (done) return;
-    // ---- body
+    __syncthreads();
+    if (plan_done) return;
     if (!body) {  // no FLUID cell: d, q stay 0
         if (threadIdx.x == 0) pout[blockIdx.x] = 0.0;
         return;
     }
     const float ih2[3] = {ihx2, ihy2, ihz2};
-    const float fb = (float)beta;
-    auto D = [&](int64_t n) { return fb * dold[n] + z[n]; };  // AXpY(beta, d, s, &d)
+    const float fb = (float)plan_beta;
     double v[1] = {0.0};
-    struct In {
-        uint16_t cd;
-        float dc, nb[6];
-    };
-    auto use = [&](int64_t c, const In& t) {
-        const float qc = code_apply_nb(t.cd, code_center(t.cd, ih2), ih2, t.dc, t.nb);
-        dnew[c] = t.dc;
+    auto use = [&](int64_t c, const Raw& w) {  // AXpY(beta, d, s, &d), here and at the neighbours
+        const float dc = fb * w.dc + w.zc;
+        float nb[6];
+#pragma unroll
+        for (int k = 0; k < 6; ++k) nb[k] = fb * w.dn[k] + w.zn[k];
+        const float qc = code_apply_nb(w.cd, code_center(w.cd, ih2), ih2, dc, nb);
+        dnew[c] = dc;
         q[c] = qc;
-        v[0] += (double)t.dc * (double)qc;
+        v[0] += (double)dc * (double)qc;
     };
-    if (pre) {  // the prefetched group: D from the raw values, as D(n) forms it
 #pragma unroll
-        for (int u = 0; u < G; ++u) {
-            In t;
-            t.cd = raw[u].cd;
-            t.dc = fb * raw[u].dc + raw[u].zc;
-#pragma unroll
-            for (int k = 0; k < 6; ++k) t.nb[k] = fb * raw[u].dn[k] + raw[u].zn[k];
-            use(g0 + (int64_t)u * kBlock, t);
-        }
-    }
-    span_groups_from<G, In>(
-        pre ? g0 + (int64_t)G * kBlock : g0, sp.c1,
-        [&](int64_t c) {
-            In t;
-            t.cd = code[c];
-            t.dc = D(c);
-            code_neighbours(c, st, D, t.nb);
-            return t;
-        },
-        use);
+    for (int u = 0; u < G; ++u)
+        if (g0 + (int64_t)u * kBlock < sp.c1) use(g0 + (int64_t)u * kBlock, raw[u]);
+    span_groups_from<G, Raw>(g0 + (int64_t)G * kBlock, sp.c1, fetch, use);
     write_partials<1>(v, pout);
 }
 
+template <int G>
 __global__ __launch_bounds__(kBlock) void k_cg_update(Geom g, const uint16_t* __restrict__ code,
                                                       const float* __restrict__ b, const double* __restrict__ xo,
                                                       double* __restrict__ xn, const float* __restrict__ d,
@@ -430,47 +432,60 @@ __global__ __launch_bounds__(kBlock) void k_cg_update(Geom g, const uint16_t* __
                                                       const uint8_t* __restrict__ cfl, int64_t chunk, int64_t padded) {
     const int64_t nc = cell_count(g);
     const Span sp = block_span(nc, chunk, padded);
-    // The chunk's FLUID flag, then the loads of the thread's first group of
-    // cells, issued before the partial sum and the solver state are waited for
-    // (they depend on neither; after a stop, or when r is recomputed, they go
-    // unused).
-    const bool body = !cfl || cfl[sp.lb] != 0;
-    constexpr int G = 4;
+    const bool body = sp.c0 < sp.c1 && cfl[sp.lb] != 0;
     struct In {
         double x;
         float d, q, r;
         uint16_t cd;
     };
+    auto fetch = [&](int64_t c) {
+        In t;
+        t.x = xo[c];
+        t.d = d[c];
+        t.q = q[c];
+        t.r = r[c];
+        t.cd = mgx ? code[c] : (uint16_t)0;  // for the first sweep
+        return t;
+    };
     const int64_t g0 = sp.c0 + threadIdx.x;
-    const bool pre = body && g0 + (int64_t)(G - 1) * kBlock < sp.c1;
     In raw[G];
-    if (pre) {
+    if (body) {
 #pragma unroll
-        for (int u = 0; u < G; ++u) {
-            const int64_t c = g0 + (int64_t)u * kBlock;
-            raw[u].x = xo[c];
-            raw[u].d = d[c];
-            raw[u].q = q[c];
-            raw[u].r = r[c];
-            raw[u].cd = code[c];
+        for (int u = 0; u < G; ++u) raw[u] = fetch(min(g0 + (int64_t)u * kBlock, sp.c1 - 1));
+    }
+    __shared__ double sm[1][kBlock / 64];
+    __shared__ double plan_alpha;
+    __shared__ int plan_done, plan_replace;
+    {
+        double t[1] = {0.0};
+        add_partials<1>(pin, 1, 0, (int)threadIdx.x, kBlock, nparts, t);
+        wave_sums(t, sm);
+    }
+    __syncthreads();
+    if (threadIdx.x < 64) {
+        const int done = sc->done, replaces = sc->replace;
+        const double sigma = sc->sigma, dq = waves_total(sm[0]);
+        if (threadIdx.x == 0) {
+            plan_done = done;
+            plan_replace = replaces;
+            plan_alpha = sigma / dq;
+            if (blockIdx.x == 0 && !done) {
+                sc->dq = dq;
+                sc->alpha = plan_alpha;
+            }
         }
     }
-    double t[1];
-    sum_partials<1>(pin, nparts, t);
-    if (sc->done) {  // uniform: keep the x rotation consistent
+    __syncthreads();
+    if (plan_done) {  // keep the x rotation consistent
         for (int64_t c = sp.c0 + threadIdx.x; c < sp.c1; c += kBlock) xn[c] = xo[c];
         return;
-    }
-    const double alpha = sc->sigma / t[0];
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        sc->dq = t[0];
-        sc->alpha = alpha;
     }
     if (!body) {  // no FLUID cell: x, r and the first sweep stay 0
         if (threadIdx.x == 0) pout[2 * blockIdx.x] = pout[2 * blockIdx.x + 1] = 0.0;
         return;
     }
-    const bool replace = sc->replace != 0;
+    const double alpha = plan_alpha;
+    const bool replace = plan_replace != 0;
     const float ih2[3] = {ihx2, ihy2, ihz2};
     const double ih2d[3] = {ihx2, ihy2, ihz2};
     const Stride st = stride_of(g.n[0], g.n[1], g.n[2]);
@@ -494,22 +509,10 @@ __global__ __launch_bounds__(kBlock) void k_cg_update(Geom g, const uint16_t* __
             xn[c] = alpha * (double)t.d + t.x;
             finish(c, t.cd, -fa * t.q + t.r);
         };
-        if (pre) {
 #pragma unroll
-            for (int u = 0; u < G; ++u) use(g0 + (int64_t)u * kBlock, raw[u]);
-        }
-        span_groups_from<G, In>(
-            pre ? g0 + (int64_t)G * kBlock : g0, sp.c1,
-            [&](int64_t c) {
-                In t;
-                t.x = xo[c];
-                t.d = d[c];
-                t.q = q[c];
-                t.r = r[c];
-                t.cd = mgx ? code[c] : (uint16_t)0;  // for the first sweep
-                return t;
-            },
-            use);
+        for (int u = 0; u < G; ++u)
+            if (g0 + (int64_t)u * kBlock < sp.c1) use(g0 + (int64_t)u * kBlock, raw[u]);
+        span_groups_from<G, In>(g0 + (int64_t)G * kBlock, sp.c1, fetch, use);
     }
     write_partials<2>(v, pout);
 }
@@ -527,9 +530,9 @@ __global__ __launch_bounds__(kBlock) void k_cg_update(Geom g, const uint16_t* __
 // recomputed, the iteration takes two launches: r' = b - A x' with x', then
 // d' and q' with the sums of that r'.
 //
-// Bound by latency on all but large grids: the launch, the partial sums, the
-// state, one round of loads (issued before any of these is waited for), the
-// block's sums.  An iteration of 190 k cells in two launches took 12.7 us.
+// Bound by latency on all but large grids: the launch, one round of loads, the
+// partial sums, the state, the block's sums.  An iteration of 190 k cells in
+// two launches took 12.7 us.
 // After a stop at x of buffer xbuf every launch returns.
 // ---------------------------------------------------------------------------
 enum CGPhase { kHaveR = 0, kHaveAll = 1, kHaveAllSummed = 2 };  // r; r, d, q; the same with sigma and r.r in the state
@@ -579,79 +582,70 @@ __global__ __launch_bounds__(kBlock) void k_cg_step(Geom g, const uint16_t* __re
 #pragma unroll
         for (int u = 0; u < G; ++u) raw[u] = fetch(min(g0 + (int64_t)u * kBlock, sp.c1 - 1));
     }
-    if (in->done) {  // uniform
-        if (blockIdx.x == 0 && threadIdx.x == 0) *out = *in;
-        return;
+    __shared__ double sm[4][kBlock / 64];
+    __shared__ double plan_alpha, plan_beta;
+    __shared__ int plan_done, plan_only_d, plan_only_r;
+    {
+        double t[4] = {0.0, 0.0, 0.0, 0.0};  // r.z, r.r, d.q, q.M^-1 q of the read buffers
+        add_partials<4, 4>(pin, 4, 0, (int)threadIdx.x, kBlock, nparts, t);
+        wave_sums(t, sm);
     }
-    double t[4];  // r.z, r.r, d.q, q.M^-1 q of the read buffers
-    sum_partials<4>(pin, nparts, t);
-    const int phase = in->phase;
-    double sigma, rr, rr_ref;
-    int it, trig, repl, confirm, conv = 0, done = 0;
-    if (phase == kHaveAllSummed) {
-        sigma = in->sigma;
-        rr = in->rr;
-        rr_ref = in->rr_ref;
-        it = in->it;
-        trig = in->trigger;
-        repl = in->replace;
-        confirm = in->confirm;
-    } else {
-        sigma = t[0];
-        rr = t[1];
-        confirm = 0;
-        if (in->it < 0) {  // the sums are k_cg_init's
-            it = 0;
-            trig = 0;
-            rr_ref = rr;
-            conv = stop_rule(in, in->bnorm2, sigma, rr) ? 1 : 0;
-            done = (conv || in->max_it <= 0) ? 1 : 0;
-        } else {
-            const bool replaced = phase == kHaveR;
-            rr_ref = replaced ? rr : in->rr_ref;
-            it = in->it + 1;
-            trig = sigma > in->sigma ? 1 : 0;
-            bool stop = stop_rule(in, in->bnorm2, sigma, rr);
-            if (stop && in->relative && !replaced) {  // confirm on the true residual
-                stop = false;
-                trig = 1;
-                confirm = 1;
-            }
-            conv = stop ? 1 : 0;
-            done = (stop || it >= in->max_it) ? 1 : 0;
-        }
-        repl = (trig || (it % 50 == 0 && it > 0) || rr < kReliableDrop2 * rr_ref) ? 1 : 0;
-    }
-    double alpha = 0.0, beta = 0.0;
-    if (phase == kHaveR) {
-        beta = in->it < 0 ? 0.0 : sigma / in->sigma;
-    } else {
-        alpha = sigma / t[2];
-        beta = (alpha * alpha * t[3] - sigma) / sigma;
-        if (!(beta > 0.0)) repl = 1;
-    }
-    const bool only_d = phase == kHaveR, only_r = !only_d && repl;
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
+    __syncthreads();
+    if (threadIdx.x < 64) {
         SolverScalars o = *in;
-        o.sigma_old = in->sigma;
-        o.sigma = sigma;
-        o.rr = rr;
-        o.dq = t[2];
-        o.alpha = alpha;
-        o.beta = beta;
-        o.it = it;
-        o.trigger = trig;
-        o.converged = conv;
-        o.done = done;
-        o.replace = repl;
-        o.rr_ref = rr_ref;
-        o.confirm = confirm;
-        o.phase = only_d ? kHaveAllSummed : (only_r ? kHaveR : kHaveAll);
-        o.launches = in->launches + 1;
-        o.xbuf = parity;
-        *out = o;
+        const int phase = o.phase;
+        if (!o.done) {
+            const double sold = o.sigma;
+            const bool first = o.it < 0, replaced = phase == kHaveR;
+            if (phase != kHaveAllSummed) {
+                o.sigma_old = sold;
+                o.sigma = waves_total(sm[0]);
+                o.rr = waves_total(sm[1]);
+                o.confirm = 0;
+                bool stop = stop_rule(in, o.bnorm2, o.sigma, o.rr);
+                if (first) {  // the sums are k_cg_init's
+                    o.it = 0;
+                    o.trigger = 0;
+                    o.rr_ref = o.rr;
+                } else {
+                    if (replaced) o.rr_ref = o.rr;
+                    ++o.it;
+                    o.trigger = o.sigma > sold ? 1 : 0;
+                    if (stop && o.relative && !replaced) {  // confirm on the true residual
+                        stop = false;
+                        o.trigger = 1;
+                        o.confirm = 1;
+                    }
+                }
+                o.converged = stop ? 1 : 0;
+                o.done = (stop || o.it >= o.max_it) ? 1 : 0;
+                o.replace = (o.trigger || (o.it % 50 == 0 && o.it > 0) || o.rr < kReliableDrop2 * o.rr_ref) ? 1 : 0;
+            }
+            if (phase == kHaveR) {
+                o.beta = first ? 0.0 : o.sigma / sold;
+            } else {
+                o.dq = waves_total(sm[2]);
+                o.alpha = o.sigma / o.dq;
+                o.beta = (o.alpha * o.alpha * waves_total(sm[3]) - o.sigma) / o.sigma;
+                if (!(o.beta > 0.0)) o.replace = 1;
+            }
+            o.phase = phase == kHaveR ? kHaveAllSummed : (o.replace ? kHaveR : kHaveAll);
+            ++o.launches;
+            o.xbuf = parity;
+        }
+        if (threadIdx.x == 0) {
+            plan_alpha = o.alpha;
+            plan_beta = o.beta;
+            plan_done = o.done;
+            plan_only_d = phase == kHaveR;
+            plan_only_r = phase != kHaveR && o.replace;
+            if (blockIdx.x == 0) *out = o;
+        }
     }
-    if (done) return;
+    __syncthreads();
+    if (plan_done) return;
+    const double alpha = plan_alpha, beta = plan_beta;
+    const bool only_d = plan_only_d != 0, only_r = plan_only_r != 0;
     if (!body) {  // no FLUID cell: every vector stays 0
         if (threadIdx.x < 4) pout[4 * (int64_t)blockIdx.x + threadIdx.x] = 0.0;
         return;
@@ -918,10 +912,13 @@ static CGSetup cg_setup(fe_scene* s, int precond) {
 
 static void cg_update(fe_scene* s, const CGSetup& c, CGRun& R, int kk) {
     R.dcur = 1 - R.dcur;
-    launch_timed(s, FE_KERNEL_CG_UPDATE, kk, k_cg_update, dim3((unsigned)c.sh.blocks), dim3(kBlock), c.g,
-                 (const uint16_t*)s->code, (const float*)s->b, (const double*)R.xa, R.xb, (const float*)s->d[R.dcur],
-                 (const float*)s->q, s->r, c.mgx, s->sc + ((kk + 1) & 1), (const double*)c.PA, c.PB, c.nparts,
-                 c.ih2[0], c.ih2[1], c.ih2[2], (const uint8_t*)s->chunk_fluid, c.sh.chunk, c.sh.blocks);
+    with_group(c.sh, [&](auto G) {
+        launch_timed(s, FE_KERNEL_CG_UPDATE, kk, k_cg_update<G.value>, dim3((unsigned)c.sh.blocks), dim3(kBlock), c.g,
+                     (const uint16_t*)s->code, (const float*)s->b, (const double*)R.xa, R.xb,
+                     (const float*)s->d[R.dcur], (const float*)s->q, s->r, c.mgx, s->sc + ((kk + 1) & 1),
+                     (const double*)c.PA, c.PB, c.nparts, c.ih2[0], c.ih2[1], c.ih2[2],
+                     (const uint8_t*)s->chunk_fluid, c.sh.chunk, c.sh.blocks);
+    });
     std::swap(R.xa, R.xb);
     (void)mg_apply(s, s->r, s->z, s->sc + ((kk + 1) & 1), c.PZ, kk, c.PB, c.nparts);
 }
@@ -930,11 +927,13 @@ static void cg_update(fe_scene* s, const CGSetup& c, CGRun& R, int kk) {
 // last spmv's iteration afterwards.
 static void cg_batch(fe_scene* s, const CGSetup& c, CGRun& R, int nb) {
     for (int t = 0; t < nb; ++t) {
-        launch_timed(s, FE_KERNEL_CG_SPMV, R.k, k_cg_spmv, dim3((unsigned)c.sh.blocks), dim3(kBlock), c.g,
-                     (const uint16_t*)s->code, (const float*)s->z, (const float*)s->d[R.dcur], s->d[1 - R.dcur], s->q,
-                     (const SolverScalars*)(s->sc + (R.k & 1)), s->sc + ((R.k + 1) & 1), (const double*)c.PB,
-                     (const double*)c.PZ, c.nz, c.PA, c.nparts, c.ih2[0], c.ih2[1], c.ih2[2], (const uint8_t*)s->chunk_fluid, c.sh.chunk,
-                     c.sh.blocks);
+        with_group(c.sh, [&](auto G) {
+            launch_timed(s, FE_KERNEL_CG_SPMV, R.k, k_cg_spmv<G.value>, dim3((unsigned)c.sh.blocks), dim3(kBlock), c.g,
+                         (const uint16_t*)s->code, (const float*)s->z, (const float*)s->d[R.dcur], s->d[1 - R.dcur],
+                         s->q, (const SolverScalars*)(s->sc + (R.k & 1)), s->sc + ((R.k + 1) & 1),
+                         (const double*)c.PB, (const double*)c.PZ, c.nz, c.PA, c.nparts, c.ih2[0], c.ih2[1], c.ih2[2],
+                         (const uint8_t*)s->chunk_fluid, c.sh.chunk, c.sh.blocks);
+        });
         if (t == nb - 1) break;
         cg_update(s, c, R, R.k);
         ++R.k;
