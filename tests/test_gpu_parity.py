@@ -418,3 +418,31 @@ def test_dam_break_pic_32_run_drift(ctx):
     assert np.abs(gx.mean(0) - ox.mean(0)).max() < 2e-3
     print(f"[gpu] fluid cells t0={fluid0} t50: gpu={fg} oracle={fo}", flush=True)
     g.close()
+
+
+@pytest.mark.parametrize("n", [(2, 2, 2), (5, 3, 9), (40, 40, 40), (41, 40, 41), (33, 7, 70)])
+@pytest.mark.parametrize("search", [capi.SDF_SEARCH_CELLS, capi.SDF_SEARCH_BUCKETS])
+def test_sdf_lane_variants(ctx, n, search):
+    """Grids on both sides of the size up to which the cell scan takes 8 lanes
+    per cell (2^16 cells), with ragged blocks, anisotropic spacing, cells of
+    no, one and many particles: the negative values (bucket search: all) are
+    the oracle's bit for bit."""
+    print(f"[gpu] sdf lanes {n} search={search}", flush=True)
+    rng = np.random.default_rng(sum(n))
+    size = (1.0, 0.9, 1.3)
+    count = 3 * n[0] * n[1] * n[2] // 2
+    x = (rng.uniform(0.0, 1.0, (count, 3)) * np.array(size) * np.array([0.7, 0.5, 0.9])).astype(np.float32)
+    x[: count // 8] = x[0] + (rng.uniform(-0.01, 0.01, (count // 8, 3))).astype(np.float32)  # a crowd in few cells
+    x = np.clip(x, 0.0, np.array(size, np.float32))
+    desc = capi.scene_desc(n, method=capi.FLIP, size=size, max_particles=count)
+    g = capi.Scene(ctx, desc)
+    g.set_sdf_search(search)
+    g.upload_particles(x, np.zeros_like(x))
+    g.run_stage(capi.STAGE_SDF)
+    o = orc.Scene(n, size=size, method=orc.FLIP, blend=desc.blend, max_cfl=desc.max_cfl)
+    o.set_particles(x.astype(np.float64), np.zeros(x.shape))
+    o.build_sdf()
+    got, want = g.get(capi.GRID_SDF), o.get(orc.SDF)
+    where = np.ones(want.shape, bool) if search == capi.SDF_SEARCH_BUCKETS else (want < 0) | (got < 0)
+    assert np.array_equal(got[where], want[where])
+    g.close()
