@@ -59,14 +59,19 @@ def kernel_bytes_per_cell(kernel, solver, mg_split=False):
     return b
 
 
+def p2g_components(n):
+    """Components per launch of the P2G scatter: all three below 4096 workgroups (8x8x8 faces) each."""
+    return 1 if ((n + 8) // 8) * ((n + 7) // 8) ** 2 >= 4096 else 3
+
+
 def kernel_bytes_per_launch(kernel, solver, n, npart, mg_split=False):
     """Algorithmic HBM bytes of one launch of a timed kernel on the n^3 FLIP scene."""
     cells = n ** 3
     if kernel in KERNEL_BYTES_PER_CELL:
         return int(kernel_bytes_per_cell(kernel, solver, mg_split) * cells)
     faces = (n + 1) * n * n  # per component
-    if kernel == "p2g":  # one of three component launches: a third of the x, v read (8 of 24 per particle),
-        return 8 * npart + 8 * faces  # the face velocity and the FLIP snapshot written (8 per face)
+    if kernel == "p2g":  # per component a third of the x, v read (8 of 24 per particle), the face velocity and the
+        return p2g_components(n) * (8 * npart + 8 * faces)  # FLIP snapshot written (8 per face)
     if kernel == "g2p_move":  # read x, v (24) and write x, v (24) per particle; read u, v, w + snapshot (24 per face)
         return 48 * npart + 8 * 3 * faces
     if kernel == "sdf":  # read every particle position (12), cell starts (4) and write the SDF (8) per cell
@@ -81,7 +86,7 @@ def kernel_impl_bytes_per_launch(kernel, n, npart):
         # candidate of about 900 / 512 face blocks (10 x 10 x 9 candidate cells per 8 x 8 x 8 faces); two bin
         # starts (8) per row of candidate cells (100 rows per 512 faces); u + marker + FLIP snapshot (9) per face
         faces = (n + 1) * n * n
-        return int(20 * npart * 900 / 512 + 8 * 100 * faces / 512 + 9 * faces)
+        return p2g_components(n) * int(20 * npart * 900 / 512 + 8 * 100 * faces / 512 + 9 * faces)
     return None
 
 

@@ -737,21 +737,36 @@ constexpr int kScRows = (kScB + 2) * (kScB + 2);               // x rows of cand
 constexpr int kScBases = (kScB + 1) * (kScB + 1) * (kScB + 1); // stencil bases with a node in the block
 static_assert(kScRows <= 128, "one wavefront scans the row lengths, two per lane");
 
+struct ScatterLds {
+    unsigned long long num[kScSlots], den[kScSlots];
+    uint32_t occ[(kScBases + 31) / 32];
+    int32_t first[kScRows], pre[kScRows + 1];
+};
+
+struct ScatterArgs {
+    float* out[3];
+    uint8_t* mark[3];
+    float* snap[3];
+    int nb[3][3];  // face blocks per axis of each component
+    int padded;    // workgroups per component (a multiple of 8)
+};
+
 template <int C, int METHOD>
-__global__ __launch_bounds__(kScThreads) void k_p2g_scatter(Geom g, const float* __restrict__ V,
-                                                        const float* __restrict__ Cm,
-                                                        const float4* __restrict__ pos4, int64_t cap,
-                                                        const int32_t* __restrict__ start,
-                                                        const uint32_t* __restrict__ bound, int head,
-                                                        float* __restrict__ out, uint8_t* __restrict__ mark,
-                                                        float* __restrict__ snap, int nbx, int nby, int nbz,
-                                                        int64_t padded) {
-    __shared__ unsigned long long s_num[kScSlots], s_den[kScSlots];
-    __shared__ uint32_t s_occ[(kScBases + 31) / 32];
-    __shared__ int32_t s_first[kScRows], s_pre[kScRows + 1];
+__device__ inline void p2g_scatter_block(const Geom& g, const float* __restrict__ V, const float* __restrict__ Cm,
+                                         const float4* __restrict__ pos4, int64_t cap,
+                                         const int32_t* __restrict__ start, const uint32_t* __restrict__ bound,
+                                         int head, const ScatterArgs& A, ScatterLds& L) {
+    unsigned long long *s_num = L.num, *s_den = L.den;
+    uint32_t* s_occ = L.occ;
+    int32_t *s_first = L.first, *s_pre = L.pre;
+    float* __restrict__ out = A.out[C];
+    uint8_t* __restrict__ mark = A.mark[C];
+    float* __restrict__ snap = A.snap[C];
+    const int nbx = A.nb[C][0], nby = A.nb[C][1], nbz = A.nb[C][2];
     const P2GFixed fx = p2g_fixed(bound, C, head);
-    const int64_t blk = xcd_remap(blockIdx.x, padded);
-    if (blk >= (int64_t)nbx * nby * nbz) return;  // the whole workgroup
+    const int per = A.padded / kXcds;  // xcd_remap
+    const int blk = (int)(blockIdx.x % kXcds) * per + (int)(blockIdx.x / kXcds);
+    if (blk >= nbx * nby * nbz) return;  // the whole workgroup
     int bi, bj, bk;
     split_index(blk, nbx, nby, bi, bj, bk);
     const int F0[3] = {bi * kScB, bj * kScB, bk * kScB};
@@ -912,6 +927,27 @@ __global__ __launch_bounds__(kScThreads) void k_p2g_scatter(Geom g, const float*
         out[f] = res;
         mark[f] = (uint8_t)m;
         if (METHOD == FE_FLIP) snap[f] = res;  // FLIP snapshot right after P2G (flip_simulator.cpp:107-118)
+    }
+}
+
+// COMP: the component, or 3 for all three in one launch (blockIdx.y).
+template <int COMP, int METHOD>
+__global__ __launch_bounds__(kScThreads, 8) void k_p2g_scatter(Geom g, const float* __restrict__ V,
+                                                               const float* __restrict__ Cm,
+                                                               const float4* __restrict__ pos4, int64_t cap,
+                                                               const int32_t* __restrict__ start,
+                                                               const uint32_t* __restrict__ bound, int head,
+                                                               ScatterArgs A) {
+    __shared__ ScatterLds L;
+    if constexpr (COMP < 3) {
+        p2g_scatter_block<COMP, METHOD>(g, V, Cm, pos4, cap, start, bound, head, A, L);
+    } else {
+        if (blockIdx.y == 0)
+            p2g_scatter_block<0, METHOD>(g, V, Cm, pos4, cap, start, bound, head, A, L);
+        else if (blockIdx.y == 1)
+            p2g_scatter_block<1, METHOD>(g, V, Cm, pos4, cap, start, bound, head, A, L);
+        else
+            p2g_scatter_block<2, METHOD>(g, V, Cm, pos4, cap, start, bound, head, A, L);
     }
 }
 
@@ -1206,19 +1242,35 @@ static hipError_t p2g_method(fe_scene* s) {
     const Particles& P = s->P[s->cur];
     const Geom& g = s->g;
     const int head = p2g_head(s->np);
-    for (int c = 0; c < 3; ++c) {
-        if (s->tune.p2g == FE_P2G_SCATTER) {
-            const int nb[3] = {(face_dim(g, c, 0) + kScB - 1) / kScB, (face_dim(g, c, 1) + kScB - 1) / kScB,
-                               (face_dim(g, c, 2) + kScB - 1) / kScB};
-            const int64_t padded = pad_blocks((int64_t)nb[0] * nb[1] * nb[2]);
-            auto kern = c == 0 ? k_p2g_scatter<0, METHOD>
-                               : (c == 1 ? k_p2g_scatter<1, METHOD> : k_p2g_scatter<2, METHOD>);
-            launch_timed(s, FE_KERNEL_P2G, 0, kern, dim3((unsigned)padded), dim3(kScThreads), g, (const float*)P.v,
-                         (const float*)P.C, (const float4*)s->pos4, s->cap,
-                         (const int32_t*)s->cell_start, (const uint32_t*)s->p2g_bound, head, s->u[c], s->mark[c],
-                         s->snap[c], nb[0], nb[1], nb[2], padded);
-            continue;
+    if (s->tune.p2g == FE_P2G_SCATTER) {
+        ScatterArgs A{};
+        for (int c = 0; c < 3; ++c) {
+            A.out[c] = s->u[c];
+            A.mark[c] = s->mark[c];
+            A.snap[c] = s->snap[c];
+            for (int a = 0; a < 3; ++a) A.nb[c][a] = (face_dim(g, c, a) + kScB - 1) / kScB;
+            A.padded = std::max(A.padded, (int)pad_blocks((int64_t)A.nb[c][0] * A.nb[c][1] * A.nb[c][2]));
         }
+        auto launch = [&](auto kern, unsigned comps) {
+            launch_timed(s, FE_KERNEL_P2G, 0, kern, dim3((unsigned)A.padded, comps), dim3(kScThreads), g,
+                         (const float*)P.v, (const float*)P.C, (const float4*)s->pos4, s->cap,
+                         (const int32_t*)s->cell_start, (const uint32_t*)s->p2g_bound, head, A);
+        };
+        // One launch: on a small grid a component's blocks do not fill the chip
+        // and each launch costs its latency (32^3 FLIP 47 us in three, 19 in
+        // one; 96^3 150 / 141; APIC 128^3 437 / 411).  From 4096 blocks a
+        // component, without APIC's affine rows, the kernel for one component
+        // with its fewer registers wins (128^3 FLIP 265 / 275).
+        if (METHOD == FE_APIC || A.padded < 4096) {
+            launch(k_p2g_scatter<3, METHOD>, 3);
+        } else {
+            launch(k_p2g_scatter<0, METHOD>, 1);
+            launch(k_p2g_scatter<1, METHOD>, 1);
+            launch(k_p2g_scatter<2, METHOD>, 1);
+        }
+        return hipGetLastError();
+    }
+    for (int c = 0; c < 3; ++c) {
         if (s->tune.p2g == FE_P2G_FACES) {
             const int64_t padded = pad_blocks((face_count(g, c) + kBlock - 1) / kBlock);
             auto kern = c == 0 ? k_p2g_face<0, METHOD> : (c == 1 ? k_p2g_face<1, METHOD> : k_p2g_face<2, METHOD>);
