@@ -1531,8 +1531,8 @@ int fe_surface_build(fe_scene* s, int64_t* vertex_count, int64_t* triangle_count
     HIPCHK(ctx, hipSetDevice(ctx->device));
     HIPCHK(ctx, surface_build(s));
     const McState& m = s->mc;
-    if (vertex_count) *vertex_count = m.nv3 + (int64_t)m.cap_pos.size() / 3;
-    if (triangle_count) *triangle_count = m.nt3 + (int64_t)m.cap_tri.size() / 3;
+    if (vertex_count) *vertex_count = m.vertices;
+    if (triangle_count) *triangle_count = m.triangles;
     return FE_OK;
 }
 

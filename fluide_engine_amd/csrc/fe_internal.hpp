@@ -473,15 +473,15 @@ struct McState {
     int32_t *flag = nullptr, *vid = nullptr, *cnt = nullptr, *toff = nullptr, *sums = nullptr;
     void* tables = nullptr;      // FE_SURFACE_CLOSED cube tables
     void* tables_ref = nullptr;  // FE_SURFACE_REFERENCE cube tables
-    double* planes = nullptr;
-    int64_t plane_stride = 0;
+    void *caps = nullptr, *caps_ref = nullptr;  // and the two modes' square tables
+    int32_t *capv = nullptr, *capt = nullptr, *capvo = nullptr, *capto = nullptr;  // per boundary square: vertices
+                                                                                   // and triangles, their offsets
+    int32_t* capid = nullptr;  // vertex index by cap key
     double *pos = nullptr, *nrm = nullptr;
     int32_t* tri = nullptr;
     double* comb = nullptr;  // fluid SDF combined with the collider's
     int64_t vcap = 0, ncap = 0, tcap = 0;
-    int64_t nv3 = 0, nt3 = 0;  // cube-part vertices and triangles of the last build
-    std::vector<double> cap_pos, cap_nrm;
-    std::vector<int32_t> cap_tri;
+    int64_t vertices = 0, triangles = 0;  // of the last build, the caps' last
     bool built = false;
 };
 }  // namespace fe

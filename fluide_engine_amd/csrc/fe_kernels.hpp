@@ -65,7 +65,7 @@ float* mg_first_sweep_target(fe_scene* s);  // where the CG kernels write level 
 void mg_free(fe_scene* s);
 
 // k_surface.hip: MarchingCubesSolver::BuildSurface on the fluid SDF
-hipError_t surface_build(fe_scene* s);  // counts in s->mc (nv3 + caps, nt3 + caps)
+hipError_t surface_build(fe_scene* s);  // counts in s->mc
 hipError_t surface_download(fe_scene* s, double* pos, double* nrm, int32_t* tri);
 void surface_free(fe_scene* s);
 

@@ -81,6 +81,20 @@ def test_surface_parity(ctx, case, mode):
 
 
 @pytest.mark.parametrize("mode", MODES)
+@pytest.mark.parametrize("n", [(2, 2, 2), (2, 3, 5), (5, 2, 3), (3, 5, 2), (67, 3, 2), (3, 2, 70), (9, 41, 11)])
+def test_surface_caps_on_ragged_planes(ctx, n, mode):
+    """Every square case on every boundary plane, planes of one square, rows
+    that end inside a block, nodes exactly on the surface."""
+    print(f"[gpu] surface caps {n} mode {mode}", flush=True)
+    sdf = np.random.default_rng(5).integers(-2, 3, (n[2], n[1], n[0])).astype(np.float64)
+    g, o = _scene_pair(ctx, n, sdf)
+    g.set_surface_mode(mode)
+    o.set_surface_mode(mode)
+    _compare(g.surface(), o.surface())
+    g.close()
+
+
+@pytest.mark.parametrize("mode", MODES)
 def test_surface_of_dam_break(ctx, mode):
     """GetSurface after a frame (src/simulation_runner.cpp:35-36): the fluid
     SDF of the last substep's start, with the reference's positive values.
