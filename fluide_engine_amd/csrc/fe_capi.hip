@@ -1395,64 +1395,20 @@ int fe_net_loss_and_grads(fe_net* n, const int32_t dims[3], const double h[3], c
     fe_ctx* ctx = n->ctx;
     HIPCHK(ctx, hipSetDevice(ctx->device));
     const int64_t V = (int64_t)dims[0] * dims[1] * dims[2];
-    float *db = nullptr, *dt = nullptr, *dl = nullptr;
-    uint8_t* df = nullptr;
-    uint16_t* dc = nullptr;
-    auto cleanup = [&]() {
-        if (db) (void)hipFree(db);
-        if (dt) (void)hipFree(dt);
-        if (dl) (void)hipFree(dl);
-        if (df) (void)hipFree(df);
-        if (dc) (void)hipFree(dc);
-    };
-    hipError_t e = hipSuccess;
-    if ((e = hipMalloc((void**)&db, sizeof(float) * V)) != hipSuccess ||
-        (e = hipMalloc((void**)&dt, sizeof(float) * V)) != hipSuccess ||
-        (e = hipMalloc((void**)&dl, sizeof(float))) != hipSuccess || (e = hipMalloc((void**)&df, V)) != hipSuccess ||
-        (e = hipMalloc((void**)&dc, sizeof(uint16_t) * V)) != hipSuccess ||
-        (e = hipMemcpy(db, b, sizeof(float) * V, hipMemcpyHostToDevice)) != hipSuccess ||
-        (e = hipMemcpy(dt, target, sizeof(float) * V, hipMemcpyHostToDevice)) != hipSuccess ||
-        (e = hipMemcpy(df, flags, V, hipMemcpyHostToDevice)) != hipSuccess) {
-        cleanup();
-        return hip_fail(ctx, e, "fe_net_loss_and_grads upload");
-    }
-    double ss = 0.0;
-    for (int64_t v = 0; v < V; ++v) ss += (double)b[v] * b[v];
-    const double rms = std::sqrt(ss / (double)V);
     LossIn in;
-    double energy = 0.0;
-    for (int64_t v = 0; v < V; ++v)
-        if (flags[v] == FE_FLUID) {
-            ++in.nfluid;
-            energy += (double)b[v] * target[v];
-        }
-    in.target = dt;
-    in.flags = df;
-    in.code = dc;
-    in.b = db;
-    in.energy = energy;
     for (int a = 0; a < 3; ++a) {
         const double ha = h ? h[a] : 1.0 / dims[a];
         in.ih2[a] = 1.0 / (ha * ha);
     }
-    if ((e = net_ensure(n, dims)) == hipSuccess && (e = net_codes(n, dims, df, dc)) == hipSuccess &&
-        (e = net_forward(n, db, df, rms > 0 ? rms : 1.0)) == hipSuccess && (e = net_backward(n, in, dl)) == hipSuccess)
-        e = hipStreamSynchronize(n->stream);
-    if (e == hipSuccess && loss) e = hipMemcpy(loss, n->scal, sizeof(double), hipMemcpyDeviceToHost);
-    if (e == hipSuccess && prediction) e = hipMemcpy(prediction, n->out, sizeof(float) * V, hipMemcpyDeviceToHost);
-    if (e == hipSuccess && grads) {
-        float* g = grads;
-        for (auto& L : n->L) {
-            const int64_t wsz = 27LL * L.cin * L.cout;
-            if (e == hipSuccess) e = hipMemcpy(g, L.gw, sizeof(float) * wsz, hipMemcpyDeviceToHost);
-            g += wsz;
-            if (e == hipSuccess) e = hipMemcpy(g, L.gb, sizeof(float) * L.cout, hipMemcpyDeviceToHost);
-            g += L.cout;
-        }
-        if (e == hipSuccess) e = hipMemcpy(g, n->ghead, sizeof(float) * 17, hipMemcpyDeviceToHost);
-    }
-    cleanup();
-    HIPCHK(ctx, e);
+    double rms = 0.0;
+    HIPCHK(ctx, net_host_inputs(n, dims, b, flags, target, in, &rms));
+    HIPCHK(ctx, net_forward(n, in.b, in.flags, rms > 0 ? rms : 1.0));
+    HIPCHK(ctx, net_backward(n, in, n->in_loss));
+    HIPCHK(ctx, hipStreamSynchronize(n->stream));
+    if (loss) HIPCHK(ctx, hipMemcpy(loss, n->scal, sizeof(double), hipMemcpyDeviceToHost));
+    if (prediction) HIPCHK(ctx, hipMemcpy(prediction, n->out, sizeof(float) * V, hipMemcpyDeviceToHost));
+    if (grads)
+        HIPCHK(ctx, hipMemcpy(grads, n->grads, sizeof(float) * (size_t)net_param_count(), hipMemcpyDeviceToHost));
     return FE_OK;
 }
 

@@ -29,7 +29,7 @@ struct NetLayer {
     int cin = 0, cout = 0;
     float* w = nullptr;  // 27 * cin * cout, (t * cin + ci) * cout + co
     float* b = nullptr;
-    float *gw = nullptr, *gb = nullptr;
+    float *gw = nullptr, *gb = nullptr;  // inside fe_net::grads
     float *mw = nullptr, *vw = nullptr, *mb = nullptr, *vb = nullptr;  // Adam moments
     uint16_t* wp = nullptr;   // BF16, packed for the forward MFMA B operand
     uint16_t* wpt = nullptr;  // BF16, flipped and transposed, packed for the backward data pass
@@ -70,6 +70,7 @@ struct fe_net {
     hipStream_t stream = nullptr;
     fe::NetLayer L[fe::kNetLayers];
     float *head = nullptr, *ghead = nullptr, *mhead = nullptr, *vhead = nullptr;  // 1x1 head: 16 weights + bias
+    float* grads = nullptr;  // every layer's gw and gb, then ghead: the parameters' order
     int64_t adam_t = 0;
     std::vector<fe::NetSample> samples;
 
@@ -86,6 +87,10 @@ struct fe_net {
     float *wpart = nullptr, *bpart = nullptr;  // weight- and bias-gradient partials
     uint16_t* Xt[4] = {nullptr, nullptr, nullptr, nullptr};  // per level: a layer's input as zero-bordered planes
     uint16_t* Gt[4] = {nullptr, nullptr, nullptr, nullptr};  // and its dpre as planes
+    // fe_net_loss_and_grads's inputs, row codes and loss (allocated by its first call)
+    float *in_b = nullptr, *in_target = nullptr, *in_loss = nullptr;
+    uint8_t* in_flags = nullptr;
+    uint16_t* in_code = nullptr;
     double* red = nullptr;   // reduction partials (FP64)
     int64_t red_cap = 0;
     float* losses = nullptr; // per training step
@@ -116,6 +121,10 @@ hipError_t net_add_sample(fe_net* net, fe_scene* s);
 hipError_t net_train(fe_net* net, int steps, float lr, uint64_t seed);
 // x0 = alpha * prediction in the scene's pressure (FP64), from its b and flags
 hipError_t net_warm_start(fe_net* net, fe_scene* s);
+// Host inputs to the device, their sums (rms of b, FLUID cells, b . target) and
+// row codes; the buffers are the net's and last until its grid size changes.
+hipError_t net_host_inputs(fe_net* net, const int n[3], const float* b, const uint8_t* flags, const float* target,
+                           LossIn& in, double* rms_b);
 hipError_t net_fluid_count(fe_net* net, const uint8_t* flags, int64_t V, int64_t* count);
 
 }  // namespace fe
