@@ -410,8 +410,13 @@ __device__ inline uint32_t byte_of(uint32_t w, int q) { return (w >> (8 * q)) & 
 // Each block covers kBlock quads (4 consecutive faces) of one component
 // (blocks [0, b0) u, [b0, b1) v, [b1, ...) w), so the component and its arrays
 // are uniform per block.  A thread reads the validity bytes of its quad and of
-// the quad's six neighbour quads as 32-bit words (12 loads for 4 faces instead
-// of 28 byte loads) before it uses any of them.
+// the quad's six neighbour quads as 32-bit words (7 loads for 4 faces instead
+// of 28 byte loads) before it uses any of them.  The sweep is bound by its
+// instructions, and most quads have no face to fill: all four valid, or none of
+// the 24 neighbours (a neighbour across the grid's edge only makes this test
+// pass, the faces' own tests follow).  Those leave before the index division
+// and the neighbours' tests, and quads whose neighbour words lie inside the
+// array read them unaligned without bytes4's clamps.
 __global__ __launch_bounds__(kBlock) void k_extrapolate(Geom g, FaceSet a, ValidSet vs, int64_t b0, int64_t b1) {
     const int64_t blk = blockIdx.x;
     const int c = blk < b0 ? 0 : (blk < b1 ? 1 : 2);
@@ -425,48 +430,69 @@ __global__ __launch_bounds__(kBlock) void k_extrapolate(Geom g, FaceSet a, Valid
     const int64_t f0 = 4 * (lb * kBlock + threadIdx.x);
     if (f0 >= nf) return;
     // neighbour order of ExtrapolateToRegion: i+1, i-1, j+1, j-1, k+1, k-1
-    const uint32_t self = bytes4(vin, nf, f0);
-    const uint32_t xm = bytes4(vin, nf, f0 - 1), xp = bytes4(vin, nf, f0 + 1);
-    const uint32_t ym = bytes4(vin, nf, f0 - st[1]), yp = bytes4(vin, nf, f0 + st[1]);
-    const uint32_t zm = bytes4(vin, nf, f0 - st[2]), zp = bytes4(vin, nf, f0 + st[2]);
-    int i, j, k;
-    split_index(f0, sx, sy, i, j, k);
-    uint32_t out = 0;
+    uint32_t self, xm, xp, ym, yp, zm, zp;
+    if (f0 >= st[2] && f0 + st[2] + 4 <= nf) {
+        const uint8_t* p = vin + f0;
+        auto word = [](const uint8_t* q) {
+            uint32_t w;
+            __builtin_memcpy(&w, q, 4);
+            return w;
+        };
+        self = word(p);
+        xm = word(p - 1);
+        xp = word(p + 1);
+        ym = word(p - sx);
+        yp = word(p + sx);
+        zm = word(p - st[2]);
+        zp = word(p + st[2]);
+    } else {
+        self = bytes4(vin, nf, f0);
+        xm = bytes4(vin, nf, f0 - 1);
+        xp = bytes4(vin, nf, f0 + 1);
+        ym = bytes4(vin, nf, f0 - st[1]);
+        yp = bytes4(vin, nf, f0 + st[1]);
+        zm = bytes4(vin, nf, f0 - st[2]);
+        zp = bytes4(vin, nf, f0 + st[2]);
+    }
+    // 1 in every byte of self that is not 0
+    uint32_t out = (((self & 0x7f7f7f7fu) + 0x7f7f7f7fu) | self) >> 7 & 0x01010101u;
+    if (f0 + 4 > nf || (out != 0x01010101u && (xm | xp | ym | yp | zm | zp) != 0)) {
+        int i, j, k;
+        split_index(f0, sx, sy, i, j, k);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const int64_t f = f0 + q;
-        if (f < nf) {
-            if (byte_of(self, q)) {
-                out |= 1u << (8 * q);
-            } else {
-                const bool in[6] = {i + 1 < sx, i > 0, j + 1 < sy, j > 0, k + 1 < sz, k > 0};
-                const uint32_t nb[6] = {byte_of(xp, q), byte_of(xm, q), byte_of(yp, q),
-                                        byte_of(ym, q), byte_of(zp, q), byte_of(zm, q)};
-                float sum = 0.0f;
-                unsigned count = 0;
+        for (int q = 0; q < 4; ++q) {
+            const int64_t f = f0 + q;
+            if (f < nf) {
+                if (!byte_of(self, q)) {
+                    const bool in[6] = {i + 1 < sx, i > 0, j + 1 < sy, j > 0, k + 1 < sz, k > 0};
+                    const uint32_t nb[6] = {byte_of(xp, q), byte_of(xm, q), byte_of(yp, q),
+                                            byte_of(ym, q), byte_of(zp, q), byte_of(zm, q)};
+                    float sum = 0.0f;
+                    unsigned count = 0;
 #pragma unroll
-                for (int d = 0; d < 6; ++d) {
-                    if (!in[d] || !nb[d]) continue;
-                    sum += A[(d & 1) ? f - st[d >> 1] : f + st[d >> 1]];
-                    ++count;
-                }
-                if (count > 0) {
-                    A[f] = sum / (float)count;
-                    out |= 1u << (8 * q);
+                    for (int d = 0; d < 6; ++d) {
+                        if (!in[d] || !nb[d]) continue;
+                        sum += A[(d & 1) ? f - st[d >> 1] : f + st[d >> 1]];
+                        ++count;
+                    }
+                    if (count > 0) {
+                        A[f] = sum / (float)count;
+                        out |= 1u << (8 * q);
+                    }
                 }
             }
-        }
-        if (++i == sx) {
-            i = 0;
-            if (++j == sy) {
-                j = 0;
-                ++k;
+            if (++i == sx) {
+                i = 0;
+                if (++j == sy) {
+                    j = 0;
+                    ++k;
+                }
             }
         }
     }
     uint8_t* o = vout + f0;
-    if (f0 + 4 <= nf && ((uintptr_t)o & 3) == 0) {
-        *(uint32_t*)o = out;
+    if (f0 + 4 <= nf) {
+        __builtin_memcpy(o, &out, 4);
     } else {
 #pragma unroll
         for (int q = 0; q < 4; ++q)
