@@ -350,12 +350,6 @@ __device__ inline float lane_read(float v, int lane) {
     return __int_as_float(__builtin_amdgcn_ds_bpermute(lane << 2, __float_as_int(v)));
 }
 
-// mg_weight of any row: a non-FLUID row's weight is omega (diagonal 1).
-__device__ inline float lanes_weight(uint32_t cd, const CodeLanes& t, float omega) {
-    const float w = lane_read(t.wgt, code_lane(cd));
-    return (cd & kFluidBit) ? w : omega;
-}
-
 // A x at a FLUID row whose neighbours outside FLUID hold 0: a FLUID row
 // couples to exactly its FLUID neighbours, and every vector of the V-cycle is
 // 0 outside FLUID cells (the CG start puts the solution's non-FLUID entries at
@@ -582,24 +576,28 @@ __global__ __launch_bounds__(kBlock) void k_mg_prolong(const float* __restrict__
 // same order; only the source of a neighbour value differs, and a neighbour
 // outside the grid, which enters with weight 0, reads 0 here).  The sweeps and
 // residuals take the FLUID-row forms (mg_sweep_fluid_row: diagonal and weight
-// from a per-wavefront lane table, coupling terms without the code's selects,
-// non-FLUID cells written as the 0 they are without reading their
-// neighbours): the finest level's phases are VALU-bound (16 waves of a tile
-// share one CU's four SIMDs), and these forms take about half the
-// instructions of the general ones.
+// from a per-wavefront lane table, coupling terms without the code's selects),
+// half the instructions of the general ones: the finest level's phases are
+// VALU-bound (16 waves of a tile share one CU's four SIMDs).
+// For the same reason a thread keeps one column of the window through all
+// phases, P consecutive planes of it (FCols): its cells' place is decoded
+// once instead of in every phase, their own values, diagonals and weights and
+// the neighbours along z within its planes stay in registers, and every other
+// neighbour is at a constant distance in LDS.  With the window's cells dealt
+// to the threads anew in each phase a wavefront ran about three times the
+// instructions (MEASURED).
 //   descent:  x1 = w b (first sweep from zero), x2 = x1 + w (b - A x1) (kept
 //             for the ascent), r = b - A x2, coarse b = R r;
 //   ascent:   y = x2 + P xc, x' = y + w (b - A y), out = x' + w (b - A x'),
 //             with level 0's out = z and the partials of r.z.
 // Window of halo H around the fine tile: coordinates 0 .. T::fx + 2H - 1
 // stand for fine indices f0 - H ...
-// Two tile shapes: the finest level's work is throughput-bound and takes large
-// tiles (little halo per cell); the levels below are latency-bound (a 32^3
+// Two tile shapes (small_tiles): a level of many tiles is throughput-bound and
+// takes large ones (little halo per cell); the others are latency-bound (a 32^3
 // level has 16 large tiles for 256 CUs, and each workgroup's chain of LDS
 // phases sets the kernel's time), so they take small tiles: 2.5x fewer cells
 // per thread in every phase for more halo work in all.  A cell's value does
-// not depend on the tile it is computed in.  A finest level of few tiles is
-// such a level too (small_finest).
+// not depend on the tile it is computed in.
 // ---------------------------------------------------------------------------
 template <int RX, int RY, int RZ>
 struct FusedTile {
@@ -607,8 +605,8 @@ struct FusedTile {
     static constexpr int fx = 2 * RX, fy = 2 * RY, fz = 2 * RZ;  // fine tile
     static constexpr int coarse = RX * RY * RZ;
 };
-using TileFinest = FusedTile<8, 8, 4>;
-using TileCoarse = FusedTile<4, 4, 4>;
+using TileLarge = FusedTile<8, 8, 4>;
+using TileSmall = FusedTile<4, 4, 4>;
 template <class T, int H>
 struct FWin {
     static constexpr int x = T::fx + 2 * H, y = T::fy + 2 * H, z = T::fz + 2 * H;
@@ -619,6 +617,24 @@ template <class T>
 struct CWin {
     static constexpr int x = T::rx + 4, y = T::ry + 4, z = T::rz + 4;
     static constexpr int sy = x, sz = x * y, n = x * y * z;
+};
+
+// Columns of the window of halo H, lane-contiguous in LDS: thread g * cols + c
+// has planes [g P, (g + 1) P) of column c, P the least that kFusedThreads
+// threads cover the window with.  Arrays hold G * P planes.
+constexpr int kFusedThreads = 1024;  // 16 waves per tile
+template <class T, int H>
+struct FCols {
+    using W = FWin<T, H>;
+    static constexpr int cols = W::sz;
+    static constexpr int planes() {
+        int p = 1;
+        while (cols * ((W::z + p - 1) / p) > kFusedThreads) ++p;
+        return p;
+    }
+    static constexpr int P = planes(), G = (W::z + P - 1) / P;
+    static constexpr int threads = (cols * G + 63) / 64 * 64;
+    static constexpr int n = cols * G * P;
 };
 
 struct FusedArgs {
@@ -644,7 +660,6 @@ __device__ inline uint32_t fused_index(int i, int j, int k, const int n[3]) {
 // tfl (level 0 only): per tile, whether its fine tile holds a FLUID cell.  A
 // tile without one has every output 0 (its right-hand side and its coarse
 // cells' are 0), and those stay as the solve's start left them.
-constexpr int kFusedThreads = 1024;  // 16 waves per tile
 
 // sum_partials for a kFusedThreads workgroup: every workgroup adds the NV-wide
 // partials in the same fixed order (threads strided over the partials, lanes
@@ -668,13 +683,11 @@ __global__ __launch_bounds__(kFusedThreads) void k_mg_down(FusedArgs a, const fl
                                                     const uint16_t* __restrict__ ccode, float* __restrict__ cb,
                                                     const SolverScalars* st, const double* __restrict__ pconf,
                                                     int nconf, const uint8_t* __restrict__ tfl) {
-    using W3 = FWin<T, 3>;
-    using W2 = FWin<T, 2>;
-    using W1 = FWin<T, 1>;
-    __shared__ float sX1[W3::n];  // x1; later, over W1, the residual
-    __shared__ float sB[W2::n];
-    __shared__ uint16_t sC[W2::n];
-    __shared__ float sX2[W2::n];
+    using C = FCols<T, 3>;
+    using W = typename C::W;
+    constexpr int P = C::P;
+    __shared__ float sX1[C::n];  // x1; later the residual
+    __shared__ float sX2[C::n];
     const int done = st->done;  // read with the data, tested before the first write
     if (L0 && pconf) {
         // the V-cycle's first kernel: after a stop it returns; a relative stop
@@ -706,268 +719,258 @@ __global__ __launch_bounds__(kFusedThreads) void k_mg_down(FusedArgs a, const fl
     const int TX = (int)(t % tx0), TY = (int)((t % txy) / tx0), TZ = (int)(t / txy);
     const int I0 = TX * T::rx, J0 = TY * T::ry, K0 = TZ * T::rz;
     const int fx0 = 2 * I0, fy0 = 2 * J0, fz0 = 2 * K0;
-    // this thread's coarse cell (the restriction; the first T::coarse threads)
-    const int tx = threadIdx.x % T::rx, ty = (threadIdx.x / T::rx) % T::ry, tz = threadIdx.x / (T::rx * T::ry);
+    // this thread's coarse cell (the restriction: four lanes per cell, one per
+    // fine plane of its taps)
+    const int tq = threadIdx.x & 3, tc = threadIdx.x >> 2;
+    const int tx = tc % T::rx, ty = (tc / T::rx) % T::ry, tz = tc / (T::rx * T::ry);
     const int I = I0 + tx, J = J0 + ty, K = K0 + tz;
-    const bool cin = threadIdx.x < T::coarse && I < a.c[0] && J < a.c[1] && K < a.c[2];
+    const bool cin = tc < T::coarse && I < a.c[0] && J < a.c[1] && K < a.c[2];
     const uint32_t ci = fused_index(I, J, K, a.c);
-    // b and the row codes on the tile + 3: every load issued before any LDS
-    // store (the codes in whole registers, so no load waits for another)
-    constexpr int kPer = (W3::n + kFusedThreads - 1) / kFusedThreads;
-    float vb[kPer];
-    uint32_t vc[kPer];
+    // this thread's column of the tile + 3
+    const int g = threadIdx.x / C::cols, col = threadIdx.x - g * C::cols, z0 = g * P;
+    const int wx = col % W::x, wy = col / W::x;
+    const int i = fx0 - 3 + wx, j = fy0 - 3 + wy, k0 = fz0 - 3 + z0;
+    const bool mine = g < C::G;
+    const bool col_in = mine && i >= 0 && j >= 0 && i < a.n[0] && j < a.n[1];
+    const uint32_t slab = (uint32_t)a.n[0] * (uint32_t)a.n[1];
+    const uint32_t f0 = fused_index(i, j, k0, a.n);
+    const int e = col + W::sz * z0;
+    const int em = z0 > 0 ? e - W::sz : e;                                         // the plane below its planes
+    const int ep = e + W::sz * (g < C::G - 1 ? P : P - 1);                         // and the one above
+    const auto inner = [&](int h) { return mine && wx >= h && wx < W::x - h && wy >= h && wy < W::y - h; };
+    // b and the row codes: every load issued before any LDS store (the codes
+    // in whole registers, so no load waits for another)
+    float vb[P];
+    uint32_t vc[P];
 #pragma unroll
-    for (int u = 0; u < kPer; ++u) {
-        const int e = threadIdx.x + u * kFusedThreads;
+    for (int u = 0; u < P; ++u) {
         vb[u] = 0.0f;
         vc[u] = 0;
-        if (e < W3::n) {
-            const int wx = e % W3::x, wy = (e / W3::x) % W3::y, wz = e / W3::sz;
-            const int i = fx0 - 3 + wx, j = fy0 - 3 + wy, k = fz0 - 3 + wz;
-            if (fine_in(a, i, j, k)) {
-                const uint32_t f = fused_index(i, j, k, a.n);
-                vb[u] = b[f];
-                vc[u] = code[f];
-            }
+        if (col_in && (unsigned)(k0 + u) < (unsigned)a.n[2]) {
+            vb[u] = b[f0 + u * slab];
+            vc[u] = code[f0 + u * slab];
         }
     }
     const uint32_t ccd = cin ? (uint32_t)ccode[ci] : 0u;
     constexpr MgSmooth SM = L0 ? kMgFine : kMgCoarse;
     const CodeLanes lanes = code_lanes(a.ih2, SM.omega);
     const float nih2[3] = {-a.ih2[0], -a.ih2[1], -a.ih2[2]};
+    float cen[P], wgt[P], x[P];
+    uint32_t fluid = 0;
 #pragma unroll
-    for (int u = 0; u < kPer; ++u) {
-        const int e = threadIdx.x + u * kFusedThreads;
-        const float w = lanes_weight(vc[u], lanes, SM.omega);  // every lane: a cross-lane read
-        if (e < W3::n) {
-            sX1[e] = w * vb[u];  // the first sweep from zero
-            const int wx = e % W3::x, wy = (e / W3::x) % W3::y, wz = e / W3::sz;
-            if (wx >= 1 && wx < W3::x - 1 && wy >= 1 && wy < W3::y - 1 && wz >= 1 && wz < W3::z - 1) {
-                const int e2 = (wx - 1) + W2::sy * (wy - 1) + W2::sz * (wz - 1);
-                sB[e2] = vb[u];
-                sC[e2] = (uint16_t)vc[u];
-            }
-        }
+    for (int u = 0; u < P; ++u) {
+        const int li = code_lane(vc[u]);  // every lane: cross-lane reads
+        cen[u] = lane_read(lanes.cen, li);
+        wgt[u] = lane_read(lanes.wgt, li);
+        const bool fl = vc[u] & kFluidBit;
+        fluid |= fl ? 1u << u : 0u;
+        x[u] = (fl ? wgt[u] : SM.omega) * vb[u];  // the first sweep from zero
+        if (mine) sX1[e + W::sz * u] = x[u];
     }
     __syncthreads();
     if (done) return;  // uniform: the solve has stopped
-    // x2 on the tile + 2; the tile's own cells also go to global memory
-    for (int e0 = 0; e0 < W2::n; e0 += kFusedThreads) {
-        const int e = e0 + (int)threadIdx.x;
-        const bool on = e < W2::n;
-        const uint32_t cd = on ? sC[e] : 0u;
-        const int li = code_lane(cd);
-        const float cen = lane_read(lanes.cen, li), w = lane_read(lanes.wgt, li);
-        if (!on) continue;
-        const int wx = e % W2::x, wy = (e / W2::x) % W2::y, wz = e / W2::sz;
-        const int e3 = (wx + 1) + W3::sy * (wy + 1) + W3::sz * (wz + 1);
-        float x2 = 0.0f;
-        if (cd & kFluidBit) {
-            const float nb[6] = {sX1[e3 - 1],       sX1[e3 + 1],       sX1[e3 - W3::sy],
-                                 sX1[e3 + W3::sy], sX1[e3 - W3::sz], sX1[e3 + W3::sz]};
-            const float x1 = sX1[e3];
-            x2 = mg_cheb2(x1, 0.0f, SM.w21 * w, sB[e] - mg_apply_fluid_row(cen, x1, nb, nih2), SM.beta);
-        }
-        sX2[e] = x2;
-        if (wx >= 2 && wx < 2 + T::fx && wy >= 2 && wy < 2 + T::fy && wz >= 2 && wz < 2 + T::fz) {
-            const int i = fx0 + wx - 2, j = fy0 + wy - 2, k = fz0 + wz - 2;
-            if (fine_in(a, i, j, k)) x2out[fused_index(i, j, k, a.n)] = x2;
+    // x2 on the tile + 2; the tile's own cells also go to global memory.  The
+    // planes past the window's halo take values that nothing reads.
+    if (inner(1)) {
+        const bool tile_col = inner(3) && col_in;
+        float lo = sX1[em];
+        const float hi = sX1[ep];
+#pragma unroll
+        for (int u = 0; u < P; ++u) {
+            const float* q = sX1 + e + W::sz * u;
+            const float nb[6] = {q[-1], q[1], q[-W::x], q[W::x], lo, u < P - 1 ? x[u < P - 1 ? u + 1 : u] : hi};
+            lo = x[u];
+            const float x2 = mg_cheb2(x[u], 0.0f, SM.w21 * wgt[u], vb[u] - mg_apply_fluid_row(cen[u], x[u], nb, nih2),
+                                      SM.beta);
+            x[u] = (fluid >> u) & 1u ? x2 : 0.0f;
+            sX2[e + W::sz * u] = x[u];
+            if (tile_col && z0 + u >= 3 && z0 + u < 3 + T::fz && k0 + u < a.n[2]) x2out[f0 + u * slab] = x[u];
         }
     }
     __syncthreads();
     // r on the tile + 1 (into sX1, whose x1 is no longer read)
     float* sR = sX1;
-    for (int e0 = 0; e0 < W1::n; e0 += kFusedThreads) {
-        const int e = e0 + (int)threadIdx.x;
-        const bool on = e < W1::n;
-        const int wx = e % W1::x, wy = (e / W1::x) % W1::y, wz = e / W1::sz;
-        const int e2 = (wx + 1) + W2::sy * (wy + 1) + W2::sz * (wz + 1);
-        const uint32_t cd = on ? sC[e2] : 0u;
-        const float cen = lane_read(lanes.cen, code_lane(cd));
-        if (!on) continue;
-        float rv = 0.0f;
-        if (cd & kFluidBit) {
-            const float nb[6] = {sX2[e2 - 1],       sX2[e2 + 1],       sX2[e2 - W2::sy],
-                                 sX2[e2 + W2::sy], sX2[e2 - W2::sz], sX2[e2 + W2::sz]};
-            rv = sB[e2] - mg_apply_fluid_row(cen, sX2[e2], nb, nih2);
+    if (inner(2)) {
+        float lo = sX2[em];
+        const float hi = sX2[ep];
+#pragma unroll
+        for (int u = 0; u < P; ++u) {
+            const float* q = sX2 + e + W::sz * u;
+            const float nb[6] = {q[-1], q[1], q[-W::x], q[W::x], lo, u < P - 1 ? x[u < P - 1 ? u + 1 : u] : hi};
+            lo = x[u];
+            const float r = vb[u] - mg_apply_fluid_row(cen[u], x[u], nb, nih2);
+            sR[e + W::sz * u] = (fluid >> u) & 1u ? r : 0.0f;
         }
-        sR[e] = rv;
     }
     __syncthreads();
-    // coarse b = R r: fine index 2I-1+t sits at window coordinate 2*(I - I0) + t
-    if (!cin) return;
-    float v = 0.0f;
-    if (ccd & kFluidBit) {
+    // coarse b = R r: fine index 2I-1+t sits at window coordinate 2*(I - I0) + 2 + t
+    if (tc >= T::coarse) return;  // whole wavefronts
+    float acc = 0.0f;
+    if (cin && (ccd & kFluidBit)) {
         int ix[4], iy[4], iz[4];
-        float wx[4], wy[4], wz[4];
-        restrict_taps(I, a.n[0], a.c[0], ix, wx);
-        restrict_taps(J, a.n[1], a.c[1], iy, wy);
-        restrict_taps(K, a.n[2], a.c[2], iz, wz);
-        float acc = 0.0f;
+        float cx[4], cy[4], cz[4];
+        restrict_taps(I, a.n[0], a.c[0], ix, cx);
+        restrict_taps(J, a.n[1], a.c[1], iy, cy);
+        restrict_taps(K, a.n[2], a.c[2], iz, cz);
+        const float wk = tq < 2 ? (tq == 0 ? cz[0] : cz[1]) : (tq == 2 ? cz[2] : cz[3]);
+        const float* q = sR + (2 * tx + 2) + W::sy * (2 * ty + 2) + W::sz * (2 * tz + 2 + tq);
 #pragma unroll
-        for (int tk = 0; tk < 4; ++tk) {
+        for (int tj = 0; tj < 4; ++tj) {
+            const float wjk = cy[tj] * wk;
 #pragma unroll
-            for (int tj = 0; tj < 4; ++tj) {
-                const float wjk = wy[tj] * wz[tk];
-#pragma unroll
-                for (int ti = 0; ti < 4; ++ti)
-                    acc += (wx[ti] * wjk) * sR[(2 * tx + ti) + W1::sy * (2 * ty + tj) + W1::sz * (2 * tz + tk)];
-            }
+            for (int ti = 0; ti < 4; ++ti) acc += (cx[ti] * wjk) * q[ti + W::sy * tj];
         }
-        v = acc * 0.125f;
     }
-    cb[ci] = v;
+    acc += __shfl_xor(acc, 1, 4);
+    acc += __shfl_xor(acc, 2, 4);
+    if (cin && tq == 0) cb[ci] = acc * 0.125f;
 }
 
 // out = the level's corrected and post-smoothed solution.  With prz (level 0)
 // every launched workgroup leaves one partial of b . out (r.z).
 template <bool L0, class T>
-__global__ __launch_bounds__(kFusedThreads) void k_mg_up(FusedArgs a, const float* __restrict__ x2,
+__global__ __launch_bounds__((FCols<T, 2>::threads)) void k_mg_up(FusedArgs a, const float* __restrict__ x2,
                                                   const float* __restrict__ xc, const float* __restrict__ b,
                                                   const uint16_t* __restrict__ code, float* __restrict__ out,
                                                   double* __restrict__ prz, const SolverScalars* __restrict__ st,
                                                   const uint8_t* __restrict__ tfl) {
-    using W2 = FWin<T, 2>;
-    using W1 = FWin<T, 1>;
-    __shared__ float sY[W2::n];
-    __shared__ uint16_t sC[W2::n];
-    __shared__ float sB[W1::n];
-    __shared__ float sXp[W1::n];
-    __shared__ float sXc[CWin<T>::n];
+    using C = FCols<T, 2>;
+    using W = typename C::W;
+    using Wc = CWin<T>;
+    constexpr int P = C::P;
+    static_assert(P % 2 == 0, "a thread's planes start at an even fine index");
+    __shared__ float sY[C::n];
+    __shared__ float sXp[C::n];
+    __shared__ float sXc[Wc::n];
     const int done = st->done;  // read with the data, tested before the first write
     const uint32_t t = (uint32_t)fused_tile(a);
     const bool real = t < (uint32_t)(a.tiles[0] * a.tiles[1] * a.tiles[2]) && !(L0 && tfl && !tfl[t]);
-    int fx0 = 0, fy0 = 0, fz0 = 0, cx0 = 0, cy0 = 0, cz0 = 0;
+    const uint32_t tx0 = (uint32_t)a.tiles[0], txy = tx0 * (uint32_t)a.tiles[1];
+    const int TX = (int)(t % tx0), TY = (int)((t % txy) / tx0), TZ = (int)(t / txy);
+    const int fx0 = 2 * TX * T::rx, fy0 = 2 * TY * T::ry, fz0 = 2 * TZ * T::rz;
+    // this thread's column of the tile + 2
+    const int g = threadIdx.x / C::cols, col = threadIdx.x - g * C::cols, z0 = g * P;
+    const int wx = col % W::x, wy = col / W::x;
+    const int i = fx0 - 2 + wx, j = fy0 - 2 + wy, k0 = fz0 - 2 + z0;
+    const bool mine = g < C::G;
+    const bool col_in = mine && i >= 0 && j >= 0 && i < a.n[0] && j < a.n[1];
+    const uint32_t slab = (uint32_t)a.n[0] * (uint32_t)a.n[1];
+    const uint32_t f0 = fused_index(i, j, k0, a.n);
+    const int e = col + W::sz * z0;
+    const int em = z0 > 0 ? e - W::sz : e;                  // the plane below its planes
+    const int ep = e + W::sz * (g < C::G - 1 ? P : P - 1);  // and the one above
+    const auto inner = [&](int h) { return mine && wx >= h && wx < W::x - h && wy >= h && wy < W::y - h; };
+    float y[P], vb[P];
+    uint32_t vc[P];
     if (real) {
-        const uint32_t tx0 = (uint32_t)a.tiles[0], txy = tx0 * (uint32_t)a.tiles[1];
-        const int TX = (int)(t % tx0), TY = (int)((t % txy) / tx0), TZ = (int)(t / txy);
-        fx0 = 2 * TX * T::rx;
-        fy0 = 2 * TY * T::ry;
-        fz0 = 2 * TZ * T::rz;
-        cx0 = TX * T::rx - 2;
-        cy0 = TY * T::ry - 2;
-        cz0 = TZ * T::rz - 2;
-        // x2 and the row codes on the tile + 2, b on the tile + 1, the coarse
-        // correction on its window: every load issued before any LDS store
-        // (the codes in whole registers, so no load waits for another)
-        constexpr int kP2 = (W2::n + kFusedThreads - 1) / kFusedThreads;
-        constexpr int kPc = (CWin<T>::n + kFusedThreads - 1) / kFusedThreads;
-        float vx[kP2], vb[kP2];
-        uint32_t vc[kP2];
-        float vxc[kPc];
+        // x2, b and the row codes of the column and the coarse correction on
+        // its window (clamped into the grid, as the prolongation clamps): every
+        // load issued before any LDS store (the codes in whole registers, so no
+        // load waits for another)
 #pragma unroll
-        for (int u = 0; u < kP2; ++u) {
-            const int e = threadIdx.x + u * kFusedThreads;
-            vx[u] = vb[u] = 0.0f;
+        for (int u = 0; u < P; ++u) {
+            y[u] = vb[u] = 0.0f;
             vc[u] = 0;
-            if (e < W2::n) {
-                const int wx = e % W2::x, wy = (e / W2::x) % W2::y, wz = e / W2::sz;
-                const int i = fx0 - 2 + wx, j = fy0 - 2 + wy, k = fz0 - 2 + wz;
-                if (fine_in(a, i, j, k)) {
-                    const uint32_t f = fused_index(i, j, k, a.n);
-                    vx[u] = x2[f];
-                    vc[u] = code[f];
-                    const bool w1 = wx >= 1 && wx < W2::x - 1 && wy >= 1 && wy < W2::y - 1 && wz >= 1 && wz < W2::z - 1;
-                    if (w1) vb[u] = b[f];
-                }
+            if (col_in && (unsigned)(k0 + u) < (unsigned)a.n[2]) {
+                y[u] = x2[f0 + u * slab];
+                vb[u] = b[f0 + u * slab];
+                vc[u] = code[f0 + u * slab];
             }
         }
+        constexpr int kPc = (Wc::n + C::threads - 1) / C::threads;
+        float vxc[kPc];
 #pragma unroll
         for (int u = 0; u < kPc; ++u) {
-            const int e = threadIdx.x + u * kFusedThreads;
+            const int q = threadIdx.x + u * C::threads;
             vxc[u] = 0.0f;
-            if (e < CWin<T>::n) {
-                const int wx = e % CWin<T>::x, wy = (e / CWin<T>::x) % CWin<T>::y, wz = e / CWin<T>::sz;
-                const int I = min(max(cx0 + wx, 0), a.c[0] - 1), J = min(max(cy0 + wy, 0), a.c[1] - 1),
-                          K = min(max(cz0 + wz, 0), a.c[2] - 1);
+            if (q < Wc::n) {
+                const int qx = q % Wc::x, qy = (q / Wc::x) % Wc::y, qz = q / Wc::sz;
+                const int I = min(max(fx0 / 2 - 2 + qx, 0), a.c[0] - 1), J = min(max(fy0 / 2 - 2 + qy, 0), a.c[1] - 1),
+                          K = min(max(fz0 / 2 - 2 + qz, 0), a.c[2] - 1);
                 vxc[u] = xc[fused_index(I, J, K, a.c)];
             }
         }
 #pragma unroll
-        for (int u = 0; u < kP2; ++u) {
-            const int e = threadIdx.x + u * kFusedThreads;
-            if (e < W2::n) {
-                sY[e] = vx[u];
-                sC[e] = (uint16_t)vc[u];
-                const int wx = e % W2::x, wy = (e / W2::x) % W2::y, wz = e / W2::sz;
-                if (wx >= 1 && wx < W2::x - 1 && wy >= 1 && wy < W2::y - 1 && wz >= 1 && wz < W2::z - 1)
-                    sB[(wx - 1) + W1::sy * (wy - 1) + W1::sz * (wz - 1)] = vb[u];
-            }
-        }
-#pragma unroll
         for (int u = 0; u < kPc; ++u) {
-            const int e = threadIdx.x + u * kFusedThreads;
-            if (e < CWin<T>::n) sXc[e] = vxc[u];
+            const int q = threadIdx.x + u * C::threads;
+            if (q < Wc::n) sXc[q] = vxc[u];
         }
     }
     constexpr MgSmooth SM = L0 ? kMgFine : kMgCoarse;
     const CodeLanes lanes = code_lanes(a.ih2, SM.omega);
     const float nih2[3] = {-a.ih2[0], -a.ih2[1], -a.ih2[2]};
+    float cen[P], wgt[P];
+    uint32_t fluid = 0;
+    if (real) {  // the whole workgroup: cross-lane reads
+#pragma unroll
+        for (int u = 0; u < P; ++u) {
+            const int li = code_lane(vc[u]);
+            cen[u] = lane_read(lanes.cen, li);
+            wgt[u] = lane_read(lanes.wgt, li);
+            fluid |= vc[u] & kFluidBit ? 1u << u : 0u;
+        }
+    }
     __syncthreads();
     if (done) return;  // uniform: the solve has stopped
     double v[1] = {0.0};
-    if (real) {
-        // y = x2 + P xc on FLUID cells (each from its own x2: in place)
-        for (int e = threadIdx.x; e < W2::n; e += kFusedThreads) {
-            if (!(sC[e] & kFluidBit)) continue;
-            const int wx = e % W2::x, wy = (e / W2::x) % W2::y, wz = e / W2::sz;
-            const float add = prolong_at3(fx0 - 2 + wx, fy0 - 2 + wy, fz0 - 2 + wz, a.c[0], a.c[1], a.c[2],
-                                          [&](int I, int J, int K) {
-                                              return sXc[(I - cx0) + CWin<T>::sy * (J - cy0) + CWin<T>::sz * (K - cz0)];
-                                          });
-            sY[e] = sY[e] + add;
+    if (real && mine) {
+        // y = x2 + P xc on FLUID cells: prolong_at3's terms, the window's
+        // coarse index (fine index >> 1) - (tile's first - 2); the bilinear
+        // part of a coarse plane serves the two to four fine planes it feeds
+        const int ia = (wx >> 1) + (wx & 1), ja = (wy >> 1) + (wy & 1);  // the lower neighbour of each axis
+        const float wia = wx & 1 ? 0.75f : 0.25f, wja = wy & 1 ? 0.75f : 0.25f;
+        const float wib = 1.0f - wia, wjb = 1.0f - wja;
+        const float* q = sXc + ia + Wc::sy * ja + Wc::sz * (z0 >> 1);
+        float S[P / 2 + 2];
+#pragma unroll
+        for (int m = 0; m < P / 2 + 2; ++m) {
+            const float* r = q + Wc::sz * m;
+            S[m] = wja * (wia * r[0] + wib * r[1]) + wjb * (wia * r[Wc::sy] + wib * r[Wc::sy + 1]);
+        }
+#pragma unroll
+        for (int u = 0; u < P; ++u) {
+            const float add = u & 1 ? 0.75f * S[u / 2 + 1] + 0.25f * S[u / 2 + 2] : 0.25f * S[u / 2] + 0.75f * S[u / 2 + 1];
+            y[u] = (fluid >> u) & 1u ? y[u] + add : y[u];
+            sY[e + W::sz * u] = y[u];
         }
     }
     __syncthreads();
-    if (real) {
-        // x' on the tile + 1
-        for (int e0 = 0; e0 < W1::n; e0 += kFusedThreads) {
-            const int e = e0 + (int)threadIdx.x;
-            const bool on = e < W1::n;
-            const int wx = e % W1::x, wy = (e / W1::x) % W1::y, wz = e / W1::sz;
-            const int e2 = (wx + 1) + W2::sy * (wy + 1) + W2::sz * (wz + 1);
-            const uint32_t cd = on ? sC[e2] : 0u;
-            const int li = code_lane(cd);
-            const float cen = lane_read(lanes.cen, li), w = lane_read(lanes.wgt, li);
-            if (!on) continue;
-            float xp = 0.0f;
-            if (cd & kFluidBit) {
-                const float nb[6] = {sY[e2 - 1],       sY[e2 + 1],       sY[e2 - W2::sy],
-                                     sY[e2 + W2::sy], sY[e2 - W2::sz], sY[e2 + W2::sz]};
-                xp = mg_sweep_fluid_row(cen, w, sY[e2], sB[e], nb, nih2);
-            }
-            sXp[e] = xp;
+    float xp[P];
+    if (real && inner(1)) {
+        // x' on the tile + 1 (the planes past it take values that nothing reads)
+        float lo = sY[em];
+        const float hi = sY[ep];
+#pragma unroll
+        for (int u = 0; u < P; ++u) {
+            const float* q = sY + e + W::sz * u;
+            const float nb[6] = {q[-1], q[1], q[-W::x], q[W::x], lo, u < P - 1 ? y[u < P - 1 ? u + 1 : u] : hi};
+            lo = y[u];
+            const float x1 = mg_sweep_fluid_row(cen[u], wgt[u], y[u], vb[u], nb, nih2);
+            xp[u] = (fluid >> u) & 1u ? x1 : 0.0f;
+            sXp[e + W::sz * u] = xp[u];
         }
     }
     __syncthreads();
-    if (real) {
+    if (real && inner(2) && col_in) {
         // out on the tile
-        constexpr int kTile = T::fx * T::fy * T::fz;
-        for (int e0 = 0; e0 < kTile; e0 += kFusedThreads) {
-            const int e = e0 + (int)threadIdx.x;
-            const bool on = e < kTile;
-            const int wx = e % T::fx, wy = (e / T::fx) % T::fy, wz = e / (T::fx * T::fy);
-            const int i = fx0 + wx, j = fy0 + wy, k = fz0 + wz;
-            const int e1 = (wx + 1) + W1::sy * (wy + 1) + W1::sz * (wz + 1);
-            const int e2 = (wx + 2) + W2::sy * (wy + 2) + W2::sz * (wz + 2);
-            const uint32_t cd = on ? sC[e2] : 0u;
-            const int li = code_lane(cd);
-            const float cen = lane_read(lanes.cen, li), w = lane_read(lanes.wgt, li);
-            if (!on || !fine_in(a, i, j, k)) continue;
+        float lo = sXp[em];
+        const float hi = sXp[ep];
+#pragma unroll
+        for (int u = 0; u < P; ++u) {
+            const float* q = sXp + e + W::sz * u;
+            const float nb[6] = {q[-1], q[1], q[-W::x], q[W::x], lo, u < P - 1 ? xp[u < P - 1 ? u + 1 : u] : hi};
+            lo = xp[u];
+            if (z0 + u < 2 || z0 + u >= 2 + T::fz || k0 + u >= a.n[2]) continue;
             float o = 0.0f;
-            if (cd & kFluidBit) {
-                const float nb[6] = {sXp[e1 - 1],       sXp[e1 + 1],       sXp[e1 - W1::sy],
-                                     sXp[e1 + W1::sy], sXp[e1 - W1::sz], sXp[e1 + W1::sz]};
-                const float bc = sB[e1];
-                const float x1 = sXp[e1];
-                o = mg_cheb2(x1, sY[e2], SM.w21 * w, bc - mg_apply_fluid_row(cen, x1, nb, nih2), SM.beta);
-                if (L0) v[0] += (double)bc * (double)o;
+            if ((fluid >> u) & 1u) {
+                o = mg_cheb2(xp[u], y[u], SM.w21 * wgt[u], vb[u] - mg_apply_fluid_row(cen[u], xp[u], nb, nih2), SM.beta);
+                if (L0) v[0] += (double)vb[u] * (double)o;
             }
-            out[fused_index(i, j, k, a.n)] = o;
+            out[f0 + u * slab] = o;
         }
     }
     if (L0 && prz) {  // one partial per workgroup
-        __shared__ double sm[1][kFusedThreads / 64];
+        __shared__ double sm[1][C::threads / 64];
         wave_sums(v, sm);
         __syncthreads();
         if (threadIdx.x == 0) prz[blockIdx.x] = waves_total(sm[0]);
@@ -1444,20 +1447,20 @@ static FusedArgs fused_args(const MGLevel& l, const MGLevel& c) {
     return a;
 }
 
-// Whether the finest level takes the small tiles: up to two of them per CU.
-// There the level's kernels are bound by the latency of a workgroup's chain of
-// phases, and a small tile has 2.5x fewer cells per thread in each; above, by
+// Whether a level takes the small tiles: up to 1.5 of them per CU.  There the
+// level's kernels are bound by the latency of a workgroup's chain of phases,
+// and a small tile has 2.5x fewer cells per thread in each; above, by
 // throughput, and the small tiles' halos cost more than they save.  Measured
-// on whole solves to 1e-10 (large tiles / small): 32^3 0.61 / 0.52 ms, 48^3
-// 0.74 / 0.65, 64^3 (512 tiles) 0.875 / 0.838, 80x64x72 (720) 1.01 / 1.05,
-// 96^3 1.24 / 1.39, 128^3 1.74 / 2.11.
-static bool small_finest(const MGLevel& l) {
+// on whole solves to 1e-10, finest level on large tiles / small: 32^3 0.473 /
+// 0.423 ms, 48^3 (216 small tiles) 0.549 / 0.500, 56^3 (343) 0.573 / 0.571,
+// 64^3 (512) 0.680 / 0.695, 96^3 0.99 / 1.18, 128^3 1.51 / 1.90.
+static bool small_tiles(const MGLevel& l) {
     constexpr int64_t kCus = 256;
-    return l.cells <= 2 * kCus * TileCoarse::coarse * 8;
+    return 2 * l.cells <= 3 * kCus * TileSmall::coarse * 8;
 }
 
-static FusedArgs finest_args(const MGLevel& l, const MGLevel& c) {
-    return small_finest(l) ? fused_args<TileCoarse>(l, c) : fused_args<TileFinest>(l, c);
+static FusedArgs level_args(const MGLevel& l, const MGLevel& c) {
+    return small_tiles(l) ? fused_args<TileSmall>(l, c) : fused_args<TileLarge>(l, c);
 }
 
 void mg_free(fe_scene* s);
@@ -1512,7 +1515,7 @@ static hipError_t mg_alloc(fe_scene* s) {
         if ((e = hipMalloc((void**)&l.r, n * sizeof(float))) != hipSuccess) break;
     }
     // the fused V-cycle's level-0 tile flags and r.z partials
-    const FusedArgs fa = finest_args(lv[0], lv[1]);
+    const FusedArgs fa = level_args(lv[0], lv[1]);
     s->mg_npz = fa.padded;
     if (e == hipSuccess) e = hipMalloc((void**)&s->mg_tfl, (size_t)fa.padded);
     if (e == hipSuccess) e = hipMalloc((void**)&s->mg_pz, sizeof(double) * (size_t)fa.padded);
@@ -1560,13 +1563,13 @@ hipError_t mg_setup(fe_scene* s) {
         pa.flags[q] = lv[q].flags;
     }
     if (s->tune.mg == FE_MG_FUSED) {
-        const FusedArgs fa = finest_args(lv[0], lv[1]);
+        const FusedArgs fa = level_args(lv[0], lv[1]);
         pa.tfl = s->mg_tfl;
         for (int a = 0; a < 3; ++a) pa.tiles[a] = fa.tiles[a];
-        const bool small = small_finest(lv[0]);
-        pa.rx = small ? TileCoarse::rx : TileFinest::rx;
-        pa.ry = small ? TileCoarse::ry : TileFinest::ry;
-        pa.rz = small ? TileCoarse::rz : TileFinest::rz;
+        const bool small = small_tiles(lv[0]);
+        pa.rx = small ? TileSmall::rx : TileLarge::rx;
+        pa.ry = small ? TileSmall::ry : TileLarge::ry;
+        pa.rz = small ? TileSmall::rz : TileLarge::rz;
     }
     const unsigned nb = (unsigned)(((lv[1].n[0] + 7) / 8) * ((lv[1].n[1] + 7) / 8) * ((lv[1].n[2] + 7) / 8));
     hipLaunchKernelGGL(k_mg_pyramid, dim3(nb), dim3(kPyrThreads), 0, s->stream, pa);
@@ -1649,57 +1652,55 @@ static hipError_t mg_apply_fused(fe_scene* s, const float* r, float* z, SolverSc
     std::vector<MGLevel>& lv = s->mg;
     const int T = s->mg_tail;
     lv[0].b = const_cast<float*>(r);
-    const bool small = small_finest(lv[0]);
-    auto down = [&](auto kernel, int q, const FusedArgs& a) {
+    auto down = [&](int q) {
         const MGLevel& l = lv[q];
         const MGLevel& c = lv[q + 1];
+        const FusedArgs a = level_args(l, c);
+        const bool sm = small_tiles(l);
         const dim3 grid((unsigned)a.padded);
         if (q == 0)
-            launch_timed(s, FE_KERNEL_MG_DOWN, tag, kernel, grid, dim3(kFusedThreads), a, (const float*)l.b,
-                         (const uint16_t*)l.code, l.x2, (const uint16_t*)c.code, c.b, (const SolverScalars*)st, pconf,
-                         nparts, (const uint8_t*)s->mg_tfl);
-        else
-            hipLaunchKernelGGL(kernel, grid, dim3(kFusedThreads), 0, s->stream, a, (const float*)l.b,
-                               (const uint16_t*)l.code, l.x2, (const uint16_t*)c.code, c.b, (const SolverScalars*)st,
-                               (const double*)nullptr, 0, (const uint8_t*)nullptr);
-    };
-    auto up = [&](auto kernel, int q, const FusedArgs& a) {
-        const MGLevel& l = lv[q];
-        const MGLevel& c = lv[q + 1];
-        const dim3 grid((unsigned)a.padded);
-        const float* xc = q + 1 == T ? c.x2 : c.x;
-        if (q == 0)
-            launch_timed(s, FE_KERNEL_MG_UP, tag, kernel, grid, dim3(kFusedThreads), a, (const float*)l.x2, xc,
-                         (const float*)l.b, (const uint16_t*)l.code, z, prz, (const SolverScalars*)st,
+            launch_timed(s, FE_KERNEL_MG_DOWN, tag, sm ? k_mg_down<true, TileSmall> : k_mg_down<true, TileLarge>, grid,
+                         dim3(kFusedThreads), a, (const float*)l.b, (const uint16_t*)l.code, l.x2,
+                         (const uint16_t*)c.code, c.b, (const SolverScalars*)st, pconf, nparts,
                          (const uint8_t*)s->mg_tfl);
         else
-            hipLaunchKernelGGL(kernel, grid, dim3(kFusedThreads), 0, s->stream, a, (const float*)l.x2, xc,
-                               (const float*)l.b, (const uint16_t*)l.code, l.x, (double*)nullptr,
-                               (const SolverScalars*)st, (const uint8_t*)nullptr);
+            hipLaunchKernelGGL((sm ? k_mg_down<false, TileSmall> : k_mg_down<false, TileLarge>), grid,
+                               dim3(kFusedThreads), 0, s->stream, a, (const float*)l.b, (const uint16_t*)l.code, l.x2,
+                               (const uint16_t*)c.code, c.b, (const SolverScalars*)st, (const double*)nullptr, 0,
+                               (const uint8_t*)nullptr);
     };
-    const FusedArgs a0 = finest_args(lv[0], lv[1]);
-    if (small)
-        down(k_mg_down<true, TileCoarse>, 0, a0);
-    else
-        down(k_mg_down<true, TileFinest>, 0, a0);
+    auto up = [&](int q) {
+        const MGLevel& l = lv[q];
+        const MGLevel& c = lv[q + 1];
+        const FusedArgs a = level_args(l, c);
+        const bool sm = small_tiles(l);
+        const dim3 grid((unsigned)a.padded);
+        const dim3 threads((unsigned)(sm ? FCols<TileSmall, 2>::threads : FCols<TileLarge, 2>::threads));
+        const float* xc = q + 1 == T ? c.x2 : c.x;
+        if (q == 0)
+            launch_timed(s, FE_KERNEL_MG_UP, tag, sm ? k_mg_up<true, TileSmall> : k_mg_up<true, TileLarge>, grid,
+                         threads, a, (const float*)l.x2, xc, (const float*)l.b, (const uint16_t*)l.code, z, prz,
+                         (const SolverScalars*)st, (const uint8_t*)s->mg_tfl);
+        else
+            hipLaunchKernelGGL((sm ? k_mg_up<false, TileSmall> : k_mg_up<false, TileLarge>), grid, threads, 0,
+                               s->stream, a, (const float*)l.x2, xc, (const float*)l.b, (const uint16_t*)l.code, l.x,
+                               (double*)nullptr, (const SolverScalars*)st, (const uint8_t*)nullptr);
+    };
+    down(0);
     // the last level above the coarsest goes with it into one workgroup, where
     // their iterates fit its LDS (all but very long grids)
     BottomArgs ba{};
     const bool bottom = T >= 2 && T + 1 == (int)lv.size() &&
                         2 * ((ba = bottom_args(lv[T - 1], lv[T])).pf + ba.pc) <= kBotLds;
     const int B = bottom ? T - 1 : T;
-    for (int q = 1; q < B; ++q) down(k_mg_down<false, TileCoarse>, q, fused_args<TileCoarse>(lv[q], lv[q + 1]));
+    for (int q = 1; q < B; ++q) down(q);
     if (bottom)
         hipLaunchKernelGGL(k_mg_bottom, dim3(1), dim3(kBotThreads), sizeof(float) * (2 * (ba.pf + ba.pc) + 3), s->stream, ba,
                            (const float*)lv[B].b, (const uint16_t*)lv[B].code, (const uint16_t*)lv[T].code, lv[B].x,
                            (const SolverScalars*)st);
     else
         launch_tail(s, st);
-    for (int q = B - 1; q > 0; --q) up(k_mg_up<false, TileCoarse>, q, fused_args<TileCoarse>(lv[q], lv[q + 1]));
-    if (small)
-        up(k_mg_up<true, TileCoarse>, 0, a0);
-    else
-        up(k_mg_up<true, TileFinest>, 0, a0);
+    for (int q = B - 1; q >= 0; --q) up(q);
     return hipGetLastError();
 }
 
