@@ -261,6 +261,15 @@ __device__ inline void restrict_taps(int I, int nf, int nc, int (&idx)[4], float
     }
 }
 
+// One x row of a coarse cell's window; R(t) is the residual at tap t.
+template <typename F>
+__device__ inline float restrict_row(const float (&w)[4], F R) {
+    float s = 0.0f;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) s += w[t] * R(t);
+    return s;
+}
+
 // (1/8) sum of the 4x4x4 fine window, 64 independent loads.
 template <typename F>
 __device__ inline float restrict_sum(int I, int J, int K, int fx, int fy, int fz, int cx, int cy, int cz, F R) {
@@ -274,10 +283,8 @@ __device__ inline float restrict_sum(int I, int J, int K, int fx, int fy, int fz
     for (int tk = 0; tk < 4; ++tk) {
 #pragma unroll
         for (int tj = 0; tj < 4; ++tj) {
-            const float wjk = wy[tj] * wz[tk];
             const int64_t row = (int64_t)fx * ((int64_t)iy[tj] + (int64_t)fy * iz[tk]);
-#pragma unroll
-            for (int ti = 0; ti < 4; ++ti) acc += (wx[ti] * wjk) * R(row + ix[ti]);
+            acc += (wy[tj] * wz[tk]) * restrict_row(wx, [&](int ti) { return R(row + ix[ti]); });
         }
     }
     return acc * 0.125f;
@@ -534,9 +541,8 @@ __global__ __launch_bounds__(kBlock) void k_mg_restrict(const float* __restrict_
         for (int tk = 0; tk < 4; ++tk) {
 #pragma unroll
             for (int tj = 0; tj < 4; ++tj) {
-                const float wjk = wy[tj] * wz[tk];
-#pragma unroll
-                for (int ti = 0; ti < 4; ++ti) acc += (wx[ti] * wjk) * win[2 * tz + tk][2 * ty + tj][2 * tx + ti];
+                acc += (wy[tj] * wz[tk]) *
+                       restrict_row(wx, [&](int ti) { return win[2 * tz + tk][2 * ty + tj][2 * tx + ti]; });
             }
         }
         v = acc * 0.125f;
@@ -816,9 +822,7 @@ __global__ __launch_bounds__(kFusedThreads) void k_mg_down(FusedArgs a, const fl
         const float* q = sR + (2 * tx + 2) + W::sy * (2 * ty + 2) + W::sz * (2 * tz + 2 + tq);
 #pragma unroll
         for (int tj = 0; tj < 4; ++tj) {
-            const float wjk = cy[tj] * wk;
-#pragma unroll
-            for (int ti = 0; ti < 4; ++ti) acc += (cx[ti] * wjk) * q[ti + W::sy * tj];
+            acc += (cy[tj] * wk) * restrict_row(cx, [&](int ti) { return q[ti + W::sy * tj]; });
         }
     }
     acc += __shfl_xor(acc, 1, 4);
@@ -1242,14 +1246,15 @@ struct BottomArgs {
 // 4096 * 2^-22 / n.
 __device__ inline void small_cell_ijk(int c, int nx, int ny, float rx, float ry, int& i, int& j, int& k) {
     const int q = (int)(((float)c + 0.5f) * rx);
-    i = c - q * nx;
+    i = c - __mul24(q, nx);
     k = (int)(((float)q + 0.5f) * ry);
-    j = q - k * ny;
+    j = q - __mul24(k, ny);
 }
 
-// Offset of cell (i, j, k) in an array of dims n with a border of one.
+// Offset of cell (i, j, k) in an array of dims n with a border of one (24-bit
+// products: a 32-bit one takes four times the issue time).
 __device__ inline int bordered(int i, int j, int k, const int n[3]) {
-    return (i + 1) + (n[0] + 2) * ((j + 1) + (n[1] + 2) * (k + 1));
+    return (i + 1) + __mul24(n[0] + 2, (j + 1) + __mul24(n[1] + 2, k + 1));
 }
 
 __device__ inline void bordered_neighbours(const float* x, int p, int sy, int sz, float (&nb)[6]) {
@@ -1291,7 +1296,7 @@ __global__ __launch_bounds__(kBotThreads) void k_mg_bottom(BottomArgs a, const f
     const int sy = a.n[0] + 2, sz = sy * (a.n[1] + 2), csy = a.c[0] + 2, csz = csy * (a.c[1] + 2);
     float cen[kBotPer], wgt[kBotPer];
     int p[kBotPer];
-    const float rx = 1.0f / (float)a.n[0], ry = 1.0f / (float)a.n[1];
+    const float rx = __builtin_amdgcn_rcpf((float)a.n[0]), ry = __builtin_amdgcn_rcpf((float)a.n[1]);
 #pragma unroll
     for (int u = 0; u < kBotPer; ++u) {
         const int li = code_lane(cd[u]);
@@ -1304,7 +1309,8 @@ __global__ __launch_bounds__(kBotThreads) void k_mg_bottom(BottomArgs a, const f
     const int cli = code_lane(ccd);
     const float ccen = lane_read(cl.cen, cli), cw = lane_read(cl.wgt, cli);
     int I, J, K;
-    small_cell_ijk(threadIdx.x, a.c[0], a.c[1], 1.0f / (float)a.c[0], 1.0f / (float)a.c[1], I, J, K);
+    small_cell_ijk(threadIdx.x, a.c[0], a.c[1], __builtin_amdgcn_rcpf((float)a.c[0]),
+                   __builtin_amdgcn_rcpf((float)a.c[1]), I, J, K);
     const int cp = bordered(I, J, K, a.c);
     const bool cfl = (ccd & kFluidBit) != 0;  // false where there is no cell
     __syncthreads();
@@ -1343,19 +1349,23 @@ __global__ __launch_bounds__(kBotThreads) void k_mg_bottom(BottomArgs a, const f
     float rho = 1.0f / sigma;
     float bc = 0.0f, d = 0.0f, xc = 0.0f;
     if (cfl) {
+        // the taps 2I-1 .. 2I+2 per axis at constant distances; where the last
+        // lies beyond the border (odd dims) it has weight 0 and takes the one before
         int ix[4], iy[4], iz[4];
         float wx[4], wy[4], wz[4];
         restrict_taps(I, a.n[0], a.c[0], ix, wx);
         restrict_taps(J, a.n[1], a.c[1], iy, wy);
         restrict_taps(K, a.n[2], a.c[2], iz, wz);
+        const float* row = X + bordered(2 * I - 1, 2 * J - 1, 2 * K - 1, a.n);
+        const int lx = 2 * I + 2 > a.n[0] ? 2 : 3, ly = sy * (2 * J + 2 > a.n[1] ? 2 : 3),
+                  lz = sz * (2 * K + 2 > a.n[2] ? 2 : 3);
         float acc = 0.0f;
 #pragma unroll
         for (int tk = 0; tk < 4; ++tk) {
 #pragma unroll
             for (int tj = 0; tj < 4; ++tj) {
-                const float wjk = wy[tj] * wz[tk];
-#pragma unroll
-                for (int ti = 0; ti < 4; ++ti) acc += (wx[ti] * wjk) * X[bordered(ix[ti], iy[tj], iz[tk], a.n)];
+                const float* q = row + (tk < 3 ? tk * sz : lz) + (tj < 3 ? tj * sy : ly);
+                acc += (wy[tj] * wz[tk]) * restrict_row(wx, [&](int ti) { return q[ti < 3 ? ti : lx]; });
             }
         }
         bc = acc * 0.125f;
@@ -1384,10 +1394,18 @@ __global__ __launch_bounds__(kBotThreads) void k_mg_bottom(BottomArgs a, const f
 #pragma unroll
     for (int u = 0; u < kBotPer; ++u) {
         if (!(cd[u] & kFluidBit)) continue;
+        // prolong_at3's terms from its lowest neighbour, the others one step on
+        // (none where the axis clamps both to one cell)
         int i, j, k;
         small_cell_ijk(threadIdx.x + u * kBotThreads, a.n[0], a.n[1], rx, ry, i, j, k);
-        x2[u] = x2[u] + prolong_at3(i, j, k, a.c[0], a.c[1], a.c[2],
-                                    [&](int A, int B, int C) { return V[bordered(A, B, C, a.c)]; });
+        const int A = (i - 1) >> 1, B = (j - 1) >> 1, C = (k - 1) >> 1;
+        const float wa = i & 1 ? 0.75f : 0.25f, wb = j & 1 ? 0.75f : 0.25f, wc = k & 1 ? 0.75f : 0.25f;
+        const float wa1 = 1.0f - wa, wb1 = 1.0f - wb, wc1 = 1.0f - wc;
+        const float* q = V + bordered(max(A, 0), max(B, 0), max(C, 0), a.c);
+        const int dx = A >= 0 && A + 1 < a.c[0] ? 1 : 0, dy = B >= 0 && B + 1 < a.c[1] ? csy : 0,
+                  dz = C >= 0 && C + 1 < a.c[2] ? csz : 0;
+        x2[u] = x2[u] + (wc * (wb * (wa * q[0] + wa1 * q[dx]) + wb1 * (wa * q[dy] + wa1 * q[dy + dx])) +
+                         wc1 * (wb * (wa * q[dz] + wa1 * q[dz + dx]) + wb1 * (wa * q[dz + dy] + wa1 * q[dz + dy + dx])));
         Y[p[u]] = x2[u];
     }
     __syncthreads();
@@ -1459,7 +1477,7 @@ static bool small_tiles(const MGLevel& l) {
     return 2 * l.cells <= 3 * kCus * TileSmall::coarse * 8;
 }
 
-static FusedArgs level_args(const MGLevel& l, const MGLevel& c) {
+static FusedArgs tile_args(const MGLevel& l, const MGLevel& c) {
     return small_tiles(l) ? fused_args<TileSmall>(l, c) : fused_args<TileLarge>(l, c);
 }
 
@@ -1515,7 +1533,7 @@ static hipError_t mg_alloc(fe_scene* s) {
         if ((e = hipMalloc((void**)&l.r, n * sizeof(float))) != hipSuccess) break;
     }
     // the fused V-cycle's level-0 tile flags and r.z partials
-    const FusedArgs fa = level_args(lv[0], lv[1]);
+    const FusedArgs fa = tile_args(lv[0], lv[1]);
     s->mg_npz = fa.padded;
     if (e == hipSuccess) e = hipMalloc((void**)&s->mg_tfl, (size_t)fa.padded);
     if (e == hipSuccess) e = hipMalloc((void**)&s->mg_pz, sizeof(double) * (size_t)fa.padded);
@@ -1563,7 +1581,7 @@ hipError_t mg_setup(fe_scene* s) {
         pa.flags[q] = lv[q].flags;
     }
     if (s->tune.mg == FE_MG_FUSED) {
-        const FusedArgs fa = level_args(lv[0], lv[1]);
+        const FusedArgs fa = tile_args(lv[0], lv[1]);
         pa.tfl = s->mg_tfl;
         for (int a = 0; a < 3; ++a) pa.tiles[a] = fa.tiles[a];
         const bool small = small_tiles(lv[0]);
@@ -1655,7 +1673,7 @@ static hipError_t mg_apply_fused(fe_scene* s, const float* r, float* z, SolverSc
     auto down = [&](int q) {
         const MGLevel& l = lv[q];
         const MGLevel& c = lv[q + 1];
-        const FusedArgs a = level_args(l, c);
+        const FusedArgs a = tile_args(l, c);
         const bool sm = small_tiles(l);
         const dim3 grid((unsigned)a.padded);
         if (q == 0)
@@ -1672,7 +1690,7 @@ static hipError_t mg_apply_fused(fe_scene* s, const float* r, float* z, SolverSc
     auto up = [&](int q) {
         const MGLevel& l = lv[q];
         const MGLevel& c = lv[q + 1];
-        const FusedArgs a = level_args(l, c);
+        const FusedArgs a = tile_args(l, c);
         const bool sm = small_tiles(l);
         const dim3 grid((unsigned)a.padded);
         const dim3 threads((unsigned)(sm ? FCols<TileSmall, 2>::threads : FCols<TileLarge, 2>::threads));
