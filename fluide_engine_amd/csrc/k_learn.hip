@@ -425,40 +425,74 @@ __global__ __launch_bounds__(256) void k_features(int64_t V, const float* __rest
     for (int c = 3; c < kNetIn; ++c) o[c] = 0;
 }
 
-__global__ __launch_bounds__(256) void k_pool(Lv f, Lv c, int C, const uint16_t* __restrict__ in,
-                                              uint16_t* __restrict__ out) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= c.V * C) return;
-    const int64_t vc = i / C;
-    const int ch = (int)(i - vc * C);
-    int X, Y, Z;
-    decode(c, vc, X, Y, Z);
-    float s = 0.0f;
-    for (int dz = 0; dz < 2; ++dz)
-        for (int dy = 0; dy < 2; ++dy)
-            for (int dx = 0; dx < 2; ++dx) {
-                const int64_t v = (2 * X + dx) + (int64_t)f.nx * ((2 * Y + dy) + (int64_t)f.ny * (2 * Z + dz));
-                s += from_bf16(in[v * C + ch]);
-            }
-    out[i] = to_bf16(s / 8.0f);
+// The passes between levels move data and are bound by it once a thread takes
+// 16 bytes (8 BF16 or 4 FP32 channels) and finds its voxel with 32-bit
+// divisions by constants: the concatenation at 64x96x80 takes 12 us (63 MB, the
+// rate of a copy) where one channel per thread behind 64-bit divisions took 68,
+// the seven passes of a gradient 65 us for 175.  A level's groups, 6 per finest
+// voxel at most, stay below 2^32: a network keeps some 800 bytes per voxel, so
+// 288 GB hold below 2^29.
+template <int GROUPS>
+__device__ inline bool group_of(int64_t V, uint32_t& v, uint32_t& g) {
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    v = i / GROUPS;
+    g = i - v * GROUPS;
+    return v < (uint32_t)V;
 }
 
-// out[v] = [coarse[parent(v)] (Cc channels), skip[v] (Cs channels)]
-__global__ __launch_bounds__(256) void k_upcat(Lv f, Lv c, int Cc, const uint16_t* __restrict__ coarse, int Cs,
+__device__ inline void decode32(const Lv& d, uint32_t v, uint32_t& x, uint32_t& y, uint32_t& z) {
+    const uint32_t r = v / (uint32_t)d.nx;
+    x = v - r * (uint32_t)d.nx;
+    z = r / (uint32_t)d.ny;
+    y = r - z * (uint32_t)d.ny;
+}
+
+// The voxel of the coarser level that v lies in.
+__device__ inline int64_t parent(const Lv& f, const Lv& c, uint32_t v) {
+    uint32_t x, y, z;
+    decode32(f, v, x, y, z);
+    return (x / 2) + (int64_t)c.nx * ((y / 2) + (int64_t)c.ny * (z / 2));
+}
+
+// F(voxel) for the eight voxels of the finer level in v, x fastest.
+template <typename F>
+__device__ inline void children(const Lv& f, const Lv& c, uint32_t v, F fn) {
+    uint32_t X, Y, Z;
+    decode32(c, v, X, Y, Z);
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+        fn((2 * X + (q & 1)) + (int64_t)f.nx * ((2 * Y + ((q >> 1) & 1)) + (int64_t)f.ny * (2 * Z + (q >> 2))));
+}
+
+template <int C>
+__global__ __launch_bounds__(256) void k_pool(Lv f, Lv c, const uint16_t* __restrict__ in,
+                                              uint16_t* __restrict__ out) {
+    uint32_t vc, g;
+    if (!group_of<C / 8>(c.V, vc, g)) return;
+    float s[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+    children(f, c, vc, [&](int64_t v) {
+        const u4 w = *reinterpret_cast<const u4*>(in + v * C + 8 * g);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            s[2 * q] += from_bf16((uint16_t)w[q]);
+            s[2 * q + 1] += from_bf16((uint16_t)(w[q] >> 16));
+        }
+    });
+    u4 o;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+        o[q] = (uint32_t)to_bf16(s[2 * q] / 8.0f) | ((uint32_t)to_bf16(s[2 * q + 1] / 8.0f) << 16);
+    *reinterpret_cast<u4*>(out + (int64_t)vc * C + 8 * g) = o;
+}
+
+// out[v] = [coarse[parent(v)] (CC channels), skip[v] (CS channels)]
+template <int CC, int CS>
+__global__ __launch_bounds__(256) void k_upcat(Lv f, Lv c, const uint16_t* __restrict__ coarse,
                                                const uint16_t* __restrict__ skip, uint16_t* __restrict__ out) {
-    const int Ct = Cc + Cs;
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= f.V * Ct) return;
-    const int64_t v = i / Ct;
-    const int ch = (int)(i - v * Ct);
-    if (ch < Cc) {
-        int x, y, z;
-        decode(f, v, x, y, z);
-        const int64_t p = (x / 2) + (int64_t)c.nx * ((y / 2) + (int64_t)c.ny * (z / 2));
-        out[i] = coarse[p * Cc + ch];
-    } else {
-        out[i] = skip[v * Cs + ch - Cc];
-    }
+    uint32_t v, g;
+    if (!group_of<(CC + CS) / 8>(f.V, v, g)) return;
+    const uint16_t* in = g < CC / 8 ? coarse + parent(f, c, v) * CC + 8 * g : skip + (int64_t)v * CS + (8 * g - CC);
+    *reinterpret_cast<u4*>(out + (int64_t)v * (CC + CS) + 8 * g) = *reinterpret_cast<const u4*>(in);
 }
 
 __global__ __launch_bounds__(256) void k_head(int64_t V, const float* __restrict__ D0, const float* __restrict__ hw,
@@ -576,45 +610,35 @@ __global__ __launch_bounds__(256) void k_codes(Lv d, const uint8_t* __restrict__
                        (uint32_t)d.nz);
 }
 
-// gCoarse[p][c] = sum over the 8 children of gC[child][c], c < Cc
-__global__ __launch_bounds__(256) void k_up_bwd(Lv f, Lv c, int Cc, int Ct, const float* __restrict__ gC,
+// The coarse voxel's gradient: the sum over its children of the first CC of
+// the concatenation's channels.
+template <int CC, int CS>
+__global__ __launch_bounds__(256) void k_up_bwd(Lv f, Lv c, const float* __restrict__ gC,
                                                 float* __restrict__ gCoarse) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= c.V * Cc) return;
-    const int64_t p = i / Cc;
-    const int ch = (int)(i - p * Cc);
-    int X, Y, Z;
-    decode(c, p, X, Y, Z);
-    float s = 0.0f;
-    for (int dz = 0; dz < 2; ++dz)
-        for (int dy = 0; dy < 2; ++dy)
-            for (int dx = 0; dx < 2; ++dx) {
-                const int64_t v = (2 * X + dx) + (int64_t)f.nx * ((2 * Y + dy) + (int64_t)f.ny * (2 * Z + dz));
-                s += gC[v * Ct + ch];
-            }
-    gCoarse[i] = s;
+    uint32_t p, g;
+    if (!group_of<CC / 4>(c.V, p, g)) return;
+    float4 s = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    children(f, c, p, [&](int64_t v) {
+        const float4 a = *reinterpret_cast<const float4*>(gC + v * (CC + CS) + 4 * g);
+        s.x += a.x;
+        s.y += a.y;
+        s.z += a.z;
+        s.w += a.w;
+    });
+    *reinterpret_cast<float4*>(gCoarse + (int64_t)p * CC + 4 * g) = s;
 }
 
-// gSkip[v][c] = gC[v][Cc + c]
-__global__ __launch_bounds__(256) void k_skip_bwd(int64_t V, int Cc, int Cs, const float* __restrict__ gC,
-                                                  float* __restrict__ gSkip) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= V * Cs) return;
-    const int64_t v = i / Cs;
-    gSkip[i] = gC[v * (Cc + Cs) + Cc + (i - v * Cs)];
-}
-
-// gFine[v][c] += gCoarse[parent(v)][c] / 8
-__global__ __launch_bounds__(256) void k_pool_bwd(Lv f, Lv c, int C, const float* __restrict__ gCoarse,
-                                                  float* __restrict__ gFine) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= f.V * C) return;
-    const int64_t v = i / C;
-    const int ch = (int)(i - v * C);
-    int x, y, z;
-    decode(f, v, x, y, z);
-    const int64_t p = (x / 2) + (int64_t)c.nx * ((y / 2) + (int64_t)c.ny * (z / 2));
-    gFine[i] += gCoarse[p * C + ch] / 8.0f;
+// An encoder level's gradient: the concatenation's last CS channels plus an
+// eighth of the pooled level's.
+template <int CC, int CS>
+__global__ __launch_bounds__(256) void k_enc_bwd(Lv f, Lv c, const float* __restrict__ gC,
+                                                 const float* __restrict__ gPool, float* __restrict__ gE) {
+    uint32_t v, g;
+    if (!group_of<CS / 4>(f.V, v, g)) return;
+    const float4 a = *reinterpret_cast<const float4*>(gC + (int64_t)v * (CC + CS) + CC + 4 * g);
+    const float4 b = *reinterpret_cast<const float4*>(gPool + parent(f, c, v) * CS + 4 * g);
+    *reinterpret_cast<float4*>(gE + (int64_t)v * CS + 4 * g) =
+        make_float4(a.x + b.x / 8.0f, a.y + b.y / 8.0f, a.z + b.z / 8.0f, a.w + b.w / 8.0f);
 }
 
 __global__ __launch_bounds__(256) void k_adam(int64_t n, float* __restrict__ w, const float* __restrict__ g,
@@ -987,19 +1011,19 @@ hipError_t net_forward(fe_net* n, const float* b, const uint8_t* flags, double r
         return launch_conv(st, d, X, L.cin, L.cout, L.wp, L.b, 1, Y, nullptr);
     };
     if ((e = conv(0, l0, n->X0, n->E0)) != hipSuccess) return e;
-    hipLaunchKernelGGL(k_pool, g1(l1.V * 16), dim3(256), 0, st, l0, l1, 16, (const uint16_t*)n->E0, n->P1);
+    hipLaunchKernelGGL(k_pool<16>, g1(l1.V * (16 / 8)), dim3(256), 0, st, l0, l1, (const uint16_t*)n->E0, n->P1);
     if ((e = conv(1, l1, n->P1, n->E1)) != hipSuccess) return e;
-    hipLaunchKernelGGL(k_pool, g1(l2.V * 32), dim3(256), 0, st, l1, l2, 32, (const uint16_t*)n->E1, n->P2);
+    hipLaunchKernelGGL(k_pool<32>, g1(l2.V * (32 / 8)), dim3(256), 0, st, l1, l2, (const uint16_t*)n->E1, n->P2);
     if ((e = conv(2, l2, n->P2, n->E2)) != hipSuccess) return e;
-    hipLaunchKernelGGL(k_pool, g1(l3.V * 48), dim3(256), 0, st, l2, l3, 48, (const uint16_t*)n->E2, n->P3);
+    hipLaunchKernelGGL(k_pool<48>, g1(l3.V * (48 / 8)), dim3(256), 0, st, l2, l3, (const uint16_t*)n->E2, n->P3);
     if ((e = conv(3, l3, n->P3, n->E3)) != hipSuccess) return e;
-    hipLaunchKernelGGL(k_upcat, g1(l2.V * 112), dim3(256), 0, st, l2, l3, 64, (const uint16_t*)n->E3, 48,
+    hipLaunchKernelGGL((k_upcat<64, 48>), g1(l2.V * ((64 + 48) / 8)), dim3(256), 0, st, l2, l3, (const uint16_t*)n->E3,
                        (const uint16_t*)n->E2, n->C2);
     if ((e = conv(4, l2, n->C2, n->D2)) != hipSuccess) return e;
-    hipLaunchKernelGGL(k_upcat, g1(l1.V * 80), dim3(256), 0, st, l1, l2, 48, (const uint16_t*)n->D2, 32,
+    hipLaunchKernelGGL((k_upcat<48, 32>), g1(l1.V * ((48 + 32) / 8)), dim3(256), 0, st, l1, l2, (const uint16_t*)n->D2,
                        (const uint16_t*)n->E1, n->C1);
     if ((e = conv(5, l1, n->C1, n->D1)) != hipSuccess) return e;
-    hipLaunchKernelGGL(k_upcat, g1(l0.V * 48), dim3(256), 0, st, l0, l1, 32, (const uint16_t*)n->D1, 16,
+    hipLaunchKernelGGL((k_upcat<32, 16>), g1(l0.V * ((32 + 16) / 8)), dim3(256), 0, st, l0, l1, (const uint16_t*)n->D1,
                        (const uint16_t*)n->E0, n->C0);
     {
         const NetLayer& L = n->L[6];
@@ -1035,21 +1059,21 @@ hipError_t net_backward(fe_net* n, const LossIn& in, float* loss_slot) {
                        1.0);
     // decoder
     if ((e = layer_back(n, 6, l0, n->C0, n->D0, n->gD0, n->gC0)) != hipSuccess) return e;
-    hipLaunchKernelGGL(k_up_bwd, g1(l1.V * 32), dim3(256), 0, st, l0, l1, 32, 48, (const float*)n->gC0, n->gD1);
-    hipLaunchKernelGGL(k_skip_bwd, g1(l0.V * 16), dim3(256), 0, st, l0.V, 32, 16, (const float*)n->gC0, n->gE0);
+    hipLaunchKernelGGL((k_up_bwd<32, 16>), g1(l1.V * (32 / 4)), dim3(256), 0, st, l0, l1, (const float*)n->gC0, n->gD1);
     if ((e = layer_back(n, 5, l1, n->C1, n->D1, n->gD1, n->gC1)) != hipSuccess) return e;
-    hipLaunchKernelGGL(k_up_bwd, g1(l2.V * 48), dim3(256), 0, st, l1, l2, 48, 80, (const float*)n->gC1, n->gD2);
-    hipLaunchKernelGGL(k_skip_bwd, g1(l1.V * 32), dim3(256), 0, st, l1.V, 48, 32, (const float*)n->gC1, n->gE1);
+    hipLaunchKernelGGL((k_up_bwd<48, 32>), g1(l2.V * (48 / 4)), dim3(256), 0, st, l1, l2, (const float*)n->gC1, n->gD2);
     if ((e = layer_back(n, 4, l2, n->C2, n->D2, n->gD2, n->gC2)) != hipSuccess) return e;
-    hipLaunchKernelGGL(k_up_bwd, g1(l3.V * 64), dim3(256), 0, st, l2, l3, 64, 112, (const float*)n->gC2, n->gE3);
-    hipLaunchKernelGGL(k_skip_bwd, g1(l2.V * 48), dim3(256), 0, st, l2.V, 64, 48, (const float*)n->gC2, n->gE2);
+    hipLaunchKernelGGL((k_up_bwd<64, 48>), g1(l3.V * (64 / 4)), dim3(256), 0, st, l2, l3, (const float*)n->gC2, n->gE3);
     // encoder
     if ((e = layer_back(n, 3, l3, n->P3, n->E3, n->gE3, n->gP3)) != hipSuccess) return e;
-    hipLaunchKernelGGL(k_pool_bwd, g1(l2.V * 48), dim3(256), 0, st, l2, l3, 48, (const float*)n->gP3, n->gE2);
+    hipLaunchKernelGGL((k_enc_bwd<64, 48>), g1(l2.V * (48 / 4)), dim3(256), 0, st, l2, l3, (const float*)n->gC2,
+                       (const float*)n->gP3, n->gE2);
     if ((e = layer_back(n, 2, l2, n->P2, n->E2, n->gE2, n->gP2)) != hipSuccess) return e;
-    hipLaunchKernelGGL(k_pool_bwd, g1(l1.V * 32), dim3(256), 0, st, l1, l2, 32, (const float*)n->gP2, n->gE1);
+    hipLaunchKernelGGL((k_enc_bwd<48, 32>), g1(l1.V * (32 / 4)), dim3(256), 0, st, l1, l2, (const float*)n->gC1,
+                       (const float*)n->gP2, n->gE1);
     if ((e = layer_back(n, 1, l1, n->P1, n->E1, n->gE1, n->gP1)) != hipSuccess) return e;
-    hipLaunchKernelGGL(k_pool_bwd, g1(l0.V * 16), dim3(256), 0, st, l0, l1, 16, (const float*)n->gP1, n->gE0);
+    hipLaunchKernelGGL((k_enc_bwd<32, 16>), g1(l0.V * (16 / 4)), dim3(256), 0, st, l0, l1, (const float*)n->gC0,
+                       (const float*)n->gP1, n->gE0);
     if ((e = layer_back(n, 0, l0, n->X0, n->E0, n->gE0, nullptr)) != hipSuccess) return e;
     return hipGetLastError();
 }
