@@ -56,9 +56,13 @@ inline dim3 g1(int64_t n) { return dim3((unsigned)((n + 255) / 256)); }
 // reads at an offset past the buffer's end, which the load gives as zeros.
 // Bound by the first-level cache: per 32 of K it reads MT KB of activations
 // and NT KB of packed weights for MT NT matrix instructions, so a large level
-// takes MT = 4.  At 64x96x80 (us per launch, with one 16-voxel tile and 16 of
-// K per step before): 16 and 48 -> 16 channels on the finest level 100 (mean),
-// 16 -> 48 there and 32, 112 -> 48 below 73 (mean), 48 -> 112 on the third 80.
+// takes MT = 4.  A small level is bound by the latency of a wavefront's chain
+// of K steps (0.6 us each), so there the four wavefronts of a workgroup share
+// a tile, every fourth step each, and add their sums in order at the end
+// (KS = 4).  At 64x96x80 (us per launch; with one 16-voxel tile, 16 of K per
+// step and a wavefront per tile in brackets): 16 and 48 -> 16 channels on the
+// finest level 69 (100), 16 -> 48 there 57 (73); all launches of the three
+// levels below together 166 where a wavefront per tile took 245.
 typedef __bf16 b8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u4 __attribute__((ext_vector_type(4)));
 __device__ inline b8 as_b8(const u4& w) { return __builtin_bit_cast(b8, w); }
@@ -68,7 +72,7 @@ constexpr int kMaxCh = 112;
 constexpr int kMaxChunks = (27 * kMaxCh + 31) / 32;
 constexpr uint32_t kConvReach = 0x7FFFFFFFu;  // bytes a load may reach from its wave's base
 
-template <int MT, int NT>
+template <int MT, int NT, int KS>
 __global__ __launch_bounds__(256) void k_conv(Lv d, const uint16_t* __restrict__ X, int cin, int cout,
                                               const u4* __restrict__ Wp, const float* __restrict__ bias, int relu,
                                               uint16_t* __restrict__ Ybf, float* __restrict__ Yf) {
@@ -81,8 +85,9 @@ __global__ __launch_bounds__(256) void k_conv(Lv d, const uint16_t* __restrict__
     }
     __syncthreads();
     const int wave = threadIdx.x >> 6, l = threadIdx.x & 63, row = l & 15, kq = l >> 4;
-    const int64_t v0 = ((int64_t)blockIdx.x * 4 + wave) * (16 * MT);
-    if (v0 >= d.V) return;  // uniform per wavefront
+    const int first = wave % KS;  // of this wave's share of K
+    const int64_t v0 = ((int64_t)blockIdx.x * (4 / KS) + wave / KS) * (16 * MT);
+    if (v0 >= d.V) return;  // uniform per wavefront (KS = 4: never)
     const int nt0 = blockIdx.y * NT, nts = cout / 16;
     // the buffer starts a z slice and a row before the wave's first voxel
     const int64_t reach = (int64_t)d.nx * d.ny + d.nx + 1;
@@ -123,9 +128,9 @@ __global__ __launch_bounds__(256) void k_conv(Lv d, const uint16_t* __restrict__
         }
     };
     b8 a[MT], b[NT], an[MT], bn[NT];
-    load(0, a, b);
-    for (int c = 0; c < chunks; ++c) {
-        load(min(c + 1, chunks - 1), an, bn);  // the next step's, before this one's products
+    load(first, a, b);  // 14 steps at least
+    for (int c = first; c < chunks; c += KS) {
+        load(min(c + KS, chunks - 1), an, bn);  // the next step's, before this one's products
 #pragma unroll
         for (int m = 0; m < MT; ++m)
 #pragma unroll
@@ -135,6 +140,24 @@ __global__ __launch_bounds__(256) void k_conv(Lv d, const uint16_t* __restrict__
         for (int m = 0; m < MT; ++m) a[m] = an[m];
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) b[nt] = bn[nt];
+    }
+    if constexpr (KS > 1) {  // the shares' sums, in order
+        static_assert(KS == 4, "a workgroup's waves share one tile");
+        __shared__ f4 part[KS - 1][MT * NT][64];
+        if (wave > 0) {
+#pragma unroll
+            for (int m = 0; m < MT; ++m)
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt) part[wave - 1][m * NT + nt][l] = acc[m][nt];
+        }
+        __syncthreads();
+        if (wave > 0) return;
+#pragma unroll
+        for (int q = 0; q < KS - 1; ++q)
+#pragma unroll
+            for (int m = 0; m < MT; ++m)
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt) acc[m][nt] += part[q][m * NT + nt][l];
     }
 #pragma unroll
     for (int m = 0; m < MT; ++m)
@@ -725,26 +748,31 @@ __global__ __launch_bounds__(256) void k_zero_f(int64_t n, float* __restrict__ a
 // ---------------------------------------------------------------------------
 // Host drivers
 // ---------------------------------------------------------------------------
-template <int MT, int NT>
+template <int MT, int NT, int KS>
 hipError_t launch_conv_tile(hipStream_t st, const Lv& d, const uint16_t* X, int cin, int cout, const uint16_t* wp,
                             const float* bias, int relu, uint16_t* ybf, float* yf) {
-    const dim3 grid((unsigned)((d.V + 64 * MT - 1) / (64 * MT)), (unsigned)(cout / 16 / NT));
-    hipLaunchKernelGGL((k_conv<MT, NT>), grid, dim3(256), 0, st, d, X, cin, cout, reinterpret_cast<const u4*>(wp),
+    const int64_t voxels = 16 * MT * (4 / KS);  // per workgroup
+    const dim3 grid((unsigned)((d.V + voxels - 1) / voxels), (unsigned)(cout / 16 / NT));
+    hipLaunchKernelGGL((k_conv<MT, NT, KS>), grid, dim3(256), 0, st, d, X, cin, cout, reinterpret_cast<const u4*>(wp),
                        bias, relu, ybf, yf);
     return hipGetLastError();
 }
 
-// Large tiles as long as they leave every SIMD a wave or two (1024 SIMDs); a
-// small level's launch is one wave's chain of loads, so it takes the most
-// waves: single tiles, an output group each.
+// Large tiles as long as they leave every SIMD a wave or two (1024 SIMDs).
+// Below, a workgroup's wavefronts share a tile, and the smallest levels take
+// the most workgroups: single tiles, an output group each.  From five output
+// groups on the sums' LDS and their one wavefront cost more than the sharing
+// saves (32 -> 80 channels on 61 440 voxels: 38 us for 30).  Loss and gradients
+// with a wavefront per tile / with shared tiles: 16^3 540 / 480 us, 32x40x32
+// 673 / 564, 64^3 1079 / 970, 64x96x80 1484 / 1397.
 hipError_t launch_conv(hipStream_t st, const Lv& d, const uint16_t* X, int cin, int cout, const uint16_t* wp,
                        const float* bias, int relu, uint16_t* ybf, float* yf) {
     const int mt = d.V >= 64 * 2048 ? 4 : (d.V >= 32 * 1024 ? 2 : 1);
-    if (mt == 1) return launch_conv_tile<1, 1>(st, d, X, cin, cout, wp, bias, relu, ybf, yf);
+    if (mt == 1) return launch_conv_tile<1, 1, 4>(st, d, X, cin, cout, wp, bias, relu, ybf, yf);
 #define FE_CONV(NT)                                                                                        \
     case NT:                                                                                               \
-        return mt == 4 ? launch_conv_tile<4, NT>(st, d, X, cin, cout, wp, bias, relu, ybf, yf)             \
-                       : launch_conv_tile<2, NT>(st, d, X, cin, cout, wp, bias, relu, ybf, yf)
+        return mt == 4 ? launch_conv_tile<4, NT, 1>(st, d, X, cin, cout, wp, bias, relu, ybf, yf)             \
+                       : launch_conv_tile<2, NT, (NT < 5 ? 4 : 1)>(st, d, X, cin, cout, wp, bias, relu, ybf, yf)
     switch (cout / 16) {
         FE_CONV(1);
         FE_CONV(2);

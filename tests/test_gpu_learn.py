@@ -77,6 +77,13 @@ def test_gradients_on_ragged_levels(ctx, shape):
     test_forward_backward_matches_restatement(ctx, shape, "mse")
 
 
+@pytest.mark.parametrize("shape", [(32, 32, 40), (64, 64, 64)])
+def test_gradients_on_every_convolution_tile(ctx, shape):
+    """Levels on 16, 32 and 64 voxels a wavefront (below 32 768 cells, below
+    131 072, above), their last tiles partly filled; bounds as above."""
+    test_forward_backward_matches_restatement(ctx, shape, "mse")
+
+
 def _dam_scene(ctx, n, box_hi, seed=0):
     desc = capi.scene_desc((n, n, n), method=capi.FLIP, blend=0.03, max_particles=8 * n ** 3)
     x = capi.seed_particles(desc, [capi.box((-1, -1, -1), box_hi)], seed=seed)
