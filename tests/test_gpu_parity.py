@@ -228,6 +228,23 @@ def test_pressure_cg_reaches_tolerance(ctx, kind, shape):
     g.close()
 
 
+@pytest.mark.parametrize("cap", [1, 2, 5])
+@pytest.mark.parametrize("shape", [(5, 4, 3), (33, 20, 17), (70, 65, 64)])  # the last: four cells a thread (above 2^18)
+@pytest.mark.parametrize("kind", [capi.SOLVER_CG, capi.SOLVER_PCG_JACOBI])
+def test_cg_iterates_match_oracle(ctx, kind, shape, cap):
+    """The iterate after exactly cap iterations against the oracle's FP64 one.
+    The right-hand side is held in FP32 (6e-8 of its largest value) and an
+    iterate of up to five steps is a polynomial in it whose sensitivity on
+    these systems is below 100: 1e-5 of the largest pressure."""
+    print(f"[gpu] cg iterates kind={kind} shape={shape} cap={cap}", flush=True)
+    g, o = _pressure_pair(ctx, shape, 19)
+    sg = g.run_stage(capi.STAGE_PRESSURE, desc=capi.solver(kind, cap, 0, 1e-14, relative=True, warm_start=False))
+    so = o.pressure(orc.solver(ORC_SOLVER[kind], cap, 0, 1e-14, relative=True, warm_start=False))
+    assert sg.iterations == so.iterations == cap
+    rel_close(g.get(capi.GRID_PRESSURE), o.get(orc.PRESSURE), 1e-5, "cg iterate")
+    g.close()
+
+
 @pytest.mark.parametrize("n", [48, 64])
 @pytest.mark.parametrize("kind", [capi.SOLVER_MGPCG, capi.SOLVER_CG])
 def test_first_substep_solve_converges(ctx, kind, n):
