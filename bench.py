@@ -30,10 +30,11 @@ HBM_PEAK_GBS = 8000.0
 # Algorithmic HBM bytes per cell for one launch of each timed kernel (FP32
 # vectors, FP64 solution, 1-byte markers whose 6 neighbours come from cache).
 KERNEL_BYTES_PER_CELL = {
-    # k_cg_update: read x(8) d(4) q(4) r(4), write x'(8) r(4); the diagonal
-    # preconditioner adds the row code(2) and z(4) (see update_bytes)
+    # k_cg_update: read x(8) d(4) q(4) r(4), write x'(8) r(4)
     "cg_update": 32,
-    # k_cg_spmv: read z(4) d(4) row code(2), write d'(4) q(4)
+    # k_cg_spmv: read z(4) d(4) row code(2), write d'(4) q(4); without multigrid
+    # a whole iteration, k_cg_step: read r(4) d(4) q(4) x(8) row code(2), write
+    # r'(4) d'(4) q'(4) x'(8)
     "cg_spmv": 18,
     # k_jacobi: read x(4) b(4) row code(2), write x'(4)
     "jacobi": 14,
@@ -52,8 +53,8 @@ SOLVER_TEXT = {"jacobi": "Jacobi sweeps", "cg": "CG", "pcg": "Jacobi-PCG", "mgpc
 
 def kernel_bytes_per_cell(kernel, solver, mg_split=False):
     b = KERNEL_BYTES_PER_CELL[kernel]
-    if kernel == "cg_update" and solver == "pcg":
-        b += 6
+    if kernel == "cg_spmv" and solver in ("cg", "pcg"):
+        b = 42
     if kernel == "cg_update" and solver == "mgpcg" and mg_split:  # row code(2) + the V-cycle's first sweep(4)
         b += 6
     return b
@@ -315,8 +316,9 @@ def main():
     # the other timed kernels' rooflines, each over a few more substeps after the timed region
     rooflines = {}
     if args.kernel != "none":
-        others = ["g2p_move", "sdf"] + ([] if args.solver == "jacobi" else ["cg_update", "cg_spmv"])
+        others = ["g2p_move", "sdf"] + ([] if args.solver == "jacobi" else ["cg_spmv"])
         if args.solver == "mgpcg":
+            others += ["cg_update"]
             others += ["mg_down", "mg_up"] if scene.mg_variant() == capi.MG_FUSED else ["mg_smooth"]
         for kern in others:
             if kern == args.kernel:

@@ -383,6 +383,9 @@ __device__ inline void add_half_solid_angle(AngleSum& z, const D3& x, const D3& 
 
 constexpr double kPi = 3.14159265358979323846;  // src/common/math_utils.hpp:11
 
+// Bound by FP64 instructions: with an atan2 and three square roots per node
+// and triangle 64^3 nodes for a mesh of 1472 triangles took 2.86 ms for the whole call,
+// with the complex product 1.34 ms.
 // tv: 9 doubles per triangle (its three vertices); tb: 6 ints per triangle,
 // the index box i0, j0, k0, i1, j1, k1 (inclusive).
 template <int SLICES>

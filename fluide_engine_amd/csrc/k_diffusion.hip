@@ -161,7 +161,8 @@ __device__ inline double diff_offdiag(uint16_t cd, const double (&c)[3], const d
 // and whether any value differs from the snapshot of an earlier state, which
 // `snap` 1 renews.  !WRITE: the partials only (a check after the last sweep).
 //
-// Bound by the latency of its loads (1.5 M faces at 96x80x64 in 7.4 us, of
+// Bound by the latency of its loads (1.5 M faces at 96x80x64 in 7.4 us, where
+// a launch per component took 3 x 5.2 us and every fifth sweep 3 x 7.9 us more; of
 // which about 20 MB are read for the fluid rows, from cache): the row code
 // decides only whether a thread reads at all, and the six neighbours and b of
 // all its rows are then loaded together instead of one after another under the

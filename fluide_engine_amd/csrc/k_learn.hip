@@ -305,6 +305,10 @@ __global__ __launch_bounds__(256) void k_mask(Lv d, int C, const float* __restri
     });
 }
 
+// 16 input channels and the finest level's 491 520 voxels: 44 us, 48 channels
+// 116 us, where voxel-major operands gathered a value at a time took 1.1 ms for
+// the seven layers and their partials' sum 0.6 ms (now 0.26, 0.15 for the
+// planes, and 0.04 ms).
 // blockIdx.y = 3 kc + dz (16 input channels, z offset dz - 1).  Wave w of block
 // b takes the 32-voxel steps [ (4 b + w) spw, ... + spw ).
 template <int NT>

@@ -23,14 +23,12 @@
 // Non-FLUID cells carry no residual into the coarse levels and take no
 // correction; on level 0 they are smoothed like the identity rows they are.
 //
-// Kernels per V-cycle on the large levels: the first sweep from zero is fused
-// into the kernel that produces the level's right-hand side (the CG update on
-// level 0, the restriction below it), then one sweep, the residual, the
-// restriction; on the way up the prolongation and two sweeps.  The coarsest
-// level (at most 512 cells) runs in one workgroup in LDS (k_mg_tail).  The
-// tail once also took the next level up (16^3 at 128^3): one workgroup on one
-// CU then did 4096 cells' sweeps, about 15 us per V-cycle, where the fused
-// kernels' 8 workgroups take 11 us for that level's descent and ascent.
+// Kernels per V-cycle (FE_MG_FUSED): a descent and an ascent per level over LDS
+// tiles (k_mg_down, k_mg_up), the last two levels in one workgroup
+// (k_mg_bottom), or, where they do not fit it, the coarsest alone (k_mg_tail).
+// FE_MG_SPLIT takes one kernel per sweep, residual, restriction and
+// prolongation, the first sweep from zero fused into the kernel that produces
+// the level's right-hand side.
 #include <algorithm>
 
 #include "fe_stencil.hpp"
@@ -590,8 +588,9 @@ __global__ __launch_bounds__(kBlock) void k_mg_prolong(const float* __restrict__
 // once instead of in every phase, their own values, diagonals and weights and
 // the neighbours along z within its planes stay in registers, and every other
 // neighbour is at a constant distance in LDS.  With the window's cells dealt
-// to the threads anew in each phase a wavefront ran about three times the
-// instructions (MEASURED).
+// to the threads anew in each phase the finest level's descent and ascent of a
+// 128^3 dam break took 14.0 and 16.1 us, now 11.4 and 12.7; the small tiles
+// below 5.6 us each, now 4.3 and 3.8.
 //   descent:  x1 = w b (first sweep from zero), x2 = x1 + w (b - A x1) (kept
 //             for the ascent), r = b - A x2, coarse b = R r;
 //   ascent:   y = x2 + P xc, x' = y + w (b - A y), out = x' + w (b - A x'),
@@ -1221,7 +1220,7 @@ __global__ __launch_bounds__(kTailThreads) void k_mg_tail(TailArgs a, const floa
 // the coarsest level, its Chebyshev iteration, and the ascent.  Bound by the
 // chain of phases between barriers (a level of 16^3 over one of 8^3: 16
 // barriers); it replaces three launches (4.7 + 4.2 + 5.1 us and the gaps
-// between them) with one.
+// between them) with one of 10 us.
 //
 // A thread keeps up to four fine cells (right-hand side, diagonal, weight and
 // place, in registers) and at most one coarse cell.  The iterates lie in LDS

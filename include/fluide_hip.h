@@ -474,8 +474,8 @@ int fe_stage_times(const fe_scene* scene, double* ms, int32_t count);
  * fe_kernel_timer(scene, FE_KERNEL_NONE) switches it off. */
 enum fe_kernel_id {
     FE_KERNEL_NONE = 0,
-    FE_KERNEL_CG_SPMV = 1,    /* d = z + beta d, q = A d, d.q */
-    FE_KERNEL_CG_UPDATE = 2,  /* x += alpha d, r -= alpha q, z = M^-1 r, r.z */
+    FE_KERNEL_CG_SPMV = 1,    /* d = z + beta d, q = A d, d.q; without multigrid an iteration whole */
+    FE_KERNEL_CG_UPDATE = 2,  /* multigrid PCG: x += alpha d, r -= alpha q, z = M^-1 r, r.z */
     FE_KERNEL_P2G = 3,        /* per-face gather (3 launches per substep, one per component) */
     FE_KERNEL_G2P_MOVE = 4,   /* fused G2P + advection */
     FE_KERNEL_SDF = 5,        /* fluid SDF */
