@@ -170,6 +170,31 @@ def test_extrapolate_bc_gravity_parity(ctx, shape):
     g.close()
 
 
+@pytest.mark.parametrize("density", [0.0, 0.004, 0.97, 1.0])
+@pytest.mark.parametrize("shape", [(2, 2, 2), (67, 5, 3), (13, 11, 7)])
+def test_extrapolate_sparse_and_full(ctx, shape, density):
+    """Groups of four faces with nothing to fill (none of their neighbours
+    marked, or all four) beside groups that have, at rows and arrays that do
+    not end on a group."""
+    print(f"[gpu] extrapolate {shape} density {density}", flush=True)
+    desc = capi.scene_desc(shape, method=capi.FLIP, max_particles=16)
+    g = capi.Scene(ctx, desc)
+    o = orc.Scene(shape, method=orc.FLIP)
+    rng = np.random.default_rng(9)
+    for (gf, of), (gm, om) in zip(GRID, MARK):
+        shp = g.shape(gf)
+        vals = rng.normal(size=shp).astype(np.float32)
+        mk = (rng.uniform(size=shp) < density).astype(np.uint8)
+        vals[mk == 0] = 0.0
+        g.set(gf, vals); o.set(of, vals.astype(np.float64))
+        g.set(gm, mk); o.set(om, mk.astype(np.int32))
+    g.run_stage(capi.STAGE_EXTRAPOLATE)
+    o.extrapolate_to_air()
+    for gf, of in GRID:  # three sweeps of means of six FP32 values: 3 x 6 roundings of 6e-8
+        rel_close(g.get(gf), o.get(of), 1.1e-6, f"extrapolated {gf}")
+    g.close()
+
+
 # ---------------------------------------------------------------------------
 # pressure projection
 # ---------------------------------------------------------------------------
