@@ -3,8 +3,8 @@
 // FP32 accumulation.  No counterpart in the reference.
 //
 // Convolutions are implicit GEMMs over channel-last BF16 activations, K = 27
-// taps x input channels, 32 at a time (v_mfma_f32_16x16x32_bf16; a lane holds
-// A[l % 16][8 (l / 16) + j], B[8 (l / 16) + j][l % 16] and returns
+// taps x input channels, 16 at a time (v_mfma_f32_16x16x16_bf16; a lane holds
+// A[l % 16][4 (l / 16) + j], B[4 (l / 16) + j][l % 16] and returns
 // C[4 (l / 16) + i][l % 16], checked on the device).
 // The backward data pass is the same kernel on the flipped, transposed weights;
 // the weight gradient is a GEMM over voxels (M = input channel, N = output
@@ -51,32 +51,41 @@ inline dim3 g1(int64_t n) { return dim3((unsigned)((n + 255) / 256)); }
 // Convolution (forward, and backward data on the flipped weights)
 // ---------------------------------------------------------------------------
 // A wavefront computes 16 MT consecutive voxels x 16 NT output channels.  K
-// runs over (tap, channel) pairs 32 at a time; the 8 channels of a lane belong
-// to one tap, whose offset comes from a table in LDS.  A voxel outside the grid
+// runs over blocks of one tap and 16 channels, taps outermost, two blocks per
+// step.  An output is one chain of products in that order whatever the tile,
+// so no launch shape moves the BF16 roundings of the layers behind; an
+// instruction of twice the depth, or shares of K added up, do (26 % of its sums
+// change by a bit at the same error of 3.9e-8, and a gradient by 6.5e-4).
+// A lane loads 16 bytes, half a block's channels of a voxel; two swaps of 16
+// lanes turn the step's four halves into its blocks' operands, where lane group
+// q holds channels 4 q .. 4 q + 3 (8-byte loads straight into that place touch
+// twice the cache lines: 130 us for the 92 below).  A voxel outside the grid
 // reads at an offset past the buffer's end, which the load gives as zeros.
-// Bound by the first-level cache: per 32 of K it reads MT KB of activations
-// and NT KB of packed weights for MT NT matrix instructions, so a large level
-// takes MT = 4.  A small level is bound by the latency of a wavefront's chain
-// of K steps (0.6 us each), so there the four wavefronts of a workgroup share
-// a tile, every fourth step each, and add their sums in order at the end
-// (KS = 4).  At 64x96x80 (us per launch; with one 16-voxel tile, 16 of K per
-// step and a wavefront per tile in brackets): 16 and 48 -> 16 channels on the
-// finest level 69 (100), 16 -> 48 there 57 (73); all launches of the three
-// levels below together 166 where a wavefront per tile took 245.
+// Bound by the first-level cache: per step it reads MT KB of activations and
+// NT KB of packed weights for 2 MT NT matrix instructions.  A step's loads are
+// issued AHEAD steps before its products; a small level, bound by the latency
+// of a wavefront's chain of steps, keeps more of them in flight.  At 64x96x80
+// (us per launch): 16 and 48 -> 16 channels on the finest level 32 and 92, 16
+// -> 48 there 64, all launches of the three levels below together 157; with a
+// 16-voxel tile, 8-byte loads and a step of one block they took 200 for the
+// first two, 73 and 245.
 typedef __bf16 b8 __attribute__((ext_vector_type(8)));
+typedef short s4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u4 __attribute__((ext_vector_type(4)));
 __device__ inline b8 as_b8(const u4& w) { return __builtin_bit_cast(b8, w); }
+__device__ inline s4 as_s4(const u2& w) { return __builtin_bit_cast(s4, w); }
 
 __host__ __device__ inline int conv_chunks(int cin) { return (27 * cin + 31) / 32; }
 constexpr int kMaxCh = 112;
 constexpr int kMaxChunks = (27 * kMaxCh + 31) / 32;
 constexpr uint32_t kConvReach = 0x7FFFFFFFu;  // bytes a load may reach from its wave's base
 
-template <int MT, int NT, int KS>
+template <int MT, int NT, int AHEAD>
 __global__ __launch_bounds__(256) void k_conv(Lv d, const uint16_t* __restrict__ X, int cin, int cout,
                                               const u4* __restrict__ Wp, const float* __restrict__ bias, int relu,
                                               uint16_t* __restrict__ Ybf, float* __restrict__ Yf) {
-    __shared__ int2 table[4 * kMaxChunks];  // per chunk and lane group: byte offset, tap (27: none)
+    __shared__ int2 table[4 * kMaxChunks];  // per half block: byte offset, tap (27: none)
     const int chunks = conv_chunks(cin);
     for (int e = threadIdx.x; e < 4 * chunks; e += 256) {
         const int t = 8 * e / cin, ch = 8 * e - t * cin;
@@ -85,9 +94,8 @@ __global__ __launch_bounds__(256) void k_conv(Lv d, const uint16_t* __restrict__
     }
     __syncthreads();
     const int wave = threadIdx.x >> 6, l = threadIdx.x & 63, row = l & 15, kq = l >> 4;
-    const int first = wave % KS;  // of this wave's share of K
-    const int64_t v0 = ((int64_t)blockIdx.x * (4 / KS) + wave / KS) * (16 * MT);
-    if (v0 >= d.V) return;  // uniform per wavefront (KS = 4: never)
+    const int64_t v0 = ((int64_t)blockIdx.x * 4 + wave) * (16 * MT);
+    if (v0 >= d.V) return;  // uniform per wavefront
     const int nt0 = blockIdx.y * NT, nts = cout / 16;
     // the buffer starts a z slice and a row before the wave's first voxel
     const int64_t reach = (int64_t)d.nx * d.ny + d.nx + 1;
@@ -117,48 +125,50 @@ __global__ __launch_bounds__(256) void k_conv(Lv d, const uint16_t* __restrict__
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) acc[m][nt] = f4{0.f, 0.f, 0.f, 0.f};
     const u4* wb = Wp + (int64_t)nt0 * 64 + l;
-    auto load = [&](int c, b8 (&a)[MT], b8 (&b)[NT]) {
-        const int2 e = table[4 * c + kq];
+    const int half = (kq >> 1) | ((kq & 1) << 1);  // of the step's four half blocks
+    u4 a[AHEAD][MT], b[AHEAD][NT];
+    auto load = [&](int c, u4 (&a)[MT], u4 (&b)[NT]) {
+        const int2 e = table[4 * c + half];
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) b[nt] = as_b8(wb[((int64_t)c * nts + nt) * 64]);
+        for (int nt = 0; nt < NT; ++nt) b[nt] = wb[((int64_t)c * nts + nt) * 64];
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
             const uint32_t o = (mask[m] >> e.y) & 1u ? at[m] + (uint32_t)e.x : 0xFFFFFFF0u;
-            a[m] = as_b8(__builtin_bit_cast(u4, __builtin_amdgcn_raw_buffer_load_b128(buf, (int)o, 0, 0)));
+            a[m] = __builtin_bit_cast(u4, __builtin_amdgcn_raw_buffer_load_b128(buf, (int)o, 0, 0));
         }
     };
-    b8 a[MT], b[NT], an[MT], bn[NT];
-    load(first, a, b);  // 14 steps at least
-    for (int c = first; c < chunks; c += KS) {
-        load(min(c + KS, chunks - 1), an, bn);  // the next step's, before this one's products
+#pragma unroll
+    for (int s = 0; s < AHEAD; ++s) load(s, a[s], b[s]);  // 14 steps at least
+    auto products = [&](const u4 (&a)[MT], const u4 (&b)[NT]) {
+        u2 block[2][MT];
 #pragma unroll
         for (int m = 0; m < MT; ++m)
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt)
-                acc[m][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[m], b[nt], acc[m][nt], 0, 0, 0);
+            for (int w = 0; w < 2; ++w) {  // lane groups 1, 3 of the lower half for 0, 2 of the upper
+                const auto r = __builtin_amdgcn_permlane16_swap(a[m][w], a[m][w + 2], false, false);
+                block[0][m][w] = r[0];
+                block[1][m][w] = r[1];
+            }
 #pragma unroll
-        for (int m = 0; m < MT; ++m) a[m] = an[m];
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) b[nt] = bn[nt];
-    }
-    if constexpr (KS > 1) {  // the shares' sums, in order
-        static_assert(KS == 4, "a workgroup's waves share one tile");
-        __shared__ f4 part[KS - 1][MT * NT][64];
-        if (wave > 0) {
+        for (int h = 0; h < 2; ++h)
 #pragma unroll
             for (int m = 0; m < MT; ++m)
 #pragma unroll
-                for (int nt = 0; nt < NT; ++nt) part[wave - 1][m * NT + nt][l] = acc[m][nt];
+                for (int nt = 0; nt < NT; ++nt)
+                    acc[m][nt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(
+                        as_s4(block[h][m]), as_s4(u2{b[nt][2 * h], b[nt][2 * h + 1]}), acc[m][nt], 0, 0, 0);
+    };
+    int c = 0;
+    for (; c + AHEAD <= chunks; c += AHEAD) {
+#pragma unroll
+        for (int s = 0; s < AHEAD; ++s) {
+            products(a[s], b[s]);
+            load(min(c + s + AHEAD, chunks - 1), a[s], b[s]);
         }
-        __syncthreads();
-        if (wave > 0) return;
-#pragma unroll
-        for (int q = 0; q < KS - 1; ++q)
-#pragma unroll
-            for (int m = 0; m < MT; ++m)
-#pragma unroll
-                for (int nt = 0; nt < NT; ++nt) acc[m][nt] += part[q][m * NT + nt][l];
     }
+#pragma unroll
+    for (int s = 0; s < AHEAD - 1; ++s)
+        if (c + s < chunks) products(a[s], b[s]);
 #pragma unroll
     for (int m = 0; m < MT; ++m)
 #pragma unroll
@@ -177,15 +187,16 @@ __global__ __launch_bounds__(256) void k_conv(Lv d, const uint16_t* __restrict__
 }
 
 // Packed BF16 weights: forward [chunk][nt][lane][j] = W[t][ci][16 nt + lane % 16],
-// (t, ci) = pair 32 chunk + 8 (lane / 16) + j of the 27 cin, zero past the end;
+// t = q / (cin / 16), ci = 16 (q % (cin / 16)) + 4 (lane / 16) + j % 4 for block
+// q = 2 chunk + j / 4 of the 27 cin / 16, zero past the end;
 // backward data (cin' = cout, cout' = cin): W'[t][a][b] = W[26 - t][b][a], packed the same way.
 __device__ inline void packed_place(int64_t i, int cin, int cout, int& t, int& ci, int& co) {
     const int j = (int)(i & 7), l = (int)(i >> 3) & 63, NT = cout / 16;
     const int64_t r = i >> 9;
     const int c = (int)(r / NT), nt = (int)(r - (int64_t)c * NT);
-    const int k = 32 * c + 8 * (l >> 4) + j;
-    t = k / cin;
-    ci = k - t * cin;
+    const int q = 2 * c + (j >> 2), kcs = cin / 16;
+    t = q / kcs;
+    ci = 16 * (q - t * kcs) + 4 * (l >> 4) + (j & 3);
     co = 16 * nt + (l & 15);
 }
 
@@ -752,41 +763,34 @@ __global__ __launch_bounds__(256) void k_zero_f(int64_t n, float* __restrict__ a
 // ---------------------------------------------------------------------------
 // Host drivers
 // ---------------------------------------------------------------------------
-template <int MT, int NT, int KS>
+template <int MT, int NT, int AHEAD>
 hipError_t launch_conv_tile(hipStream_t st, const Lv& d, const uint16_t* X, int cin, int cout, const uint16_t* wp,
                             const float* bias, int relu, uint16_t* ybf, float* yf) {
-    const int64_t voxels = 16 * MT * (4 / KS);  // per workgroup
-    const dim3 grid((unsigned)((d.V + voxels - 1) / voxels), (unsigned)(cout / 16 / NT));
-    hipLaunchKernelGGL((k_conv<MT, NT, KS>), grid, dim3(256), 0, st, d, X, cin, cout, reinterpret_cast<const u4*>(wp),
-                       bias, relu, ybf, yf);
+    const dim3 grid((unsigned)((d.V + 64 * MT - 1) / (64 * MT)), (unsigned)(cout / 16 / NT));
+    hipLaunchKernelGGL((k_conv<MT, NT, AHEAD>), grid, dim3(256), 0, st, d, X, cin, cout,
+                       reinterpret_cast<const u4*>(wp), bias, relu, ybf, yf);
     return hipGetLastError();
 }
 
-// Large tiles as long as they leave every SIMD a wave or two (1024 SIMDs).
-// Below, a workgroup's wavefronts share a tile, and the smallest levels take
-// the most workgroups: single tiles, an output group each.  From five output
-// groups on the sums' LDS and their one wavefront cost more than the sharing
-// saves (32 -> 80 channels on 61 440 voxels: 38 us for 30).  Loss and gradients
-// with a wavefront per tile / with shared tiles: 16^3 540 / 480 us, 32x40x32
-// 673 / 564, 64^3 1079 / 970, 64x96x80 1484 / 1397.
+// Two tiles a wavefront as long as they leave every SIMD one (1024 SIMDs); the
+// smallest levels take the most wavefronts, single tiles of an output group
+// each.  At 64x96x80, us per launch on the finest level (48 -> 16, 16 -> 48):
+// two tiles 92, 64, four 95, 83 (their registers leave fewer waves); 61 440
+// voxels (32 -> 32): two 34, one 39.  Steps ahead: two 92, 64, 34; one 101, 62,
+// 37; four with two tiles the same as two; single tiles of 7680 voxels (112 ->
+// 48 channels) six 18.8, four 19.2.
 hipError_t launch_conv(hipStream_t st, const Lv& d, const uint16_t* X, int cin, int cout, const uint16_t* wp,
                        const float* bias, int relu, uint16_t* ybf, float* yf) {
-    const int mt = d.V >= 64 * 2048 ? 4 : (d.V >= 32 * 1024 ? 2 : 1);
-    if (mt == 1) return launch_conv_tile<1, 1, 4>(st, d, X, cin, cout, wp, bias, relu, ybf, yf);
-#define FE_CONV(NT)                                                                                        \
-    case NT:                                                                                               \
-        return mt == 4 ? launch_conv_tile<4, NT, 1>(st, d, X, cin, cout, wp, bias, relu, ybf, yf)             \
-                       : launch_conv_tile<2, NT, (NT < 5 ? 4 : 1)>(st, d, X, cin, cout, wp, bias, relu, ybf, yf)
+    if (d.V < 32 * 1024) return launch_conv_tile<1, 1, 6>(st, d, X, cin, cout, wp, bias, relu, ybf, yf);
     switch (cout / 16) {
-        FE_CONV(1);
-        FE_CONV(2);
-        FE_CONV(3);
-        FE_CONV(4);
-        FE_CONV(5);
-        FE_CONV(7);
+        case 1: return launch_conv_tile<2, 1, 2>(st, d, X, cin, cout, wp, bias, relu, ybf, yf);
+        case 2: return launch_conv_tile<2, 2, 2>(st, d, X, cin, cout, wp, bias, relu, ybf, yf);
+        case 3: return launch_conv_tile<2, 3, 2>(st, d, X, cin, cout, wp, bias, relu, ybf, yf);
+        case 4: return launch_conv_tile<2, 4, 2>(st, d, X, cin, cout, wp, bias, relu, ybf, yf);
+        case 5: return launch_conv_tile<2, 5, 2>(st, d, X, cin, cout, wp, bias, relu, ybf, yf);
+        case 7: return launch_conv_tile<2, 7, 2>(st, d, X, cin, cout, wp, bias, relu, ybf, yf);
         default: return hipErrorInvalidValue;
     }
-#undef FE_CONV
 }
 
 // Workgroups along the voxels: about 16 waves per CU in all, and a few steps

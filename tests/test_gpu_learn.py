@@ -79,9 +79,31 @@ def test_gradients_on_ragged_levels(ctx, shape):
 
 @pytest.mark.parametrize("shape", [(32, 32, 40), (64, 64, 64)])
 def test_gradients_on_every_convolution_tile(ctx, shape):
-    """Levels on 16, 32 and 64 voxels a wavefront (below 32 768 cells, below
-    131 072, above), their last tiles partly filled; bounds as above."""
+    """Levels on 16 and 32 voxels a wavefront (below 32 768 cells and above),
+    their last tiles partly filled; bounds as above."""
     test_forward_backward_matches_restatement(ctx, shape, "mse")
+
+
+def test_prediction_is_the_same_on_every_tile(ctx):
+    """The same field, a multiple of the coarsest cell in period, on a taller
+    grid: the finest level (30 720, 73 728 and 294 912 voxels) and the next
+    (36 864 on the tallest) on 16 and 32 voxels a wavefront.  Every sum is one
+    chain over the taps and channels whatever the tile, so the voxels that the
+    upper boundary cannot reach (it reaches 22 layers by the taps at their
+    levels' spacings and the rest of the pooling's blocks, 32 at most) agree
+    bit for bit."""
+    ny, nx = 32, 24
+    rng = np.random.default_rng(12)
+    unit = rng.normal(size=(8, ny, nx)).astype(np.float32)
+    mark = rng.choice([0, 1, 1, 1, 2], size=(8, ny, nx)).astype(np.uint8)
+    net = capi.Net(ctx, seed=3)
+    pred = []
+    for nz in (40, 96, 384):
+        b, flags = np.tile(unit, (nz // 8, 1, 1)), np.tile(mark, (nz // 8, 1, 1))
+        pred.append(net.loss_and_grads(b, flags, b)[2])
+    assert np.abs(pred[0]).max() > 0
+    assert np.array_equal(pred[0][:8], pred[1][:8]) and np.array_equal(pred[1][:64], pred[2][:64])
+    net.close()
 
 
 def _dam_scene(ctx, n, box_hi, seed=0):
