@@ -21,6 +21,7 @@ namespace fe {
 
 constexpr int kNetLayers = 7;  // enc0..enc3, dec2, dec1, dec0
 constexpr int kNetIn = 16;     // input channels (3 used)
+constexpr int64_t kNetMaxVoxels = 0xFFFFFFFFll / 48;  // the finest level's widest array has 48 channels: 32-bit indices
 constexpr int kNetLayerIn[kNetLayers] = {16, 16, 32, 48, 112, 80, 48};
 constexpr int kNetLayerOut[kNetLayers] = {16, 32, 48, 64, 48, 32, 16};
 constexpr int kNetLayerLevel[kNetLayers] = {0, 1, 2, 3, 2, 1, 0};

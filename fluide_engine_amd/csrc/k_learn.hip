@@ -79,7 +79,11 @@ __device__ inline s4 as_s4(const u2& w) { return __builtin_bit_cast(s4, w); }
 __host__ __device__ inline int conv_chunks(int cin) { return (27 * cin + 31) / 32; }
 constexpr int kMaxCh = 112;
 constexpr int kMaxChunks = (27 * kMaxCh + 31) / 32;
-constexpr uint32_t kConvReach = 0x7FFFFFFFu;  // bytes a load may reach from its wave's base
+// Bytes a load may reach from its wave's base, below the offset that stands for
+// outside.  A wave's taps lie within 2 (nx ny + nx + 1) + 16 MT voxels of 96
+// bytes at most on the finest level, 2.42e9 bytes on the largest grid
+// (kNetMaxVoxels on the least 8 planes of 8 rows), a quarter of that below.
+constexpr uint32_t kConvReach = 0xFFFFFFE0u;
 
 template <int MT, int NT, int AHEAD>
 __global__ __launch_bounds__(256) void k_conv(Lv d, const uint16_t* __restrict__ X, int cin, int cout,
@@ -101,8 +105,9 @@ __global__ __launch_bounds__(256) void k_conv(Lv d, const uint16_t* __restrict__
     const int64_t reach = (int64_t)d.nx * d.ny + d.nx + 1;
     const int64_t vb = v0 > reach ? v0 - reach : 0;
     const int64_t bytes = (d.V - vb) * cin * 2;
-    const __amdgpu_buffer_rsrc_t buf = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint16_t*>(X + vb * cin), 0, (int)(bytes < (int64_t)kConvReach ? bytes : (int64_t)kConvReach), 0x00020000);
+    const __amdgpu_buffer_rsrc_t buf =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(X + vb * cin), 0,
+                                          (int)(uint32_t)min(bytes, (int64_t)kConvReach), 0x00020000);
     // per tile: which of the 27 taps lie inside the grid, and the voxel's offset
     uint32_t mask[MT], at[MT];
 #pragma unroll
@@ -468,8 +473,7 @@ __global__ __launch_bounds__(256) void k_features(int64_t V, const float* __rest
 // divisions by constants: the concatenation at 64x96x80 takes 12 us (63 MB, the
 // rate of a copy) where one channel per thread behind 64-bit divisions took 68,
 // the seven passes of a gradient 65 us for 175.  A level's groups, 6 per finest
-// voxel at most, stay below 2^32: a network keeps some 800 bytes per voxel, so
-// 288 GB hold below 2^29.
+// voxel at most, stay below 2^32 (kNetMaxVoxels).
 template <int GROUPS>
 __device__ inline bool group_of(int64_t V, uint32_t& v, uint32_t& g) {
     const uint32_t i = blockIdx.x * 256u + threadIdx.x;
@@ -987,6 +991,7 @@ hipError_t net_set_params(fe_net* n, const float* host) {
 
 hipError_t net_ensure(fe_net* n, const int nn[3]) {
     if (n->lv[0].n[0] == nn[0] && n->lv[0].n[1] == nn[1] && n->lv[0].n[2] == nn[2] && n->X0) return hipSuccess;
+    if ((int64_t)nn[0] * nn[1] * nn[2] > kNetMaxVoxels) return hipErrorInvalidConfiguration;
     (void)hipStreamSynchronize(n->stream);
     free_buffers(n);
     for (int l = 0; l < 4; ++l) {

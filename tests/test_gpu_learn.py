@@ -106,6 +106,32 @@ def test_prediction_is_the_same_on_every_tile(ctx):
     net.close()
 
 
+def test_planes_of_eleven_million_voxels(ctx):
+    """The widest planes the network takes (3344 x 3344 on 8 planes, a tap one
+    plane up 1.07e9 bytes away): away from the boundaries a field of period 16
+    is predicted as on a 240 x 240 grid, bit for bit (values of a few binary
+    digits, so both sums of squares are exact).  Above 2^32 / 48 voxels the
+    call is refused."""
+    print("[gpu] net on 8 x 3344 x 3344", flush=True)
+    rng = np.random.default_rng(4)
+    unit = (rng.integers(-16, 17, size=(8, 16, 16)) / 8).astype(np.float32)
+    mark = rng.choice([0, 1, 1, 1, 2], size=unit.shape).astype(np.uint8)
+    net = capi.Net(ctx, seed=3)
+    tiles = []
+    for q in (15, 209):
+        b, flags = np.tile(unit, (1, q, q)), np.tile(mark, (1, q, q))
+        pred = net.loss_and_grads(b, flags, b)[2]
+        tiles.append(pred.reshape(8, q, 16, q, 16)[:, 3:-3, :, 3:-3])
+    want = tiles[0][:, :1, :, :1]
+    assert np.abs(want).max() > 0
+    assert np.array_equal(tiles[0], np.broadcast_to(want, tiles[0].shape))
+    assert np.array_equal(tiles[1], np.broadcast_to(want, tiles[1].shape))
+    with pytest.raises(capi.FluideError):
+        b = np.zeros((8, 3352, 3352), np.float32)
+        net.loss_and_grads(b, np.zeros(b.shape, np.uint8), b)
+    net.close()
+
+
 def _dam_scene(ctx, n, box_hi, seed=0):
     desc = capi.scene_desc((n, n, n), method=capi.FLIP, blend=0.03, max_particles=8 * n ** 3)
     x = capi.seed_particles(desc, [capi.box((-1, -1, -1), box_hi)], seed=seed)
