@@ -230,8 +230,7 @@ __global__ __launch_bounds__(kBlock) void k_sdf_extrapolate(Geom g, double* __re
 // triangle.  A term atan2(om, k) is the argument of k + i om, so the terms are
 // multiplied as complex numbers (4 operations instead of an atan2 each), with
 // the whole turns counted where a product passes the negative real axis, and
-// one atan2 at the end.  The three lengths in k come from the hardware's
-// reciprocal square root and one Newton step (relative error below 1e-14).
+// one atan2 at the end.
 // The waves of a workgroup take the same 64 nodes and a slice of the
 // triangles each; the loop index is uniform in a wave, so vertices and index
 // boxes are scalar loads, and a box that no node of the wave is in costs no
@@ -321,13 +320,17 @@ __device__ inline double triangle_distance(const D3& x, const D3& p0, const D3& 
     return dlen(dsub(c, x));
 }
 
-// |a| from the square s of a length: 0 gives 1e-150, not 0 (the caller sees a
-// vanishing product).
-__device__ inline double quick_length(double s) {
-    s = fmax(s, 1e-300);
-    const double y = __builtin_amdgcn_rsq(s);
-    const double n = s * y;
-    return fma(0.5 * y, fma(-n, n, s), n);
+// High words of 2^-664 and 2^664, about 1e-200 and 1e200.
+constexpr int kSqrtFrom = (1023 - 664) << 20, kSqrtTo = (1023 + 664) << 20;
+
+// The square root to FP64's last bit between these: the hardware's
+// reciprocal root, one step of Goldschmidt's iteration on the root and half its
+// reciprocal (relative errors below 1e-13), and the root's residual, which
+// leaves 1e-26 to the final rounding.
+__device__ inline double plain_sqrt(double s) {
+    const double y = __builtin_amdgcn_rsq(s), g = s * y, h = 0.5 * y, r = fma(-h, g, 0.5);
+    const double g1 = fma(g, r, g), h1 = fma(h, r, h);
+    return fma(fma(-g1, g1, s), h1, g1);
 }
 
 // A sum of angles as a complex number of that argument (scaled at will) and
@@ -366,7 +369,14 @@ __device__ inline void add_half_solid_angle(AngleSum& z, const D3& x, const D3& 
     omega -= B.x * A.y * C.z;
     omega -= A.x * C.y * B.z;
     auto dot = [](const D3& a, const D3& b) { return fma(a.z, b.z, fma(a.y, b.y, a.x * b.x)); };
-    const double nA = quick_length(dot(A, A)), nB = quick_length(dot(B, B)), nC = quick_length(dot(C, C));
+    const double qA = dot(A, A), qB = dot(B, B), qC = dot(C, C);
+    double nA = plain_sqrt(qA), nB = plain_sqrt(qB), nC = plain_sqrt(qC);
+    const int eA = __double2hiint(qA), eB = __double2hiint(qB), eC = __double2hiint(qC);
+    if (min(min(eA, eB), eC) < kSqrtFrom || max(max(eA, eB), eC) > kSqrtTo) {
+        nA = sqrt(qA);
+        nB = sqrt(qB);
+        nC = sqrt(qC);
+    }
     const double n3 = nA * nB * nC;
     double k = fma(nB, dot(C, A), fma(nA, dot(B, C), fma(nC, dot(A, B), n3)));
     if (fabs(omega) + fabs(k) <= 1e-9 * n3) {
@@ -385,7 +395,8 @@ constexpr double kPi = 3.14159265358979323846;  // src/common/math_utils.hpp:11
 
 // Bound by FP64 instructions: with an atan2 and three square roots per node
 // and triangle 64^3 nodes for a mesh of 1472 triangles took 2.86 ms for the whole call,
-// with the complex product 1.34 ms.
+// with the complex product and lengths by plain_sqrt 1.48 ms (by sqrt, which
+// scales its argument on every call, 1.85).
 // tv: 9 doubles per triangle (its three vertices); tb: 6 ints per triangle,
 // the index box i0, j0, k0, i1, j1, k1 (inclusive).
 template <int SLICES>
