@@ -634,8 +634,8 @@ int fe_scene_create(fe_ctx* ctx, const fe_scene_desc* d, fe_scene** out) {
     chk(dalloc(&s->d[1], nc));
     chk(dalloc(&s->q, nc));
     chk(dalloc(&s->q2, nc));
-    // CG: 4 + 4 partials per block; with multigrid 2 + 2 and r.z of the V-cycle
-    s->npartials = solver_shape_n(nc).blocks * 8;
+    // CG: 5 + 5 partials per block; with multigrid 2 + 2 and r.z of the V-cycle
+    s->npartials = solver_shape_n(nc).blocks * 10;
     chk(dalloc(&s->partials, s->npartials));
     chk(dalloc(&s->chunk_fluid, solver_shape_n(nc).blocks));
     chk(dalloc(&s->sc, 2));  // two state slots (CG alternates them)

@@ -240,6 +240,9 @@ __device__ inline Stencil64In stencil64_in(int64_t c, const uint16_t* __restrict
 // ||r|| and beta stays meaningful across recomputations.
 // ---------------------------------------------------------------------------
 constexpr double kReliableDrop2 = 1e-4;  // (100x in ||r||)^2
+// Sums per block without multigrid: r.r, d.q, q.M^-1 q, q.z and, where z is not
+// r itself, r.z.
+constexpr int cg_sums(bool diag) { return diag ? 5 : 4; }
 __global__ __launch_bounds__(kBlock) void k_cg_init(Geom g, const uint16_t* __restrict__ code,
                                                     const float* __restrict__ b, double* __restrict__ x,
                                                     float* __restrict__ r, float* __restrict__ d0, float* __restrict__ mgx, SolverScalars* sc,
@@ -287,10 +290,15 @@ __global__ __launch_bounds__(kBlock) void k_cg_init(Geom g, const uint16_t* __re
     span_groups_from<G, Stencil64In>(
         early ? g0 + (int64_t)G * kBlock : g0, sp.c1, [&](int64_t c) { return stencil64_in(c, code, x, b, st); },
         use);
-    if (stride == 2)
+    if (stride == 2) {
         write_partials<2>(v, pout);
-    else
-        write_partials<2, 4>(v, pout);
+    } else if (stride == cg_sums(false)) {
+        const double w[1] = {v[1]};
+        write_partials<1, cg_sums(false)>(w, pout);
+    } else {
+        const double w[cg_sums(true)] = {v[1], 0.0, 0.0, 0.0, v[0]};
+        write_partials<cg_sums(true)>(w, pout);
+    }
 }
 
 // The CG kernels' prologue: every block derives the iteration's scalars from the
@@ -523,12 +531,15 @@ __global__ __launch_bounds__(kBlock) void k_cg_update(Geom g, const uint16_t* __
 //   alpha = sigma / d.q,  r' = r - alpha q,  x' = x + alpha d (FP64),
 //   d' = z' + beta d,  q' = A d',
 // with r', z' and d' formed at the six neighbours too.  beta = sigma' / sigma
-// would need r'.z' before d' exists; by conjugacy (q.z = q.d) it is
-// alpha^2 q.M^-1 q - sigma, which the launch before has summed.  Only beta
-// takes that value: alpha and every test use the r.z and r.r summed from r
-// itself.  Where it is not positive (all rounding), and where the residual is
-// recomputed, the iteration takes two launches: r' = b - A x' with x', then
-// d' and q' with the sums of that r'.
+// needs sigma' = r'.z' before d' exists: r' being r - alpha q, it is sigma -
+// 2 alpha q.z + alpha^2 q.M^-1 q, of sums that the launch before has left.
+// That is r'.z' but for the FP32 roundings of r' and z', 1e-9 of it, which the
+// rounding of beta to FP32 for d' (6e-8) covers; with q.d in the place of q.z,
+// equal to it by conjugacy, beta would be off by 1e-6, as the vectors in FP32
+// are.  Only beta takes that value: alpha and every test use the r.z and r.r
+// summed from r itself.  Where it is not positive (all rounding), and where the
+// residual is recomputed, the iteration takes two launches: r' = b - A x' with
+// x', then d' and q' with the sums of that r'.
 //
 // Bound by latency on all but large grids: the launch, one round of loads, the
 // partial sums, the state, the block's sums.  An iteration of 190 k cells in
@@ -553,6 +564,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_step(Geom g, const uint16_t* __re
                                                     double* __restrict__ pout, int nparts, float ihx2, float ihy2,
                                                     float ihz2, const uint8_t* __restrict__ cfl, int64_t chunk,
                                                     int64_t padded) {
+    constexpr int NS = cg_sums(DIAG);
     const int64_t nc = cell_count(g);
     const Span sp = block_span(nc, chunk, padded);
     const Stride st = stride_of(g.n[0], g.n[1], g.n[2]);
@@ -582,12 +594,12 @@ __global__ __launch_bounds__(kBlock) void k_cg_step(Geom g, const uint16_t* __re
 #pragma unroll
         for (int u = 0; u < G; ++u) raw[u] = fetch(min(g0 + (int64_t)u * kBlock, sp.c1 - 1));
     }
-    __shared__ double sm[4][kBlock / 64];
+    __shared__ double sm[NS][kBlock / 64];
     __shared__ double plan_alpha, plan_beta;
     __shared__ int plan_done, plan_only_d, plan_only_r;
     {
-        double t[4] = {0.0, 0.0, 0.0, 0.0};  // r.z, r.r, d.q, q.M^-1 q of the read buffers
-        add_partials<4, 4>(pin, 4, 0, (int)threadIdx.x, kBlock, nparts, t);
+        double t[NS] = {};
+        add_partials<NS, 4>(pin, NS, 0, (int)threadIdx.x, kBlock, nparts, t);
         wave_sums(t, sm);
     }
     __syncthreads();
@@ -599,8 +611,8 @@ __global__ __launch_bounds__(kBlock) void k_cg_step(Geom g, const uint16_t* __re
             const bool first = o.it < 0, replaced = phase == kHaveR;
             if (phase != kHaveAllSummed) {
                 o.sigma_old = sold;
-                o.sigma = waves_total(sm[0]);
-                o.rr = waves_total(sm[1]);
+                o.rr = waves_total(sm[0]);
+                o.sigma = DIAG ? waves_total(sm[NS - 1]) : o.rr;
                 o.confirm = 0;
                 bool stop = stop_rule(in, o.bnorm2, o.sigma, o.rr);
                 if (first) {  // the sums are k_cg_init's
@@ -624,9 +636,10 @@ __global__ __launch_bounds__(kBlock) void k_cg_step(Geom g, const uint16_t* __re
             if (phase == kHaveR) {
                 o.beta = first ? 0.0 : o.sigma / sold;
             } else {
-                o.dq = waves_total(sm[2]);
+                o.dq = waves_total(sm[1]);
                 o.alpha = o.sigma / o.dq;
-                o.beta = (o.alpha * o.alpha * waves_total(sm[3]) - o.sigma) / o.sigma;
+                const double fa = (double)(float)o.alpha;  // as r' takes it
+                o.beta = (o.sigma - 2.0 * fa * waves_total(sm[3]) + fa * fa * waves_total(sm[2])) / o.sigma;
                 if (!(o.beta > 0.0)) o.replace = 1;
             }
             o.phase = phase == kHaveR ? kHaveAllSummed : (o.replace ? kHaveR : kHaveAll);
@@ -647,26 +660,27 @@ __global__ __launch_bounds__(kBlock) void k_cg_step(Geom g, const uint16_t* __re
     const double alpha = plan_alpha, beta = plan_beta;
     const bool only_d = plan_only_d != 0, only_r = plan_only_r != 0;
     if (!body) {  // no FLUID cell: every vector stays 0
-        if (threadIdx.x < 4) pout[4 * (int64_t)blockIdx.x + threadIdx.x] = 0.0;
+        if (threadIdx.x < NS) pout[NS * (int64_t)blockIdx.x + threadIdx.x] = 0.0;
         return;
     }
     const float ih2[3] = {ihx2, ihy2, ihz2};
     const double ih2d[3] = {ihx2, ihy2, ihz2};
     const float fa = (float)alpha, fb = (float)beta;
-    double v[4] = {0.0, 0.0, 0.0, 0.0};
+    double v[NS] = {};
     auto precond = [&](float r, uint16_t cd) { return DIAG ? r / code_center(cd, ih2) : r; };
-    auto direction = [&](int64_t c, uint16_t cd, float dc, const float (&nb)[6]) {
+    auto direction = [&](int64_t c, uint16_t cd, float zc, float dc, const float (&nb)[6]) {
         const float center = code_center(cd, ih2);
         const float qc = code_apply_nb(cd, center, ih2, dc, nb);
         B.dn[c] = dc;
         B.qo[c] = qc;
-        v[2] += (double)dc * (double)qc;
-        v[3] += (double)qc * (double)(DIAG ? qc / center : qc);
+        v[1] += (double)dc * (double)qc;
+        v[2] += (double)qc * (double)(DIAG ? qc / center : qc);
+        v[3] += (double)qc * (double)zc;
     };
-    auto residual = [&](int64_t c, uint16_t cd, float rc) {
+    auto residual = [&](int64_t c, float rc, float zc) {
         B.ro[c] = rc;
-        v[0] += (double)rc * (double)precond(rc, cd);
-        v[1] += (double)rc * (double)rc;
+        v[0] += (double)rc * (double)rc;
+        if constexpr (DIAG) v[NS - 1] += (double)rc * (double)zc;
     };
     auto use = [&](int64_t c, const Raw& w) {
         float nb[6];
@@ -675,28 +689,30 @@ __global__ __launch_bounds__(kBlock) void k_cg_step(Geom g, const uint16_t* __re
             const double xc = alpha * (double)w.d + w.x;
             B.xo[c] = xc;
             B.dn[c] = w.d;
-            residual(c, w.cd, (float)((double)b[c] - code_apply64(w.cd, c, st, ih2d, xc, X)));
+            const float rc = (float)((double)b[c] - code_apply64(w.cd, c, st, ih2d, xc, X));
+            residual(c, rc, precond(rc, w.cd));
         } else if (only_d) {
             B.xo[c] = w.x;
             B.ro[c] = w.r;
 #pragma unroll
             for (int k = 0; k < 6; ++k) nb[k] = fmaf(fb, w.dn[k], precond(w.rn[k], w.cn[DIAG ? k : 0]));
-            direction(c, w.cd, fmaf(fb, w.d, precond(w.r, w.cd)), nb);
+            const float zc = precond(w.r, w.cd);
+            direction(c, w.cd, zc, fmaf(fb, w.d, zc), nb);
         } else {
             B.xo[c] = alpha * (double)w.d + w.x;
-            const float rc = fmaf(-fa, w.q, w.r);
-            residual(c, w.cd, rc);
+            const float rc = fmaf(-fa, w.q, w.r), zc = precond(rc, w.cd);
+            residual(c, rc, zc);
 #pragma unroll
             for (int k = 0; k < 6; ++k)
                 nb[k] = fmaf(fb, w.dn[k], precond(fmaf(-fa, w.qn[k], w.rn[k]), w.cn[DIAG ? k : 0]));
-            direction(c, w.cd, fmaf(fb, w.d, precond(rc, w.cd)), nb);
+            direction(c, w.cd, zc, fmaf(fb, w.d, zc), nb);
         }
     };
 #pragma unroll
     for (int u = 0; u < G; ++u)
         if (g0 + (int64_t)u * kBlock < sp.c1) use(g0 + (int64_t)u * kBlock, raw[u]);
     for (int64_t c = g0 + (int64_t)G * kBlock; c < sp.c1; c += kBlock) use(c, fetch(c));
-    write_partials<4>(v, pout);
+    write_partials<NS>(v, pout);
 }
 
 // Final ||b - A p||^2 and ||b||^2 in FP64 on the FP64 solution, with FP64
@@ -895,8 +911,8 @@ static CGSetup cg_setup(fe_scene* s, int precond) {
     c.g = s->g;
     c.sh = solver_shape(s->g);
     c.nparts = (int)c.sh.blocks;
-    c.PA = s->partials;                  // 2 per block
-    c.PB = s->partials + (precond == 2 ? 2 : 4) * c.sh.blocks;  // 2 per block (without multigrid 4)
+    c.PA = s->partials;                    // 2 per block, without multigrid cg_sums
+    c.PB = s->partials + (precond == 2 ? 2 : cg_sums(precond == 1)) * c.sh.blocks;  // as many
     c.PZ = s->partials + 4 * c.sh.blocks;  // r.z of the V-cycle, 1 per block
     // BuildSystem's invH * invH (single_phase_pressure_solver.cpp:102-103); exact
     // in FP32 for power-of-two spacings
@@ -986,8 +1002,8 @@ static hipError_t cg_start(fe_scene* s, const CGSetup& c, CGRun& R) {
     zero_add(L, s->p2, 8 * nc);
     hipLaunchKernelGGL(k_zero_many, dim3((unsigned)L.first[L.n]), dim3(kBlock), 0, s->stream, L);
     hipLaunchKernelGGL(k_cg_init, dim3((unsigned)c.sh.blocks), dim3(kBlock), 0, s->stream, c.g, s->code, s->b, s->p,
-                       s->r, s->d[0], c.mgx, s->sc, c.PA, c.PB, c.mg ? 2 : 4, c.nparts, c.ih2[0], c.ih2[1], c.ih2[2],
-                       c.sh.chunk, c.sh.blocks);
+                       s->r, s->d[0], c.mgx, s->sc, c.PA, c.PB, c.mg ? 2 : cg_sums(c.precond == 1), c.nparts, c.ih2[0],
+                       c.ih2[1], c.ih2[2], c.sh.chunk, c.sh.blocks);
     if (c.mg && (e = mg_apply(s, s->r, s->z, s->sc, c.PZ, -1, nullptr, 0)) != hipSuccess) return e;
     R = CGRun{};
     R.xa = s->p;
