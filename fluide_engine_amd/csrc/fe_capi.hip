@@ -301,11 +301,6 @@ bool graph_eligible(const fe_scene* s, const fe_solver_desc* d) {
            s->np > 0 && s->kt_id == FE_KERNEL_NONE && (d->kind != FE_SOLVER_MGPCG || !s->mg.empty());
 }
 
-bool same_solver(const fe_solver_desc& a, const fe_solver_desc& b) {
-    return a.kind == b.kind && a.max_iterations == b.max_iterations && a.check_interval == b.check_interval &&
-           a.relative == b.relative && a.warm_start == b.warm_start && a.tolerance == b.tolerance;
-}
-
 void graph_release(fe::SubstepGraph& G) {
     if (G.a) (void)hipGraphExecDestroy(G.a);
     if (G.b) (void)hipGraphExecDestroy(G.b);

@@ -408,6 +408,11 @@ struct DiffState {
 // ---------------------------------------------------------------------------
 // Host-side scene.
 // ---------------------------------------------------------------------------
+inline bool same_solver(const fe_solver_desc& a, const fe_solver_desc& b) {
+    return a.kind == b.kind && a.max_iterations == b.max_iterations && a.check_interval == b.check_interval &&
+           a.relative == b.relative && a.warm_start == b.warm_start && a.tolerance == b.tolerance;
+}
+
 // The state of a conjugate-gradient solve between its launches (the
 // iterations' buffers rotate with the iteration count).
 struct CGRun {
@@ -563,6 +568,7 @@ struct fe_scene {
     double stage_ms[fe::kMaxStages] = {};
     fe_solve_stats last_stats{};
     int last_cg_launches[2] = {0, 0};  // launches of the last CG solve without and with the diagonal preconditioner
+    fe_solver_desc last_cg_desc[2] = {};  // and its settings
     int last_cg_iters[3] = {0, 0, 0};  // iterations of the last CG solve per preconditioner (none, diagonal, multigrid)
     std::vector<fe::MGLevel> mg;  // multigrid hierarchy, built on first use
     int mg_tail = 0;              // first level handled by the one-workgroup tail kernel

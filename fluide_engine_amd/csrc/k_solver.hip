@@ -1011,17 +1011,39 @@ static hipError_t cg_start(fe_scene* s, const CGSetup& c, CGRun& R) {
     return hipGetLastError();
 }
 
+// Launches of k_cg_step that end any solve: the start's, then at most two an
+// iteration.
+static int cg_step_bound(const fe_solver_desc* d) {
+    return (int)std::min<int64_t>(2 * (int64_t)std::max(d->max_iterations, 0) + 1, 1 << 30);
+}
+
 // Host-driven iterations without multigrid: batches of steps, the host reading
-// the last one's state slot.  first: steps in the first batch.
-static hipError_t cg_step_loop(fe_scene* s, const CGSetup& c, CGRun& R, int first) {
+// the last one's state slot.  expect: launches that the solve may take, from
+// the last one (0: there was none); alike: that had the same settings.
+// Waiting for the device between two batches costs about 30 us, an iteration
+// 6.5 (190 k cells) and a launch after the stop 3.  So a solve like the last
+// takes 512 at a time up to its length, any other at most as many as have run
+// (64 at first) up to there; beyond, or where nothing is known, a batch is a
+// quarter of what has run since.  No batch passes the bound.
+static hipError_t cg_step_loop(fe_scene* s, const fe_solver_desc* d, const CGSetup& c, CGRun& R, int expect,
+                               bool alike) {
     hipError_t e;
-    for (int n = first;; n = std::min(std::max(R.k / 8, 8), 64)) {
-        cg_steps(s, c, R, n);
+    const int bound = cg_step_bound(d);
+    for (;;) {
+        int n;
+        if (R.k < expect)
+            n = std::min(alike ? 512 : std::max(R.k, 64), expect - R.k);
+        else
+            n = std::max((R.k - expect) / 4, R.k > 0 ? 8 : 16);
+        cg_steps(s, c, R, std::max(1, std::min(n, bound - R.k)));
         if ((e = hipGetLastError()) != hipSuccess) return e;
         if ((e = read_scalars(s, R.k & 1)) != hipSuccess) return e;
         kt_flush(s, s->sc_host->done ? s->sc_host->launches - 1 : (1 << 30));
-        if (s->sc_host->done) return hipSuccess;  // the iteration cap ends every solve
+        if (s->sc_host->done) break;  // the iteration cap ends every solve
     }
+    s->last_cg_launches[c.precond] = s->sc_host->launches;
+    s->last_cg_desc[c.precond] = *d;
+    return hipSuccess;
 }
 
 // Host-driven iterations with multigrid: batches of spmv launches, the host
@@ -1066,9 +1088,10 @@ hipError_t launch_pressure_solve(fe_scene* s, const fe_solver_desc* d) {
         const int prev = s->last_cg_iters[2];
         if ((e = cg_host_loop(s, d, c, R, prev > 0 ? std::min(prev + 1, 64) : 4, false)) != hipSuccess) return e;
     } else {
-        int& prev = s->last_cg_launches[init.precond];
-        if ((e = cg_step_loop(s, c, R, prev > 0 ? std::min(prev + 1, 1024) : 16)) != hipSuccess) return e;
-        prev = s->sc_host->launches;
+        const int prev = s->last_cg_launches[c.precond];
+        if ((e = cg_step_loop(s, d, c, R, prev > 0 ? prev + 1 : 0, same_solver(s->last_cg_desc[c.precond], *d))) !=
+            hipSuccess)
+            return e;
         if (s->sc_host->xbuf) R.xa = s->p2;
     }
     if (R.xa != s->p) {
@@ -1119,9 +1142,10 @@ hipError_t finish_pressure_after_head(fe_scene* s, const fe_solver_desc* d, cons
     if (!c.mg) {
         if (!s->sc_host->done) {
             *resumed = true;
-            if ((e = cg_step_loop(s, c, R, 16)) != hipSuccess) return e;
+            if ((e = cg_step_loop(s, d, c, R, R.k, false)) != hipSuccess) return e;
         }
         s->last_cg_launches[c.precond] = s->sc_host->launches;
+        s->last_cg_desc[c.precond] = *d;
         if (s->sc_host->xbuf) R.xa = s->p2;
     } else if (!s->sc_host->done && R.k + 1 <= d->max_iterations) {
         *resumed = true;

@@ -270,6 +270,35 @@ def test_cg_iterates_match_oracle(ctx, kind, shape, cap):
     g.close()
 
 
+@pytest.mark.parametrize("kind", [capi.SOLVER_CG, capi.SOLVER_PCG_JACOBI])
+def test_capped_solve_after_a_long_one(ctx, kind):
+    """A solve of three iterations launches what three iterations can need,
+    whatever the scene's last solve took: as fast after a solve of 2000 as
+    alone (medians, within a factor of 3; a launch for each of the 2000 would
+    be ten times the capped solve)."""
+    import time
+
+    print(f"[gpu] capped solve after a long one kind={kind}", flush=True)
+    g, _ = _pressure_pair(ctx, 32, 5)
+    short = capi.solver(kind, 3, 0, 1e-30, relative=True, warm_start=False)
+    long = capi.solver(kind, 2000, 0, 1e-30, relative=True, warm_start=False)
+
+    def median(before):
+        t = []
+        for _ in range(9):
+            if before:
+                assert g.run_stage(capi.STAGE_PRESSURE, desc=before).iterations == 2000
+            t0 = time.perf_counter()
+            assert g.run_stage(capi.STAGE_PRESSURE, desc=short).iterations == 3
+            t.append(time.perf_counter() - t0)
+        return float(np.median(t))
+
+    alone, after = median(None), median(long)
+    print(f"[gpu]   {alone * 1e6:.0f} us alone, {after * 1e6:.0f} us after", flush=True)
+    assert after < 3 * alone
+    g.close()
+
+
 @pytest.mark.parametrize("n", [48, 64])
 @pytest.mark.parametrize("kind", [capi.SOLVER_MGPCG, capi.SOLVER_CG])
 def test_first_substep_solve_converges(ctx, kind, n):
