@@ -1119,7 +1119,7 @@ hipError_t capture_pressure_head(fe_scene* s, const fe_solver_desc* d, int iters
         slot = (R.k + 1) & 1;
     } else {  // recomputed residuals take a second launch
         const int prev = s->last_cg_launches[c.precond];
-        cg_steps(s, c, R, std::max(2, prev > 0 ? std::min(prev + 2, 1024) : iters));
+        cg_steps(s, c, R, std::min(prev > 0 ? prev + 2 : iters, cg_step_bound(d)));
         slot = R.k & 1;
     }
     if ((e = hipMemcpyAsync(s->sc_host, s->sc + slot, sizeof(SolverScalars), hipMemcpyDeviceToHost, s->stream)) !=

@@ -106,6 +106,37 @@ def test_graph_frames_with_cfl_substeps(ctx):
     g.close()
 
 
+def test_graph_holds_solves_of_any_length(ctx):
+    """A column 1400 cells deep, at rest but for a step too short to move it:
+    CG takes more than 4000 iterations every substep.  A captured solve holds as
+    many launches as the solve before took, so the host does not have to add
+    iterations to every one."""
+    print("[gpu] graph substeps of more than 1024 iterations", flush=True)
+    n, h = (4, 1600, 4), 1.0 / 512
+    out = []
+    for graph in (False, True):
+        desc = capi.scene_desc(n, method=capi.FLIP, blend=0.03, max_particles=8 * 4 * 1600 * 4,
+                               size=tuple(m * h for m in n))
+        x = capi.seed_particles(desc, [capi.box((-1, -1, -1), (1, 1400 * h, 1))], seed=7)
+        sc = capi.Scene(ctx, desc)
+        sc.upload_particles(x, np.zeros_like(x))
+        sc.set_graph(graph)
+        out.append(sc)
+    e, g = out
+    sd = capi.solver(capi.SOLVER_CG, 5000, 0, 1e-6, relative=True, warm_start=False)
+    for step in range(8):
+        se, sg = e.substep(1e-7, sd), g.substep(1e-7, sd)
+        assert se.converged and se.iterations > 1024, se.iterations
+        _same_stats(se, sg, step)
+        _same(e, g, step)
+    n_graph, captures, resumed = g.graph_stats()
+    print(f"[gpu]   iterations {se.iterations}, graph substeps {n_graph}, captures {captures}, resumed {resumed}",
+          flush=True)
+    assert n_graph == 7 and resumed < n_graph
+    e.close()
+    g.close()
+
+
 def test_graph_off_for_viscous_scenes_and_after_disable(ctx):
     print("[gpu] graph mode on a viscous scene, then switched off", flush=True)
     e, g = _pair(ctx, 24, capi.FLIP, viscosity=0.05)
