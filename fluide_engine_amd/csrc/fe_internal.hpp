@@ -403,6 +403,7 @@ struct DiffState {
     int32_t end;             // x_end is its result, once known
     int32_t converged;
     int32_t changed;         // the last checked state differs from the snapshot
+    int32_t nonfinite;       // an identity row's b is not finite, nor is b - x
 };
 
 // ---------------------------------------------------------------------------

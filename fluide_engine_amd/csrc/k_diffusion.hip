@@ -51,11 +51,13 @@ __device__ inline int64_t diff_first(const DiffGrid& D, int c) {
     return lb * (kBlock * kDiffPer);
 }
 
-// Face markers of the three components.
+// Face markers of the three components and the solves' start.
 __global__ __launch_bounds__(kBlock) void k_diff_markers(Geom g, DiffGrid D, const double* __restrict__ sdf,
                                                          const double* __restrict__ csdf, uint8_t* __restrict__ m0,
-                                                         uint8_t* __restrict__ m1, uint8_t* __restrict__ m2) {
+                                                         uint8_t* __restrict__ m1, uint8_t* __restrict__ m2,
+                                                         DiffState* __restrict__ st, DiffState init) {
 #pragma clang fp contract(off)
+    if (blockIdx.x == 0 && threadIdx.x < 3) st[threadIdx.x] = init;
     const int C = diff_component(D, blockIdx.x);
     uint8_t* mark = C == 0 ? m0 : (C == 1 ? m1 : m2);
     const int64_t f0 = diff_first(D, C) + threadIdx.x;
@@ -78,15 +80,14 @@ __global__ __launch_bounds__(kBlock) void k_diff_markers(Geom g, DiffGrid D, con
 }
 
 // Row codes, right-hand sides and x0 = u, into both iterates: an identity row
-// has the solution b = u, so no sweep needs to visit it.
+// has the solution b = u, so no sweep needs to visit it, and the residual 0, or
+// none that any tolerance meets where u is not finite.
 __global__ __launch_bounds__(kBlock) void k_diff_build(DiffGrid D, FaceSet uu, const uint8_t* __restrict__ m0,
                                                        const uint8_t* __restrict__ m1, const uint8_t* __restrict__ m2,
                                                        uint16_t* __restrict__ code, double* __restrict__ x0,
                                                        double* __restrict__ x1, double* __restrict__ b, double cx,
-                                                       double cy, double cz, DiffState* __restrict__ st,
-                                                       DiffState init) {
+                                                       double cy, double cz, DiffState* __restrict__ st) {
 #pragma clang fp contract(off)
-    if (blockIdx.x == 0 && threadIdx.x < 3) st[threadIdx.x] = init;
     const int C = diff_component(D, blockIdx.x);
     const uint8_t* __restrict__ mark = C == 0 ? m0 : (C == 1 ? m1 : m2);
     const float* __restrict__ u = uu.a[C];
@@ -125,6 +126,8 @@ __global__ __launch_bounds__(kBlock) void k_diff_build(DiffGrid D, FaceSet uu, c
                 const int q = order[t];
                 if (in[q] && mark[nb[q]] == FE_BOUNDRY) bb += c[q >> 1] * (double)u[nb[q]];
             }
+        } else if (!(bb - bb == 0.0)) {
+            st[C].nonfinite = 1;  // every writer writes the same
         }
         code[o] = cd;
         b[o] = bb;
@@ -252,6 +255,7 @@ __global__ __launch_bounds__(kBlock) void k_diff_check(DiffGrid D, const double*
     sum_partials<1>(part + D.blk[C], (int)(D.blk[C + 1] - D.blk[C]), t);
     if (threadIdx.x != 0) return;
     const int k = q * interval + 1;  // the state checked
+    if (S->nonfinite) t[0] = __builtin_nan("");
     S->rr = t[0];
     S->ring[q % kDiffRing] = t[0];
     if (sqrt(t[0]) < S->tol) {
@@ -349,16 +353,17 @@ hipError_t launch_diffusion(fe_scene* s, double dt, const fe_solver_desc* d) {
     const DiffGrid D = diff_grid(g);
     const dim3 grid((unsigned)D.blk[3]), block(kBlock);
     const FaceSet u{{s->u[0], s->u[1], s->u[2]}};
-    hipLaunchKernelGGL(k_diff_markers, grid, block, 0, s->stream, g, D, (const double*)s->sdf,
-                       (const double*)(s->has_collider ? s->csdf : nullptr), s->dmark[0], s->dmark[1], s->dmark[2]);
     DiffState init{};
     init.tol = d->tolerance;
     init.max_it = d->max_iterations;
     init.it = d->max_iterations;
     init.end = kDiffOpen;
+    hipLaunchKernelGGL(k_diff_markers, grid, block, 0, s->stream, g, D, (const double*)s->sdf,
+                       (const double*)(s->has_collider ? s->csdf : nullptr), s->dmark[0], s->dmark[1], s->dmark[2],
+                       s->dstate, init);
     hipLaunchKernelGGL(k_diff_build, grid, block, 0, s->stream, D, u, (const uint8_t*)s->dmark[0],
                        (const uint8_t*)s->dmark[1], (const uint8_t*)s->dmark[2], s->dcode, s->dx[0], s->dx[1], s->db,
-                       c[0], c[1], c[2], s->dstate, init);
+                       c[0], c[1], c[2], s->dstate);
     constexpr int kBatch = 50;  // sweeps between host reads of the stopping flags
     const int interval = d->check_interval;
     auto checked = [&](int j) { return interval > 0 && j > 0 && j % interval == 0; };  // after sweep j

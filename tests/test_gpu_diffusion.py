@@ -103,6 +103,36 @@ def test_diffusion_solver_setting(ctx):
     g.close()
 
 
+@pytest.mark.parametrize("value", [np.inf, np.nan])
+def test_diffusion_with_a_face_that_is_not_finite(ctx, value):
+    """A velocity outside the fluid that is not finite: no FLUID row reads it,
+    but its own row's residual is not a number, so that component runs to the
+    cap and does not converge, as in the oracle (where it also spreads, by
+    products with 0); the others do."""
+    print(f"[gpu] diffusion with a face of {value}", flush=True)
+    g, o = _pair(ctx, (12, 10, 8), (1.0, 0.8, 1.1), 0.01, seed=3)
+    probe, other = _pair(ctx, (12, 10, 8), (1.0, 0.8, 1.1), 0.01, seed=3)
+    other.diffusion(1.0 / 240)
+    air = np.argwhere(other.diffusion_markers(0) == orc.AIR)
+    u = g.get(capi.GRID_U)
+    u[tuple(air[len(air) // 2])] = value
+    g.set(capi.GRID_U, u)
+    o.set(orc.U, u.astype(np.float64))
+    g.set_diffusion_solver(capi.solver(capi.SOLVER_JACOBI, 60, 5, 1e-6))
+    o.set_diffusion_solver(orc.solver(orc.JACOBI, 60, 5, 1e-6))
+    g.run_stage(capi.STAGE_DIFFUSION, 1.0 / 240)
+    ost = o.diffusion(1.0 / 240)
+    gst = g.last_diffusion_stats()
+    assert [s.converged for s in gst] == [0, 1, 1] and np.isnan(gst[0].abs_residual)
+    assert np.isfinite(g.get(capi.GRID_U)).sum() == u.size - 1
+    for c, (gf, of) in enumerate(COMPS):
+        assert gst[c].iterations == ost[c].iterations
+        if c > 0:
+            assert np.abs(g.get(gf) - o.get(of)).max() <= 1e-6 * np.abs(o.get(of)).max()
+    g.close()
+    probe.close()
+
+
 def test_substep_with_viscosity_parity(ctx):
     print("[gpu] substep with viscosity", flush=True)
     n = 24
