@@ -13,8 +13,8 @@
 //   * solver: the reference's CudaJacobiIterationSolver(1000, 5, 1e-14) (:10)
 //     semantics: sweep, and after sweep it (it > 0, it % interval == 0) stop
 //     when ||b - A x||_2 < tolerance.
-// The three components' solves are independent; they run side by side in the
-// same launches, each with its own stop (DiffState).
+// The three components' solves are independent; on all but large grids they
+// run side by side in the same launches, each with its own stop (DiffState).
 // Everything is FP64 (x, b, the row arithmetic in the reference's operation
 // order with contraction off, the residual); the face velocities stay FP32
 // and are exact in FP64.  The 16-bit row code has the pressure
@@ -31,9 +31,9 @@ namespace fe {
 
 namespace {
 
-// The three components' faces back to back: component c's start at off[c] in
+// The solved components' faces back to back: component c's start at off[c] in
 // every array, its workgroups are blk[c] .. blk[c + 1] (multiples of 8 each,
-// so the XCD remap holds within a component).
+// so the XCD remap holds within a component; none where it is not solved).
 struct DiffGrid {
     int nx[3], ny[3];
     int64_t nf[3], off[3];
@@ -250,7 +250,7 @@ __global__ __launch_bounds__(kBlock) void k_diff_check(DiffGrid D, const double*
                                                        int interval, int compared, DiffState* __restrict__ st) {
     const int C = blockIdx.x;
     DiffState* S = st + C;
-    if (S->end != kDiffOpen) return;
+    if (D.blk[C + 1] == D.blk[C] || S->end != kDiffOpen) return;
     double t[1];
     sum_partials<1>(part + D.blk[C], (int)(D.blk[C + 1] - D.blk[C]), t);
     if (threadIdx.x != 0) return;
@@ -285,16 +285,32 @@ __global__ __launch_bounds__(kBlock) void k_diff_store(DiffGrid D, const double*
     }
 }
 
-DiffGrid diff_grid(const Geom& g) {
+// Up to here the three components are solved side by side, which saves two
+// launches' latency a sweep; above, a sweep of one component fills the chip and
+// its iterates stay in the last cache better, so they are solved one after
+// another, in buffers of the largest only (34 bytes a face of one component,
+// not of three).  100 sweeps of half full tanks, side by side / one after
+// another: 96x80x64 1.01 / 2.02 ms, 128^3 2.44 / 3.48, 160^3 4.11 / 5.04, 192^3
+// 9.03 / 7.61, 256^3 20.9 / 20.8.
+constexpr int64_t kDiffTogether = 1 << 22;  // faces of the largest component
+
+int64_t diff_faces(const Geom& g) {
+    return std::max(face_count(g, 0), std::max(face_count(g, 1), face_count(g, 2)));
+}
+
+// Components from c0 up to c1.
+DiffGrid diff_grid(const Geom& g, int c0, int c1) {
     DiffGrid D{};
     int64_t off = 0;
     for (int c = 0; c < 3; ++c) {
+        D.blk[c + 1] = D.blk[c];
+        if (c < c0 || c >= c1) continue;
         D.nx[c] = face_dim(g, c, 0);
         D.ny[c] = face_dim(g, c, 1);
         D.nf[c] = face_count(g, c);
         D.off[c] = off;
         off += (D.nf[c] + 15) / 16 * 16;
-        D.blk[c + 1] = D.blk[c] + pad_blocks((D.nf[c] + kBlock * kDiffPer - 1) / (kBlock * kDiffPer));
+        D.blk[c + 1] += pad_blocks((D.nf[c] + kBlock * kDiffPer - 1) / (kBlock * kDiffPer));
     }
     return D;
 }
@@ -303,14 +319,18 @@ DiffGrid diff_grid(const Geom& g) {
 
 hipError_t diffusion_alloc(fe_scene* s) {
     if (s->dstate_host) return hipSuccess;
-    const DiffGrid D = diff_grid(s->g);
-    const int64_t n = D.off[2] + D.nf[2];
+    const bool together = diff_faces(s->g) <= kDiffTogether;
+    const DiffGrid D = diff_grid(s->g, 0, 3);
+    const int64_t n = together ? D.off[2] + D.nf[2] : diff_faces(s->g);
     hipError_t e;
     for (int b = 0; b < 2; ++b)
         if ((e = hipMalloc((void**)&s->dx[b], sizeof(double) * n)) != hipSuccess) return e;
     if ((e = hipMalloc((void**)&s->dcode, sizeof(uint16_t) * n)) != hipSuccess) return e;
     if ((e = hipMalloc((void**)&s->db, sizeof(double) * n)) != hipSuccess) return e;
-    if ((e = hipMalloc((void**)&s->dsnap, sizeof(double) * n)) != hipSuccess) return e;
+    if (hipMalloc((void**)&s->dsnap, sizeof(double) * n) != hipSuccess) {
+        (void)hipGetLastError();  // without it repeated states go unseen, and every sweep is made
+        s->dsnap = nullptr;
+    }
     if ((e = hipMalloc((void**)&s->dpart, sizeof(double) * D.blk[3])) != hipSuccess) return e;
     if ((e = hipMalloc((void**)&s->dstate, sizeof(DiffState) * 3)) != hipSuccess) return e;
     for (int c = 0; c < 3; ++c)
@@ -334,23 +354,14 @@ void diffusion_free(fe_scene* s) {
     s->dstate_host = nullptr;
 }
 
-// ComputeDiffusion without its trailing ApplyBoundryCondition: the three
-// component solves (each reads and writes its own component only) as Jacobi
-// solves side by side on the scene's stream, in batches of sweeps with one
-// host read of the stopping flags per batch.  The check after sweep j is taken
-// from sweep j + 1, which reads the same rows: it leaves x_{j+1} in its input
-// buffer, so a stop found there loses nothing.
-hipError_t launch_diffusion(fe_scene* s, double dt, const fe_solver_desc* d) {
+// The solves of components c0 up to c1, side by side on the scene's stream, in
+// batches of sweeps with one host read of the stopping flags per batch.  The
+// check after sweep j is taken from sweep j + 1, which reads the same rows: it
+// leaves x_{j+1} in its input buffer, so a stop found there loses nothing.
+static hipError_t solve_components(fe_scene* s, const double (&c)[3], const fe_solver_desc* d, int c0, int c1) {
     const Geom& g = s->g;
-    const double nu = s->desc.viscosity;
-    const double c[3] = {(dt * nu) / (g.hd[0] * g.hd[0]), (dt * nu) / (g.hd[1] * g.hd[1]),
-                         (dt * nu) / (g.hd[2] * g.hd[2])};
     hipError_t e;
-    if ((e = diffusion_alloc(s)) != hipSuccess) {
-        diffusion_free(s);
-        return e;
-    }
-    const DiffGrid D = diff_grid(g);
+    const DiffGrid D = diff_grid(g, c0, c1);
     const dim3 grid((unsigned)D.blk[3]), block(kBlock);
     const FaceSet u{{s->u[0], s->u[1], s->u[2]}};
     DiffState init{};
@@ -367,16 +378,17 @@ hipError_t launch_diffusion(fe_scene* s, double dt, const fe_solver_desc* d) {
     constexpr int kBatch = 50;  // sweeps between host reads of the stopping flags
     const int interval = d->check_interval;
     auto checked = [&](int j) { return interval > 0 && j > 0 && j % interval == 0; };  // after sweep j
+    double* const snapshot = s->dsnap ? s->dsnap : s->db;  // without one: read, for nothing, and never written
     auto sweep = [&](auto kernel, int it, int snap) {
         hipLaunchKernelGGL(kernel, grid, block, 0, s->stream, D, (const uint16_t*)s->dcode, (const double*)s->db,
-                           (const double*)s->dx[it & 1], s->dx[(it + 1) & 1], c[0], c[1], c[2], it, snap, s->dsnap,
+                           (const double*)s->dx[it & 1], s->dx[(it + 1) & 1], c[0], c[1], c[2], it, snap, snapshot,
                            s->dstate, s->dpart);
     };
     auto check = [&](int q, int compared) {
         hipLaunchKernelGGL(k_diff_check, dim3(3), block, 0, s->stream, D, (const double*)s->dpart, q, interval,
                            compared, s->dstate);
     };
-    for (int comp = 0; comp < 3; ++comp) s->dstate_host[comp] = init;
+    for (int comp = c0; comp < c1; ++comp) s->dstate_host[comp] = init;
     int it = 0;
     bool done = false;
     while (it < d->max_iterations && !done) {
@@ -384,8 +396,8 @@ hipError_t launch_diffusion(fe_scene* s, double dt, const fe_solver_desc* d) {
         for (; it < end; ++it) {
             if (checked(it - 1)) {
                 const int q = (it - 1) / interval;
-                sweep(k_diff_sweep<true, true>, it, q % kDiffRing == 0);
-                check(q, q > kDiffRing);
+                sweep(k_diff_sweep<true, true>, it, s->dsnap && q % kDiffRing == 0);
+                check(q, s->dsnap && q > kDiffRing);
             } else {
                 sweep(k_diff_sweep<false, true>, it, 0);
             }
@@ -400,10 +412,10 @@ hipError_t launch_diffusion(fe_scene* s, double dt, const fe_solver_desc* d) {
             return e;
         if ((e = hipStreamSynchronize(s->stream)) != hipSuccess) return e;
         done = true;
-        for (int comp = 0; comp < 3; ++comp) done = done && s->dstate_host[comp].end <= it;
+        for (int comp = c0; comp < c1; ++comp) done = done && s->dstate_host[comp].end <= it;
     }
     int odd = 0;
-    for (int comp = 0; comp < 3; ++comp) {
+    for (int comp = c0; comp < c1; ++comp) {
         const DiffState& h = s->dstate_host[comp];
         odd |= (std::min(h.end, d->max_iterations) & 1) << comp;
         fe_solve_stats& st = s->diff_stats[comp];
@@ -417,6 +429,24 @@ hipError_t launch_diffusion(fe_scene* s, double dt, const fe_solver_desc* d) {
     hipLaunchKernelGGL(k_diff_store, grid, block, 0, s->stream, D, (const double*)s->dx[0], (const double*)s->dx[1],
                        odd, u);
     return hipGetLastError();
+}
+
+// ComputeDiffusion without its trailing ApplyBoundryCondition: the three
+// component solves (each reads and writes its own component only).
+hipError_t launch_diffusion(fe_scene* s, double dt, const fe_solver_desc* d) {
+    const Geom& g = s->g;
+    const double nu = s->desc.viscosity;
+    const double c[3] = {(dt * nu) / (g.hd[0] * g.hd[0]), (dt * nu) / (g.hd[1] * g.hd[1]),
+                         (dt * nu) / (g.hd[2] * g.hd[2])};
+    hipError_t e;
+    if ((e = diffusion_alloc(s)) != hipSuccess) {
+        diffusion_free(s);
+        return e;
+    }
+    if (diff_faces(g) <= kDiffTogether) return solve_components(s, c, d, 0, 3);
+    for (int comp = 0; comp < 3; ++comp)
+        if ((e = solve_components(s, c, d, comp, comp + 1)) != hipSuccess) return e;
+    return hipSuccess;
 }
 
 }  // namespace fe

@@ -11,6 +11,8 @@ Bars:
   * a full substep with viscosity -- markers bit-exact, velocities within the
     substep bar of the inviscid parity test (2e-4 relative).
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -46,6 +48,13 @@ def _pair(ctx, n, size, nu, seed):
     return g, o
 
 
+def _free_bytes():
+    """Device memory left, as the library's HIP runtime has it."""
+    free, total = C.c_size_t(), C.c_size_t()
+    assert capi.load().hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
 def _compare(g, o, gst, ost, rtol=1e-6):
     for c, (gf, of) in enumerate(COMPS):
         assert np.array_equal(g.get(DMARK[c]), o.diffusion_markers(c)), f"markers {c}"
@@ -68,6 +77,28 @@ def test_diffusion_stage_parity(ctx, n, size, nu):
     gst = g.last_diffusion_stats()
     _compare(g, o, gst, ost)
     assert all(s.converged for s in gst)
+    g.close()
+
+
+def test_diffusion_of_large_grids(ctx):
+    """Above 2^22 faces the components are solved one after another, in 34
+    bytes of buffers for each face of the largest component and a byte of
+    markers for each of all: the same markers, counts and values."""
+    n = (164, 162, 161)
+    print(f"[gpu] diffusion stage n={n}", flush=True)
+    g, o = _pair(ctx, n, (1.0, 0.9, 1.1), 0.02, seed=1)
+    g.set_diffusion_solver(capi.solver(capi.SOLVER_JACOBI, 8, 3, 1e-30))
+    o.set_diffusion_solver(orc.solver(orc.JACOBI, 8, 3, 1e-30))
+    free = _free_bytes()
+    g.run_stage(capi.STAGE_DIFFUSION, 1.0 / 240)
+    held = free - _free_bytes()
+    faces = 165 * 162 * 161
+    print(f"[gpu]   {held / faces:.1f} bytes a face of one component", flush=True)
+    assert held < 48 * faces  # 34 + 3, and what allocations round up to
+    ost = o.diffusion(1.0 / 240)
+    gst = g.last_diffusion_stats()
+    assert all(s.iterations == 8 and not s.converged and s.abs_residual > 0 for s in gst)
+    _compare(g, o, gst, ost)
     g.close()
 
 
