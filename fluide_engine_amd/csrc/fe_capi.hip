@@ -346,6 +346,7 @@ int substep_graph(fe_scene* s, double dt, const fe_solver_desc* d, fe_solve_stat
     int rc;
     if (fresh) {
         graph_release(G);
+        HIPCHK(ctx, pressure_alloc(s, d));  // not in the capture
         const int prev = s->last_cg_iters[precond];
         G.iters = std::max(4, std::min(prev + 2, d->max_iterations + 1));
         G.gen = s->graph_gen;
@@ -628,7 +629,6 @@ int fe_scene_create(fe_ctx* ctx, const fe_scene_desc* d, fe_scene** out) {
     chk(dalloc(&s->d[0], nc));
     chk(dalloc(&s->d[1], nc));
     chk(dalloc(&s->q, nc));
-    chk(dalloc(&s->q2, nc));
     // CG: 5 + 5 partials per block; with multigrid 2 + 2 and r.z of the V-cycle
     s->npartials = solver_shape_n(nc).blocks * 10;
     chk(dalloc(&s->partials, s->npartials));

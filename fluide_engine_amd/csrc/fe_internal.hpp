@@ -539,7 +539,7 @@ struct fe_scene {
     float* z = nullptr;           // preconditioned residual
     float* d[2] = {nullptr, nullptr};
     float* q = nullptr;
-    float* q2 = nullptr;          // q's ping-pong partner (CG without multigrid)
+    float* q2 = nullptr;          // q's ping-pong partner (CG without multigrid, from its first solve on)
     double* partials = nullptr;   // per-block FP64 partial sums (2 per block)
     uint8_t* chunk_fluid = nullptr;  // per solver block: its cells include a FLUID cell (from BuildSystem)
     int64_t npartials = 0;

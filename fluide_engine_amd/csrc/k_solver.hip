@@ -1071,10 +1071,16 @@ static hipError_t cg_host_loop(fe_scene* s, const fe_solver_desc* d, const CGSet
     return hipSuccess;
 }
 
+hipError_t pressure_alloc(fe_scene* s, const fe_solver_desc* d) {
+    if (s->q2 || (d->kind != FE_SOLVER_CG && d->kind != FE_SOLVER_PCG_JACOBI)) return hipSuccess;
+    return hipMalloc((void**)&s->q2, sizeof(float) * cell_count(s->g) + 64);
+}
+
 hipError_t launch_pressure_solve(fe_scene* s, const fe_solver_desc* d) {
     SolverScalars init;
-    hipError_t e = solve_begin(s, d, init);
+    hipError_t e = pressure_alloc(s, d);
     if (e != hipSuccess) return e;
+    if ((e = solve_begin(s, d, init)) != hipSuccess) return e;
     if (d->kind == FE_SOLVER_JACOBI) return jacobi_solve(s, d);
     if (init.precond == 2 && (e = mg_setup(s)) != hipSuccess) return e;
     const CGSetup c = cg_setup(s, init.precond);

@@ -299,6 +299,30 @@ def test_capped_solve_after_a_long_one(ctx, kind):
     g.close()
 
 
+def test_cg_buffer_comes_with_the_first_cg_solve(ctx):
+    """The vector that only CG without multigrid needs (4 bytes a cell) is held
+    from its first solve on, not by scenes that take another solver."""
+    import ctypes as C
+
+    def free_bytes():
+        free, total = C.c_size_t(), C.c_size_t()
+        assert capi.load().hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        return free.value
+
+    n = 160
+    print(f"[gpu] cg buffer n={n}", flush=True)
+    g = capi.Scene(ctx, capi.scene_desc((n, n, n), method=capi.FLIP, max_particles=16))
+    g.set(capi.GRID_SDF, np.full((n, n, n), -1.0))
+    free = [free_bytes()]
+    for kind in (capi.SOLVER_JACOBI, capi.SOLVER_CG, capi.SOLVER_PCG_JACOBI, capi.SOLVER_CG):
+        g.run_stage(capi.STAGE_PRESSURE, desc=capi.solver(kind, 2, 0, 1e-6, relative=True))
+        free.append(free_bytes())
+    held = -np.diff(free)
+    # the runtime's own first allocations take a few MB
+    assert held[0] < n ** 3 and 4 * n ** 3 <= held[1] < 5 * n ** 3 and held[2] == held[3] == 0, held
+    g.close()
+
+
 @pytest.mark.parametrize("n", [48, 64])
 @pytest.mark.parametrize("kind", [capi.SOLVER_MGPCG, capi.SOLVER_CG])
 def test_first_substep_solve_converges(ctx, kind, n):
