@@ -202,7 +202,7 @@ template <bool Buckets>
 __global__ __launch_bounds__(kBlock) void k_sdf_lanes(Geom g, const float4* __restrict__ pos4,
                                                       const int32_t* __restrict__ start, double* __restrict__ sdf,
                                                       int ex, int ey, int ez, double radius, double band, double qr2,
-                                                      float slack, int64_t padded) {
+                                                      float slack, float near2, int64_t padded) {
 #pragma clang fp contract(off)
     const int64_t blk = xcd_remap(blockIdx.x, padded);
     const int tbx = (g.n[0] + kSdfLX - 1) / kSdfLX, tby = (g.n[1] + kSdfLY - 1) / kSdfLY,
@@ -242,14 +242,14 @@ __global__ __launch_bounds__(kBlock) void k_sdf_lanes(Geom g, const float4* __re
         }
     }
     const float gx32 = (float)gp[0], gy32 = (float)gp[1], gz32 = (float)gp[2];
-    const float near2 = 0.98f * (float)(radius * radius);
     float best32 = __builtin_inff();
     double best = qr2;  // a particle at exactly the band gives the value of none
     auto consider = [&](const float4 p) {
         const float fx = p.x - gx32, fy = p.y - gy32, fz = p.z - gz32;
         const float d2f = fx * fx + fy * fy + fz * fz;
         if (d2f > best32 + slack) return;
-        // every particle nearer than r is in the buckets (the margin is for rounding)
+        // every particle nearer than r is in the buckets (near2: r^2 less the
+        // rounding of d2f, which grows with the coordinates)
         if (Buckets && d2f > near2) {
             const int bx = (int)floor((double)p.x / sp), by = (int)floor((double)p.y / sp),
                       bz = (int)floor((double)p.z / sp);
@@ -335,9 +335,13 @@ hipError_t launch_sdf(fe_scene* s, bool buckets) {
     const int bs[3] = {lanes ? kSdfLX : kSdfBX, lanes ? kSdfLY : kSdfBY, lanes ? kSdfLZ : kSdfBZ};
     const int64_t padded = pad_blocks((int64_t)((g.n[0] + bs[0] - 1) / bs[0]) * ((g.n[1] + bs[1] - 1) / bs[1]) *
                                       ((g.n[2] + bs[2] - 1) / bs[2]));
-    auto kern = buckets ? k_sdf_lanes<true> : (lanes ? k_sdf_lanes<false> : k_sdf);
-    launch_timed(s, FE_KERNEL_SDF, 0, kern, dim3((unsigned)padded), dim3(kBlock), g, (const float4*)s->pos4,
-                 (const int32_t*)s->cell_start, s->sdf, ext[0], ext[1], ext[2], radius, band, qr2, slack, padded);
+    if (lanes)
+        launch_timed(s, FE_KERNEL_SDF, 0, buckets ? k_sdf_lanes<true> : k_sdf_lanes<false>, dim3((unsigned)padded),
+                     dim3(kBlock), g, (const float4*)s->pos4, (const int32_t*)s->cell_start, s->sdf, ext[0], ext[1],
+                     ext[2], radius, band, qr2, slack, (float)(radius * radius) - slack, padded);
+    else
+        launch_timed(s, FE_KERNEL_SDF, 0, k_sdf, dim3((unsigned)padded), dim3(kBlock), g, (const float4*)s->pos4,
+                     (const int32_t*)s->cell_start, s->sdf, ext[0], ext[1], ext[2], radius, band, qr2, slack, padded);
     s->sdf_from_cells = buckets ? 0 : 1;
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;

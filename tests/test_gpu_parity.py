@@ -541,3 +541,35 @@ def test_sdf_lane_variants(ctx, n, search):
     where = np.ones(want.shape, bool) if search == capi.SDF_SEARCH_BUCKETS else (want < 0) | (got < 0)
     assert np.array_equal(got[where], want[where])
     g.close()
+
+
+@pytest.mark.parametrize("away", [0.0, 1024.0, 16384.0, 131072.0])
+@pytest.mark.parametrize("search", [capi.SDF_SEARCH_CELLS, capi.SDF_SEARCH_BUCKETS])
+def test_sdf_far_from_the_origin(ctx, search, away):
+    """A domain away from the origin, up to where FP32 coordinates are 0.4 of a
+    cell apart: the distances are taken between the FP32 positions in FP64,
+    so the values keep the oracle's bits (cells: the negative ones).  Single
+    particles about a radius from a cell centre along x, where the buckets
+    end, as well as a cloud of them."""
+    print(f"[gpu] sdf at {away} search={search}", flush=True)
+    n, h, origin = (400, 31, 25), 0.0375, (away, -away, 0.5 * away)
+    size = tuple(m * h for m in n)
+    rng = np.random.default_rng(8)
+    i, j, k = (a.ravel() for a in np.meshgrid(np.arange(2, 398, 6), np.arange(3, 24, 6), np.arange(3, 24, 6)))
+    r = 1.2 * h / np.sqrt(2.0)
+    single = np.stack([(i + (j + 2 * k) // 3 % 6 + 0.5) * h - r * rng.uniform(0.99, 1.02, i.size), (j + 0.5) * h,
+                       (k + 0.5) * h], 1)
+    cloud = rng.uniform(0, 1, (2000, 3)) * np.array([400, 4, 25]) * h + np.array([0, 27 * h, 0])
+    x = (np.array(origin) + np.concatenate([single, cloud])).astype(np.float32)
+    count = len(x)
+    g = capi.Scene(ctx, capi.scene_desc(n, method=capi.FLIP, origin=origin, size=size, max_particles=count))
+    g.set_sdf_search(search)
+    g.upload_particles(x, np.zeros_like(x))
+    g.run_stage(capi.STAGE_SDF)
+    o = orc.Scene(n, origin=origin, size=size, method=orc.FLIP, blend=0.05, max_cfl=3.0)
+    o.set_particles(x.astype(np.float64), np.zeros(x.shape))
+    o.build_sdf()
+    got, want = g.get(capi.GRID_SDF), o.get(orc.SDF)
+    where = np.ones(want.shape, bool) if search == capi.SDF_SEARCH_BUCKETS else (want < 0) | (got < 0)
+    assert np.array_equal(got[where], want[where]), (got[where] != want[where]).sum()
+    g.close()
