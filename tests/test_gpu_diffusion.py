@@ -198,9 +198,10 @@ def test_substep_with_viscosity_parity(ctx):
                                                ((5, 31, 3), 0.2, 6, 5), ((16, 16, 33), 0.1, 300, 0)])
 def test_diffusion_repeated_states(ctx, n, nu, cap, interval):
     """An unreachable tolerance: the sweeps end in repeated states long before
-    the cap, and the counts, the last residual and the values are those of
-    the whole number of sweeps (odd and even intervals and caps, none at all;
-    residuals of rounding size, so within a factor of 4 of the oracle's)."""
+    the cap, and the counts, the values (to FP32) and the last residual are
+    those of the whole number of sweeps: the residual's bits are those of a
+    run that checks at that one sweep only, compares no states and so makes
+    them all (odd and even intervals and caps, none at all)."""
     print(f"[gpu] diffusion repeated states n={n} cap={cap} interval={interval}", flush=True)
     g, o = _pair(ctx, n, (1.0, 0.8, 1.1), nu, seed=sum(n))
     g.set_diffusion_solver(capi.solver(capi.SOLVER_JACOBI, cap, interval, 1e-30))
@@ -216,4 +217,30 @@ def test_diffusion_repeated_states(ctx, n, nu, cap, interval):
             assert 0.0 <= s.abs_residual < 1e-12 if cap > 100 else s.abs_residual > 1e-12
         else:
             assert s.abs_residual == -1.0
+    g.close()
+    if interval and cap > interval:
+        g, _ = _pair(ctx, n, (1.0, 0.8, 1.1), nu, seed=sum(n))
+        g.set_diffusion_solver(capi.solver(capi.SOLVER_JACOBI, cap, (cap - 1) // interval * interval, 1e-30))
+        g.run_stage(capi.STAGE_DIFFUSION, dt)
+        assert [s.abs_residual for s in g.last_diffusion_stats()] == [s.abs_residual for s in gst]
+        g.close()
+
+
+def test_diffusion_ends_at_a_repeated_state(ctx):
+    """100 000 sweeps, which alone take 250 ms of the device, end within the few
+    hundred that bring the states to repeat themselves (the quickest of three
+    runs)."""
+    import time
+
+    print("[gpu] diffusion ends at a repeated state", flush=True)
+    g, _ = _pair(ctx, (12, 10, 8), (1.0, 0.8, 1.1), 0.05, seed=30)
+    g.set_diffusion_solver(capi.solver(capi.SOLVER_JACOBI, 100000, 5, 1e-30))
+    took = []
+    for _ in range(3):
+        t0 = time.perf_counter()
+        g.run_stage(capi.STAGE_DIFFUSION, 1.0 / 120)
+        took.append(time.perf_counter() - t0)
+        assert all(s.iterations == 100000 and not s.converged for s in g.last_diffusion_stats())
+    print(f"[gpu]   {min(took) * 1e3:.1f} ms", flush=True)
+    assert min(took) < 0.1
     g.close()

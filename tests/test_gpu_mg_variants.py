@@ -24,8 +24,8 @@ def ctx():
 
 
 def _system(ctx, shape, seed, noise=0.03):
-    # a very long grid gets cubic cells: stretched 500 : 1, point smoothing does not converge on it
-    size = [m / shape[0] for m in shape] if max(shape) >= 1000 else (1.0, 1.0, 1.0)
+    # a very long grid gets cubic cells: stretched 20 : 1 and more, point smoothing does not converge on it
+    size = [m / shape[0] for m in shape] if max(shape) > 20 * min(shape) else (1.0, 1.0, 1.0)
     desc = capi.scene_desc(shape, method=capi.FLIP, max_particles=16, size=size)
     g = capi.Scene(ctx, desc)
     rng = np.random.default_rng(seed)
@@ -63,7 +63,8 @@ def test_fused_and_split_vcycles_agree(ctx, shape):
 
 @pytest.mark.parametrize("shape", [(64, 64, 48), (64, 64, 49),  # the last on small tiles, the first on large ones
                                    (2, 2, 2), (3, 2, 33), (15, 17, 9), (129, 33, 65),  # remainders of both
-                                   (4, 4, 2000)])  # too long for the one-workgroup bottom
+                                   (4, 4, 2000),  # too long for the one-workgroup bottom
+                                   (8, 64, 64), (16, 8, 256), (8, 160, 184)])  # bottoms of 66, 75 and 78 KB of LDS
 def test_tile_shapes_agree_with_split_vcycle(ctx, shape):
     test_fused_and_split_vcycles_agree(ctx, shape)
 

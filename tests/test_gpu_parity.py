@@ -254,7 +254,8 @@ def test_pressure_cg_reaches_tolerance(ctx, kind, shape):
 
 
 @pytest.mark.parametrize("cap", [1, 2, 5])
-@pytest.mark.parametrize("shape", [(5, 4, 3), (33, 20, 17), (70, 65, 64)])  # the last: four cells a thread (above 2^18)
+@pytest.mark.parametrize("shape", [(5, 4, 3), (33, 20, 17), (70, 65, 64),  # the last: two cells a thread (above 2^18)
+                                   (88, 87, 86)])  # and three, in two groups (above 2^19)
 @pytest.mark.parametrize("kind", [capi.SOLVER_CG, capi.SOLVER_PCG_JACOBI])
 def test_cg_iterates_match_oracle(ctx, kind, shape, cap):
     """The iterate after exactly cap iterations against the oracle's FP64 one.
