@@ -576,10 +576,10 @@ __global__ __launch_bounds__(kBlock) void k_mg_prolong(const float* __restrict__
 // fine tile of twice that size below it.  It stages what the tile's sweeps
 // read, with halos, in LDS and recomputes the halo cells of each sweep itself
 // instead of waiting for a neighbour tile, so a level takes two launches
-// instead of six.  Every value is the split kernels' (the same terms in the
-// same order; only the source of a neighbour value differs, and a neighbour
-// outside the grid, which enters with weight 0, reads 0 here).  The sweeps and
-// residuals take the FLUID-row forms (mg_sweep_fluid_row: diagonal and weight
+// instead of six.  The terms of every value are the split kernels' (a neighbour
+// outside the grid, which enters with weight 0, reads 0 here), and so is their
+// order but for the restriction, whose four planes are added as a tree: the
+// variants agree to FP32 rounding.  The sweeps and residuals take the FLUID-row forms (mg_sweep_fluid_row: diagonal and weight
 // from a per-wavefront lane table, coupling terms without the code's selects),
 // half the instructions of the general ones: the finest level's phases are
 // VALU-bound (16 waves of a tile share one CU's four SIMDs).
@@ -1226,8 +1226,9 @@ __global__ __launch_bounds__(kTailThreads) void k_mg_tail(TailArgs a, const floa
 // place, in registers) and at most one coarse cell.  The iterates lie in LDS
 // with a border of zeros, so the FLUID-row forms need neither codes nor
 // clamps there: a cell's neighbours are at fixed offsets, and every cell that
-// is not FLUID holds 0, as does the border.  The terms and their order are the
-// tiles' and the tail's, so the values are too.
+// is not FLUID holds 0, as does the border.  The terms are the tiles' and the
+// tail's, in their order but for the restriction's rows, which are added one
+// after another as in the split kernels: the values agree to FP32 rounding.
 // ---------------------------------------------------------------------------
 constexpr int kBotThreads = 1024;
 constexpr int kBotPer = 4;  // fine cells per thread: a coarsest level of 512 cells halves one of at most 4096

@@ -476,7 +476,7 @@ enum fe_kernel_id {
     FE_KERNEL_NONE = 0,
     FE_KERNEL_CG_SPMV = 1,    /* d = z + beta d, q = A d, d.q; without multigrid an iteration whole */
     FE_KERNEL_CG_UPDATE = 2,  /* multigrid PCG: x += alpha d, r -= alpha q, z = M^-1 r, r.z */
-    FE_KERNEL_P2G = 3,        /* per-face gather (3 launches per substep, one per component) */
+    FE_KERNEL_P2G = 3,        /* particles to faces (a launch per component, or one for the three on small grids and APIC) */
     FE_KERNEL_G2P_MOVE = 4,   /* fused G2P + advection */
     FE_KERNEL_SDF = 5,        /* fluid SDF */
     FE_KERNEL_JACOBI = 6,     /* one Jacobi sweep */
